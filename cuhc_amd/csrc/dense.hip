@@ -14,26 +14,36 @@
 // the row's minimum; row a's new fn is the minimum of its new distances.
 //
 // The merge loop is one cooperative persistent kernel (one workgroup per CU)
-// with one grid barrier per merge. Workgroup g owns a contiguous range of
-// slots (rows): their fn and size live in its LDS, it alone writes D(k, a) /
-// D(a, k) for its rows k, and every workgroup keeps the active flags of all
-// slots as a bitmask in LDS. Phase s (between two barriers):
-//   select:  every workgroup reads all records of phase s - 1 and reduces them
-//            the same way: the previous merged row's new fn (the minimum of
-//            the workgroups' parts) and the pair (a, b) = the lowest
-//            (selection key, fn) over every row, that one included; b's bit
-//            is cleared; the owner of the previous merged slot installs its
-//            fn, size and id (sizes and ids change one phase late, so no read
-//            in the merge's own phase races the write);
-//   update:  Lance-Williams update of D(a, k) for its own k, its rows' fn,
-//            and its part of row a's new fn (minimum over its k > a);
-//   rescan:  its rows whose nearest was a or b and is not the merged distance
-//            are scanned again by the whole workgroup (no other workgroup
-//            changes an entry of such a row in this phase, and D(k, a) is the
-//            value it just stored);
-//   record:  the minimum (selection key, fn) over its rows but a, and its part
-//            of row a's fn;
-//   barrier.
+// that makes up to kMaxBatch merges per two grid barriers.
+// Workgroup g owns a contiguous range of slots (rows): their fn, size, bound
+// and pending flag live in its LDS, it alone writes D(k, a) / D(a, k) for its
+// rows k, and every workgroup keeps the active flags of all slots as a bitmask
+// in LDS. A batch has two halves, each ended by a grid barrier:
+//   A select:  every workgroup reads all records and takes the same batch: the
+//              lowest pairs in (distance, row) order, up to the first that
+//              touches a slot of an earlier one, that is not below every
+//              pending row's lower bound, or that lies beyond the rows a
+//              workgroup published. Rows left pending by the previous batch
+//              are rescanned meanwhile, in column chunks shared by all waves.
+//     update:  D(a_t, k) of every merge t of the batch for its own rows k,
+//              each rounded as the one-at-a-time loop rounds it, kept in LDS;
+//              it publishes, per merge, the smallest new distance and the two
+//              lowest keys of its part of row a_t.
+//   B commit:  from those, every workgroup finds the same valid prefix of the
+//              batch: merge t stands if its distance is below every new
+//              distance of the merges before it (then the one-at-a-time loop
+//              picks it next; the first always stands). The workgroup writes
+//              the prefix's distances of its rows and updates their fn and the
+//              lower bound of their other keys. A row whose fn was a or b, and
+//              whose new distance is not below that bound, is pending: the
+//              bound now covers all its keys.
+//     record:  its kTop lowest (distance, row) keys and fn columns, its lowest
+//              pending bound and its pending rows.
+// The merges, their order, ties and every rounding are those of merging the
+// lowest (distance, i, j) pair one at a time. Neighbouring merges rarely touch
+// each other: 12 of 16 stand per batch at n = 5,000, 14 at 12,000.
+// Bound by latency (barriers and dependent memory round trips), so the batch
+// divides it: see denseMergeKernel for the measured times.
 // Per-workgroup records replace same-address atomics, which serialize across
 // workgroups. The tree row is written on the device; there is no host round
 // trip between merges.
@@ -48,12 +58,16 @@ namespace {
 
 constexpr int kThreads = 512;
 constexpr int kChunk = 8192;                     // columns per initial-scan work item
-constexpr int kRescanChunk = 4096;               // columns per rescan work item
-constexpr int kRescanPer = kRescanChunk / kThreads;
+constexpr int kWaves = kThreads / 64;
+constexpr int kRescanCols = 1024;                // columns per rescan work item (one wave)
+constexpr int kRescanPer = kRescanCols / 64;
 constexpr int kMaxOwned = 2048;                  // rows per workgroup (LDS row state)
-constexpr int kUpdatePer = 2;                    // owned rows per thread per load batch
-constexpr int kRecordWords = 8;                  // u64 words per workgroup record
+constexpr int kUpdatePer = 4;                    // owned rows per lane per load batch
+constexpr int kMaxBatch = 16;                    // merges per batch
+constexpr int kMinGroups = 8;                    // workgroups of the merge kernel at least
+constexpr int kTop = 4;                          // lowest rows carried in a record
 constexpr int kInlineRows = 6;                   // pending rows carried in a record
+constexpr int kRecordWords = 12;                 // u64 words per workgroup record (96 bytes)
 constexpr int kGroup = 16;                       // workgroups per first-level barrier counter
 constexpr int kLineWords = 32;                   // one 128-byte line in 32-bit words
 constexpr unsigned int kSpinLimit = 1u << 22;    // barrier polls (seconds) before aborting
@@ -76,17 +90,19 @@ HD size_t condensedIndex(long long i, long long j, long long n) {
   return (size_t)(i * n - i * (i + 1) / 2 + (j - i - 1));
 }
 
-DEV double lanceWilliams(int linkage, double dak, double dbk, double dab, double na, double nb,
-                         double nk) {
-  switch (linkage) {
-  case kSingle: return fmin(dak, dbk);
-  case kComplete: return fmax(dak, dbk);
-  case kAverage: return (na * dak + nb * dbk) / (na + nb);
-  default: {
+template <int LINKAGE>
+DEV float lanceWilliams(float dakF, float dbkF, float dabF, int naI, int nbI, int nkI) {
+  const double dak = dakF, dbk = dbkF, dab = dabF, na = naI, nb = nbI, nk = nkI;
+  if constexpr (LINKAGE == kSingle) {
+    return (float)fmin(dak, dbk);
+  } else if constexpr (LINKAGE == kComplete) {
+    return (float)fmax(dak, dbk);
+  } else if constexpr (LINKAGE == kAverage) {
+    return (float)((na * dak + nb * dbk) / (na + nb));
+  } else {
     const double total = na + nb + nk;
     const double sq = ((na + nk) * dak * dak + (nb + nk) * dbk * dbk - nk * dab * dab) / total;
-    return sqrt(fmax(sq, 0.0));
-  }
+    return (float)sqrt(fmax(sq, 0.0));
   }
 }
 
@@ -153,29 +169,30 @@ DEV bool gridBarrier(const Barrier &bar, unsigned int &generation, int *ok) {
 struct DenseState {
   float *D;
   int n;
-  int linkage;
   int firstNewId;
-  // Cluster size and scipy id by slot. The owner of a merged slot writes its
-  // new size and id one phase after the merge (every workgroup still reads
-  // the old size in the merge's own phase, and knows the new one itself).
-  int *size;
+  int per;   // rows per workgroup
+  int batch; // merges per batch (at most kMaxBatch)
+  int *size; // cluster size and scipy id by slot
   int *id;
-  unsigned long long *fnKey;    // initial forward nearest per slot (denseInitKernel)
-  unsigned long long *fnRescan; // per slot: the rescan's minimum (atomicMin) while pending
-  // One record per workgroup and publish (kRecordWords words): [0] and [1]
-  // the minimum (selection key, fn) over its settled rows, [2] its part of
-  // the merged row's new fn, [3] the lowest lower-bound key of its pending
-  // rows, [4] the number of rows it made pending in the phase, [5..7] the
-  // first kInlineRows of them (two per word); all of them in pendingRows[g
-  // kMaxOwned ...] when there are more. Two buffers, alternating by publish:
-  // consecutive publishes are separated by a grid barrier, so a buffer is
-  // rewritten only after every workgroup has passed the barrier that follows
-  // its last reader's next publish.
-  unsigned long long *records; // [2][G kRecordWords]
-  int *pendingRows;            // [2][G kMaxOwned]
-  int2 *items;                 // initial fn: (row, first column) work items
-  double *tree;                // (n - 1) x 4, device
-  unsigned long long *clocks;  // null, or [4]: device-clock ticks per part of a merge
+  // Per slot, [2][n]: the forward nearest key and the second lowest key of
+  // the row, from denseInitKernel and, while a row is pending, from its rescan.
+  unsigned long long *scanned;
+  // One record per workgroup (kRecordWords words): [0..3] its kTop lowest
+  // selection keys, [4..5] their fn columns, [6] the lowest lower-bound key of
+  // its pending rows, [7] the number of its pending rows, [8..10] the first
+  // kInlineRows of them (two per word); all of them in pendingRows[g per ...]
+  // when there are more. Written in the second half of a batch and read in
+  // the first half of the next, so a barrier lies between any write and read.
+  unsigned long long *records;
+  int *pendingRows;
+  // Per merge of the batch and workgroup, [kMaxBatch][G]: the two lowest keys
+  // of its part of row a, and the ordered bits of its smallest new distance.
+  // Written in the first half, read in the second.
+  unsigned long long *partFn, *partNext;
+  unsigned int *partMin;
+  int2 *items;                // initial fn: (row, first column) work items
+  double *tree;               // (n - 1) x 4, device
+  unsigned long long *clocks; // null, or [4]: device-clock ticks per part of a batch
   Barrier bar;
 };
 
@@ -194,141 +211,38 @@ DEV unsigned long long blockMinKey(unsigned long long v, unsigned long long *red
   return r;
 }
 
-// Lexicographic minimum of (key, payload) pairs.
-DEV void pairMin(unsigned long long &k, unsigned long long &p, unsigned long long k2,
-                 unsigned long long p2) {
-  if (k2 < k || (k2 == k && p2 < p)) {
-    k = k2;
-    p = p2;
-  }
+// Keeps the two lowest keys of everything offered.
+DEV void offer(unsigned long long &lowest, unsigned long long &next, unsigned long long key) {
+  next = minKey(next, key < lowest ? lowest : key);
+  lowest = minKey(lowest, key);
 }
 
-DEV void blockMinPair(unsigned long long &k, unsigned long long &p, unsigned long long *redK,
-                      unsigned long long *redP) {
-#pragma unroll
-  for (int m = 32; m > 0; m >>= 1)
-    pairMin(k, p, shflXorKey(k, m), shflXorKey(p, m));
-  const int wave = threadIdx.x >> 6;
-  __syncthreads();
-  if ((threadIdx.x & 63) == 0) {
-    redK[wave] = k;
-    redP[wave] = p;
-  }
-  __syncthreads();
-  k = redK[0];
-  p = redP[0];
-  for (int w = 1; w < kThreads / 64; ++w)
-    pairMin(k, p, redK[w], redP[w]);
-}
-
-// Workgroup reduction of (k, p) by lexicographic minimum and of x, y and z
-// by minimum, in one LDS exchange (red: 5 kThreads / 64 words).
-DEV void blockReduce5(unsigned long long &k, unsigned long long &p, unsigned long long &x,
-                      unsigned long long &y, unsigned long long &z, unsigned long long *red) {
-  constexpr int W = kThreads / 64;
-#pragma unroll
-  for (int m = 32; m > 0; m >>= 1) {
-    pairMin(k, p, shflXorKey(k, m), shflXorKey(p, m));
-    x = minKey(x, shflXorKey(x, m));
-    y = minKey(y, shflXorKey(y, m));
-    z = minKey(z, shflXorKey(z, m));
-  }
-  const int wave = threadIdx.x >> 6;
-  __syncthreads();
-  if ((threadIdx.x & 63) == 0) {
-    red[wave] = k;
-    red[W + wave] = p;
-    red[2 * W + wave] = x;
-    red[3 * W + wave] = y;
-    red[4 * W + wave] = z;
-  }
-  __syncthreads();
-  k = red[0];
-  p = red[W];
-  x = red[2 * W];
-  y = red[3 * W];
-  z = red[4 * W];
-  for (int w = 1; w < W; ++w) {
-    pairMin(k, p, red[w], red[W + w]);
-    x = minKey(x, red[2 * W + w]);
-    y = minKey(y, red[3 * W + w]);
-    z = minKey(z, red[4 * W + w]);
-  }
-}
-
-// A blockReduce5 without z plus, in the same exchange, the exclusive prefix sum of cnt
-// (start; total receives the sum) and whether any cnt exceeds kInlineRows.
-DEV void blockReduce4Scan(unsigned long long &k, unsigned long long &p, unsigned long long &x,
-                          unsigned long long &y, int cnt, int &start, int &total,
-                          bool &spilled, unsigned long long *red, int *redInt) {
-  constexpr int W = kThreads / 64;
-  const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
-#pragma unroll
-  for (int m = 32; m > 0; m >>= 1) {
-    pairMin(k, p, shflXorKey(k, m), shflXorKey(p, m));
-    x = minKey(x, shflXorKey(x, m));
-    y = minKey(y, shflXorKey(y, m));
-  }
-  int incl = cnt;
-#pragma unroll
-  for (int d = 1; d < 64; d <<= 1) {
-    const int v = __shfl_up(incl, d, 64);
-    if (lane >= d)
-      incl += v;
-  }
-  const bool spill = __ballot(cnt > kInlineRows) != 0;
-  __syncthreads();
-  if (lane == 63)
-    redInt[wave] = incl;
-  if (lane == 0) {
-    red[wave] = k;
-    red[W + wave] = p;
-    red[2 * W + wave] = x;
-    red[3 * W + wave] = y;
-    redInt[W + wave] = spill;
-  }
-  __syncthreads();
-  k = red[0];
-  p = red[W];
-  x = red[2 * W];
-  y = red[3 * W];
-  int before = 0, sum = 0;
-  bool any = false;
-  for (int w = 0; w < W; ++w) {
-    if (w > 0) {
-      pairMin(k, p, red[w], red[W + w]);
-      x = minKey(x, red[2 * W + w]);
-      y = minKey(y, red[3 * W + w]);
-    }
-    before += w < wave ? redInt[w] : 0;
-    sum += redInt[w];
-    any |= redInt[W + w] != 0;
-  }
-  start = before + incl - cnt;
-  total = sum;
-  spilled = any;
-}
-
-// Minimum over j in [j0, j1) of denseKey(D(row, j), j), by the whole
-// workgroup (every slot is active before the first merge).
-DEV unsigned long long scanRowSegment(const DenseState &s, int row, int j0, int j1,
-                                      unsigned long long *red) {
-  unsigned long long best = kEmptyKey;
-  const size_t base = condensedIndex(row, row + 1, s.n) - (size_t)(row + 1);
-  for (int j = j0 + (int)threadIdx.x; j < j1; j += kThreads)
-    best = minKey(best, denseKey(s.D[base + j], (unsigned)j));
-  return blockMinKey(best, red);
+// Adds (lowest, next) of a part of a row to the row's two lowest keys: of the
+// minima, every one but the last is displaced into next.
+DEV void offerAtomic(unsigned long long *lowest, unsigned long long *next,
+                     unsigned long long partLowest, unsigned long long partNext) {
+  if (partLowest == kEmptyKey)
+    return;
+  const unsigned long long old = atomicMin(lowest, partLowest);
+  const unsigned long long displaced = minKey(partNext, old < partLowest ? partLowest : old);
+  if (displaced != kEmptyKey)
+    atomicMin(next, displaced);
 }
 
 __global__ void __launch_bounds__(kThreads) denseInitKernel(DenseState s, int numItems) {
   __shared__ unsigned long long red[kThreads / 64];
-  // Work item t: row r, chunk c, enumerated row by row.
+  // Work item t: row r, chunk c, enumerated row by row (every slot is active).
   for (int t = blockIdx.x; t < numItems; t += gridDim.x) {
     const int2 it = s.items[t];
     const int j1 = min(s.n, it.y + kChunk);
-    const unsigned long long k = scanRowSegment(s, it.x, it.y, j1, red);
-    if (threadIdx.x == 0 && k != kEmptyKey)
-      atomicMin(&s.fnKey[it.x], k);
+    unsigned long long lowest = kEmptyKey, next = kEmptyKey;
+    const size_t base = condensedIndex(it.x, it.x + 1, s.n) - (size_t)(it.x + 1);
+    for (int j = it.y + (int)threadIdx.x; j < j1; j += kThreads)
+      offer(lowest, next, denseKey(s.D[base + j], (unsigned)j));
+    const unsigned long long k = blockMinKey(lowest, red);
+    const unsigned long long k2 = blockMinKey(lowest == k ? next : lowest, red);
+    if (threadIdx.x == 0)
+      offerAtomic(&s.scanned[it.x], &s.scanned[s.n + it.x], k, k2);
   }
 }
 
@@ -341,55 +255,106 @@ DEV bool isActive(const unsigned int *activeBits, int j) {
   return (activeBits[j >> 5] >> (j & 31)) & 1u;
 }
 
-// Minimum over active j in [j0, j1) (at most kRescanChunk columns), j != skip,
-// of denseKey(D(row, j), j), by the whole workgroup, every load issued
-// before the first compare.
-DEV unsigned long long scanRescanChunk(const DenseState &s, const unsigned int *activeBits,
-                                       int row, int j0, int j1, int skip,
-                                       unsigned long long *red) {
-  const size_t base = condensedIndex(row, row + 1, s.n) - (size_t)(row + 1);
-  float v[kRescanPer];
-#pragma unroll
-  for (int u = 0; u < kRescanPer; ++u) {
-    const int j = j0 + (int)threadIdx.x + u * kThreads;
-    v[u] = j < j1 ? s.D[base + j] : 0.0f;
-  }
-  unsigned long long best = kEmptyKey;
-#pragma unroll
-  for (int u = 0; u < kRescanPer; ++u) {
-    const int j = j0 + (int)threadIdx.x + u * kThreads;
-    if (j < j1 && j != skip && isActive(activeBits, j))
-      best = minKey(best, denseKey(v[u], (unsigned)j));
-  }
-  return blockMinKey(best, red);
+// Wave-wide minima by DPP row shifts and broadcasts (lane 63 ends with the
+// minimum; lanes without a source keep all ones): a step costs a few VALU
+// instructions instead of an LDS permute's round trip.
+template <int CTRL> DEV unsigned int dppMin(unsigned int v) {
+  return min(v, (unsigned int)__builtin_amdgcn_update_dpp(-1, (int)v, CTRL, 0xf, 0xf, false));
+}
+template <int CTRL> DEV unsigned long long dppMin(unsigned long long v) {
+  const unsigned int lo =
+      (unsigned int)__builtin_amdgcn_update_dpp(-1, (int)(unsigned int)v, CTRL, 0xf, 0xf, false);
+  const unsigned int hi = (unsigned int)__builtin_amdgcn_update_dpp(
+      -1, (int)(unsigned int)(v >> 32), CTRL, 0xf, 0xf, false);
+  return minKey(v, ((unsigned long long)hi << 32) | lo);
+}
+template <class V> DEV V dppMinAll(V v) {
+  v = dppMin<0x111>(v); // row_shr:1, 2, 4, 8: lane 15 of each row
+  v = dppMin<0x112>(v);
+  v = dppMin<0x114>(v);
+  v = dppMin<0x118>(v);
+  v = dppMin<0x142>(v); // row_bcast:15, then 31
+  return dppMin<0x143>(v);
+}
+DEV unsigned int waveMinBits(unsigned int v) {
+  return (unsigned int)__builtin_amdgcn_readlane((int)dppMinAll(v), 63);
+}
+DEV unsigned long long waveMinKey(unsigned long long v) {
+  v = dppMinAll(v);
+  const unsigned int lo = (unsigned int)__builtin_amdgcn_readlane((int)(unsigned int)v, 63);
+  const unsigned int hi = (unsigned int)__builtin_amdgcn_readlane((int)(unsigned int)(v >> 32), 63);
+  return ((unsigned long long)hi << 32) | lo;
 }
 
+// The two lowest keys over the wave.
+DEV void waveLowest2(unsigned long long &lowest, unsigned long long &next) {
+  const unsigned long long low = waveMinKey(lowest);
+  next = waveMinKey(lowest == low ? next : lowest); // keys are distinct, or empty
+  lowest = low;
+}
+
+// LDS written by some lanes of a wave, then read by others of the same wave.
+DEV void waveSync() {
+  __builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront");
+  __builtin_amdgcn_wave_barrier();
+  __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "wavefront");
+}
+
+// Bound by latency: two grid barriers (2.7 us each) and a dozen dependent
+// memory and LDS round trips per batch at small n; by the column reads
+// (64-byte lines around scattered 4-byte entries) at large n. One merge per
+// barrier took 14.0 us per merge at n = 5,003 and 15.8 us at n = 100,000;
+// batches take 2.2 us (437 batches of 25 us) and 5.8 us.
+// Keeping a bound below a row's other keys beside its fn (instead of its old
+// fn as a pending row's bound) took n = 5,003 from 610 batches to 437: fewer
+// selections meet a pending row. One instantiation per linkage, short loops
+// left rolled: the batch's code should stay in the 64 KB instruction cache.
+template <int LINKAGE>
 __global__ void __launch_bounds__(kThreads) denseMergeKernel(DenseState s) {
-  extern __shared__ unsigned int activeBits[]; // (n + 31) / 32 words: bit j = slot j active
-  __shared__ unsigned long long ownFn[kMaxOwned];
+  static_assert(kMaxBatch * kTop == 64, "the batch's candidates fill one wave");
+  constexpr int kSorted = 32; // candidates examined in order, retired rows included
+  // [0, (n + 31) / 32): bit j = slot j active; then the new distances
+  // [batch][per] of the batch's merges to this workgroup's rows.
+  extern __shared__ unsigned int dynamicLds[];
+  // Per row: its fn, and a lower bound of its other keys (a pending row's fn
+  // is not known: the bound covers all of its keys).
+  __shared__ unsigned long long ownFn[kMaxOwned], ownNext[kMaxOwned];
   __shared__ int ownSize[kMaxOwned];
+  // -1, or the row's part in the batch: t for slot a of merge t, kMaxBatch + t
+  // for slot b.
+  __shared__ signed char ownSlot[kMaxOwned];
   __shared__ unsigned char ownPending[kMaxOwned];
-  // This workgroup's pending rows of the two latest phases and their
-  // lower-bound keys: list[older] is being (or was) rescanned, list[older ^ 1]
-  // is filled by the current update.
-  __shared__ int pendRow[2][kMaxOwned];
-  __shared__ unsigned long long pendKey[2][kMaxOwned];
-  __shared__ int pendCount[2];
-  // The rows every workgroup made pending in the previous phase:
-  // workgroup w's at [listStart[w], listStart[w + 1]).
+  __shared__ int pendRow[kMaxOwned]; // this workgroup's pending rows
+  __shared__ int pendCount;
+  // Every workgroup's pending rows: workgroup w's at [listStart[w], listStart[w + 1]).
   __shared__ int listStart[kThreads + 1];
   __shared__ int listRows[kInlineRows * kThreads];
-  __shared__ unsigned long long redK[kThreads / 64], redP[kThreads / 64];
-  __shared__ unsigned long long red4[5 * (kThreads / 64)];
-  __shared__ int redInt[2 * (kThreads / 64)];
+  __shared__ __align__(16) unsigned long long heads[kThreads]; // lowest key per workgroup
+  __shared__ int headRank[kThreads];
+  __shared__ __align__(16) unsigned long long cand[64];
+  __shared__ unsigned int candCol[64];
+  __shared__ unsigned long long sorted[kSorted];
+  __shared__ unsigned int sortedCol[kSorted];
+  __shared__ int slotA[kMaxBatch], slotB[kMaxBatch], sizeA[kMaxBatch], sizeB[kMaxBatch];
+  __shared__ int idA[kMaxBatch], idB[kMaxBatch];
+  __shared__ float dist[kMaxBatch];
+  __shared__ unsigned long long rowFn[kMaxBatch], rowNext[kMaxBatch];
+  __shared__ unsigned int newMin[kMaxBatch];
+  __shared__ int batchCount; // merges in the batch, or -1: no pair is left
+  __shared__ unsigned long long waveKey[2 * kWaves];
+  __shared__ int waveInt[2 * kWaves];
+  __shared__ __align__(16) unsigned long long topKey[kWaves * kTop];
   __shared__ int barrierOk;
-  const int n = s.n;
+
+  const int n = s.n, per = s.per;
   const int G = gridDim.x, g = blockIdx.x;
-  const int tid = threadIdx.x;
-  const int per = (n + G - 1) / G;
-  const int mine0 = min(n, g * per), mine1 = min(n, mine0 + per);
+  const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
+  const int mine0 = min(n, g * per), mine1 = min(n, mine0 + per), rows = mine1 - mine0;
   const int words = (n + 31) >> 5;
-  const int maxChunks = (n - 1 + kRescanChunk - 1) / kRescanChunk;
+  unsigned int *activeBits = dynamicLds;
+  float *newDist = reinterpret_cast<float *>(dynamicLds + words);
+  const int maxChunks = (n - 1 + kRescanCols - 1) / kRescanCols;
+  const int rankers = kThreads / G, rankSpan = (G + rankers - 1) / rankers;
   unsigned int generation = 0;
   const bool clocked = s.clocks && g == 0 && tid == 0;
   unsigned long long ticks[4] = {0, 0, 0, 0}, t0 = 0;
@@ -400,45 +365,72 @@ __global__ void __launch_bounds__(kThreads) denseMergeKernel(DenseState s) {
       t0 = t;
     }
   };
-  int published = 0; // publishes so far: the latest is in buffer (published - 1) & 1
-  auto recordsOf = [&](int buffer) { return s.records + (size_t)buffer * G * kRecordWords; };
-  auto pendingOf = [&](int buffer) { return s.pendingRows + (size_t)buffer * G * kMaxOwned; };
-  // Publishes this workgroup's record: settled rows, row-a part, pending
-  // lower bound, and the rows made pending in this phase (list[older ^ 1]);
-  // folds this thread's part of a rescan chunk of row chunkRow (-1: none) into
-  // that row's result in the same reduction.
-  auto publish = [&](unsigned long long selK, unsigned long long selP,
-                     unsigned long long rowA, int older, unsigned long long chunkMin,
-                     int chunkRow) {
-    const int buffer = published & 1;
-    unsigned long long *record = recordsOf(buffer) + (size_t)g * kRecordWords;
-    unsigned long long pmin = kEmptyKey;
-    for (int l = 0; l < 2; ++l)
-      for (int i = tid; i < pendCount[l]; i += kThreads)
-        if (isActive(activeBits, pendRow[l][i]))
-          pmin = minKey(pmin, pendKey[l][i]);
-    blockReduce5(selK, selP, rowA, pmin, chunkMin, red4);
-    if (tid == 0 && chunkRow >= 0 && chunkMin != kEmptyKey)
-      atomicMin(&s.fnRescan[chunkRow], chunkMin);
-    const int fresh = older ^ 1, count = pendCount[fresh];
-    if (count > kInlineRows)
-      for (int i = tid; i < count; i += kThreads)
-        pendingOf(buffer)[(size_t)g * kMaxOwned + i] = pendRow[fresh][i];
-    if (tid == 0) {
-      record[0] = selK;
-      record[1] = selP;
-      record[2] = rowA;
-      record[3] = pmin;
-      record[4] = (unsigned long long)count;
-      for (int w = 0; w < kInlineRows / 2; ++w) {
-        const int r0 = 2 * w < count ? pendRow[fresh][2 * w] : 0;
-        const int r1 = 2 * w + 1 < count ? pendRow[fresh][2 * w + 1] : 0;
-        record[5 + w] = (unsigned long long)(unsigned)r0 | ((unsigned long long)(unsigned)r1 << 32);
-      }
-    }
-    ++published;
+  auto entry = [&](int i, int j) -> size_t {
+    return i < j ? condensedIndex(i, j, n) : condensedIndex(j, i, n);
   };
-  // The q-th row of the previous phase's pending list (listStart ready).
+
+  // This workgroup's kTop lowest settled rows, wave by wave (thread t looks
+  // at rows t, t + kThreads, ...; keys are distinct, so the next lowest is the
+  // lowest above the last).
+  auto waveTop = [&]() {
+    auto keyOf = [&](int r) {
+      return r < rows && !ownPending[r] ? selectionKey(ownFn[r], mine0 + r) : kEmptyKey;
+    };
+    const unsigned long long first = keyOf(tid); // most workgroups own at most kThreads rows
+    unsigned long long last = 0;
+    for (int q = 0; q < kTop; ++q) {
+      unsigned long long best = q == 0 || first > last ? first : kEmptyKey;
+      for (int r = tid + kThreads; r < rows; r += kThreads) {
+        const unsigned long long key = keyOf(r);
+        if (q == 0 || key > last)
+          best = minKey(best, key);
+      }
+      best = waveMinKey(best);
+      if (lane == 0)
+        topKey[wave * kTop + q] = best;
+      last = best;
+    }
+  };
+  // After a barrier behind waveTop: the record, by wave 0.
+  auto writeRecord = [&]() {
+    if (wave != 0)
+      return;
+    unsigned long long *rec = s.records + (size_t)g * kRecordWords;
+    const unsigned long long key = lane < kWaves * kTop ? topKey[lane] : kEmptyKey;
+    // A wave's keys are in order; only the waves that own rows have any.
+    const int listed = min(kWaves, (rows + 63) / 64) * kTop;
+    int rank = lane;
+    if (listed > kTop) {
+      rank = 0;
+#pragma unroll 4
+      for (int j = 0; j < listed; ++j) {
+        const unsigned long long other = topKey[j];
+        rank += other < key || (other == key && j < lane);
+      }
+      if (lane >= listed)
+        rank = kTop;
+    }
+    if (rank < kTop) {
+      rec[rank] = key;
+      reinterpret_cast<unsigned int *>(rec + kTop)[rank] =
+          key == kEmptyKey ? 0u : (unsigned int)ownFn[keyIndex(key) - mine0];
+    }
+    const int count = pendCount;
+    unsigned long long bound = kEmptyKey;
+    for (int i = lane; i < count; i += 64)
+      bound = minKey(bound, selectionKey(ownNext[pendRow[i] - mine0], pendRow[i]));
+    bound = waveMinKey(bound);
+    if (lane == 0) {
+      rec[6] = bound;
+      rec[7] = (unsigned long long)count;
+    }
+    if (lane < kInlineRows / 2) {
+      const int r0 = 2 * lane < count ? pendRow[2 * lane] : 0;
+      const int r1 = 2 * lane + 1 < count ? pendRow[2 * lane + 1] : 0;
+      rec[8 + lane] = (unsigned long long)(unsigned)r0 | ((unsigned long long)(unsigned)r1 << 32);
+    }
+  };
+  // The q-th row of all pending rows (listStart ready).
   auto listRow = [&](int q, bool spilled) {
     if (!spilled)
       return listRows[q];
@@ -451,314 +443,502 @@ __global__ void __launch_bounds__(kThreads) denseMergeKernel(DenseState s) {
         hi = mid;
     }
     const int i = q - listStart[lo];
-    const int buffer = (published - 1) & 1;
     if (listStart[lo + 1] - listStart[lo] > kInlineRows)
-      return pendingOf(buffer)[(size_t)lo * kMaxOwned + i];
-    const unsigned long long w = recordsOf(buffer)[(size_t)lo * kRecordWords + 5 + i / 2];
+      return s.pendingRows[(size_t)lo * per + i];
+    const unsigned long long w = s.records[(size_t)lo * kRecordWords + 8 + i / 2];
     return (int)(unsigned)(i & 1 ? w >> 32 : w);
   };
-  // Rescans of the listed rows, shared by all workgroups in column chunks:
-  // item t is chunk t % maxChunks of list row t / maxChunks. Column skip
-  // (the merged slot, whose entries their owners are rewriting) is left out.
-  auto rescans = [&](int count, bool spilled, int skip, long long first) {
-    const long long numItems = (long long)count * maxChunks;
-    for (long long t = first; t < numItems; t += G) {
-      const int r = listRow((int)(t / maxChunks), spilled);
-      const int j0 = r + 1 + (int)(t % maxChunks) * kRescanChunk;
-      if (j0 >= n || !isActive(activeBits, r))
-        continue;
-      const unsigned long long m =
-          scanRescanChunk(s, activeBits, r, j0, min(n, j0 + kRescanChunk), skip, redK);
-      if (tid == 0 && m != kEmptyKey)
-        atomicMin(&s.fnRescan[r], m);
-    }
-  };
-  // Settles this workgroup's rows of list[l]: their fn is the rescan's result.
-  auto install = [&](int l) {
-    for (int i = tid; i < pendCount[l]; i += kThreads) {
-      const int r = pendRow[l][i];
-      ownPending[r - mine0] = 0;
-      ownFn[r - mine0] = isActive(activeBits, r) ? s.fnRescan[r] : kEmptyKey;
-    }
-    __syncthreads();
-    if (tid == 0)
-      pendCount[l] = 0;
-  };
-  // The settled rows' minimum (selection key, fn), all rows but skipRow.
-  auto settledMin = [&](unsigned long long &k, unsigned long long &p, int skipRow) {
-    for (int i = mine0 + tid; i < mine1; i += kThreads)
-      if (i != skipRow && !ownPending[i - mine0] && isActive(activeBits, i))
-        pairMin(k, p, selectionKey(ownFn[i - mine0], i), ownFn[i - mine0]);
-  };
 
-  // Every slot starts active and settled; this workgroup's rows' state moves
-  // to LDS, and the records of merge 0 come from the initial fn.
+  // Every slot starts active and settled.
   for (int w = tid; w < words; w += kThreads) {
     const int rest = n - 32 * w;
     activeBits[w] = rest >= 32 ? 0xffffffffu : (1u << rest) - 1u;
   }
-  for (int i = mine0 + tid; i < mine1; i += kThreads) {
-    ownFn[i - mine0] = s.fnKey[i];
-    ownSize[i - mine0] = s.size[i];
-    ownPending[i - mine0] = 0;
+  for (int r = tid; r < rows; r += kThreads) {
+    ownFn[r] = s.scanned[mine0 + r];
+    ownNext[r] = s.scanned[n + mine0 + r];
+    ownSize[r] = s.size[mine0 + r];
+    ownSlot[r] = -1;
+    ownPending[r] = 0;
   }
-  if (tid < 2)
-    pendCount[tid] = 0;
+  if (tid == 0)
+    pendCount = 0;
+  waveTop();
   __syncthreads();
-  int older = 0;
-  {
-    unsigned long long k = kEmptyKey, p = kEmptyKey;
-    settledMin(k, p, -1);
-    publish(k, p, kEmptyKey, older, kEmptyKey, -1);
-  }
+  writeRecord();
   if (!gridBarrier(s.bar, generation, &barrierOk))
     return;
   if (clocked)
     t0 = wall_clock64();
 
-  int prevA = -1, prevSize = 0; // the previous merge's slot a and merged size
-  for (int step = 0; step < n - 1; ++step) {
-    // This phase's inputs are loaded together: the latest records, and the
-    // rescan results of this workgroup's rows rescanned in the previous phase.
-    unsigned long long k = kEmptyKey, p = kEmptyKey, part = kEmptyKey, pmin = kEmptyKey;
+  for (int done = 0; done < n - 1;) {
+    // ---- First half: select the batch.
+    unsigned long long sel[kTop], bound = kEmptyKey;
+    unsigned int col[kTop] = {};
     int cnt = 0;
     int inl[kInlineRows] = {};
+#pragma unroll
+    for (int q = 0; q < kTop; ++q)
+      sel[q] = kEmptyKey;
     if (tid < G) {
-      const unsigned long long *r = recordsOf((published - 1) & 1) + (size_t)tid * kRecordWords;
+      const ulonglong2 *r =
+          reinterpret_cast<const ulonglong2 *>(s.records + (size_t)tid * kRecordWords);
       unsigned long long w[kRecordWords];
 #pragma unroll
-      for (int i = 0; i < kRecordWords; ++i)
-        w[i] = r[i];
-      k = w[0];
-      p = w[1];
-      part = w[2];
-      pmin = w[3];
-      cnt = (int)w[4];
+      for (int i = 0; i < kRecordWords / 2; ++i) {
+        const ulonglong2 v = r[i];
+        w[2 * i] = v.x;
+        w[2 * i + 1] = v.y;
+      }
+#pragma unroll
+      for (int q = 0; q < kTop; ++q) {
+        sel[q] = w[q];
+        col[q] = (unsigned)(w[kTop + q / 2] >> (32 * (q & 1)));
+      }
+      bound = w[6];
+      cnt = (int)w[7];
 #pragma unroll
       for (int i = 0; i < kInlineRows / 2; ++i) {
-        inl[2 * i] = (int)(unsigned)w[5 + i];
-        inl[2 * i + 1] = (int)(unsigned)(w[5 + i] >> 32);
+        inl[2 * i] = (int)(unsigned)w[8 + i];
+        inl[2 * i + 1] = (int)(unsigned)(w[8 + i] >> 32);
       }
     }
-    const int numInstall = pendCount[older];
-    int installRow = -1;
-    unsigned long long installFn = kEmptyKey;
-    if (tid < numInstall) {
-      installRow = pendRow[older][tid];
-      installFn = s.fnRescan[installRow];
+    heads[tid] = sel[0];
+    headRank[tid] = 0;
+    if (tid < 64)
+      cand[tid] = kEmptyKey;
+    if (tid < kMaxBatch) {
+      rowFn[tid] = kEmptyKey;
+      rowNext[tid] = kEmptyKey;
+      newMin[tid] = 0xffffffffu;
     }
-    // Every workgroup reduces the records the same way. The previous merged
-    // row's new fn is the minimum of the parts.
-    int listCount = 0, start = 0;
+    // A workgroup's rows beyond its kTop lowest are not listed: no key above
+    // such a workgroup's last listed one may be taken.
+    unsigned long long guard = waveMinKey(sel[kTop - 1]);
+    bound = waveMinKey(bound);
+    int incl = cnt;
+#pragma unroll
+    for (int d = 1; d < 64; d <<= 1) {
+      const int v = __shfl_up(incl, d, 64);
+      if (lane >= d)
+        incl += v;
+    }
+    const bool spill = __ballot(cnt > kInlineRows) != 0;
+    if (lane == 0) {
+      waveKey[wave] = bound;
+      waveKey[kWaves + wave] = guard;
+      waveInt[kWaves + wave] = spill;
+    }
+    if (lane == 63)
+      waveInt[wave] = incl;
+    __syncthreads();
+    int start = incl - cnt, listCount = 0;
     bool spilled = false;
-    blockReduce4Scan(k, p, part, pmin, cnt, start, listCount, spilled, red4, redInt);
-    if (prevA >= 0)
-      pairMin(k, p, selectionKey(part, prevA), part);
+#pragma unroll
+    for (int w = 0; w < kWaves; ++w) {
+      bound = minKey(bound, waveKey[w]);
+      guard = minKey(guard, waveKey[kWaves + w]);
+      start += w < wave ? waveInt[w] : 0;
+      listCount += waveInt[w];
+      spilled |= waveInt[kWaves + w] != 0;
+    }
     if (tid < G) {
       listStart[tid] = start;
       if (!spilled)
         for (int i = 0; i < cnt; ++i)
           listRows[start + i] = inl[i];
     }
-    if (tid == 0) {
+    if (tid == 0)
       listStart[G] = listCount;
-      pendCount[older] = 0;
-      if (prevA >= mine0 && prevA < mine1) {
-        ownFn[prevA - mine0] = part;
-        ownSize[prevA - mine0] = prevSize;
-        s.size[prevA] = prevSize;
-        s.id[prevA] = s.firstNewId + step - 1;
-      }
-    }
-    // Rows rescanned in the previous phase settle; this phase's list is new.
-    if (installRow >= 0) {
-      ownPending[installRow - mine0] = 0;
-      ownFn[installRow - mine0] = isActive(activeBits, installRow) ? installFn : kEmptyKey;
-    }
-    for (int i = kThreads + tid; i < numInstall; i += kThreads) {
-      const int r = pendRow[older][i];
-      ownPending[r - mine0] = 0;
-      ownFn[r - mine0] = isActive(activeBits, r) ? s.fnRescan[r] : kEmptyKey;
+    // The kMaxBatch lowest heads' workgroups hold the kMaxBatch lowest keys:
+    // each head's rank, by kThreads / G threads per head.
+    if (tid < rankers * G) {
+      const int i = tid % G, lo = tid / G * rankSpan, hi = min(G, lo + rankSpan);
+      const unsigned long long key = heads[i];
+      int below = 0;
+#pragma unroll 8
+      for (int j = lo; j < hi; ++j)
+        below += heads[j] < key;
+      if (below)
+        atomicAdd(&headRank[i], below);
     }
     __syncthreads();
-    older ^= 1;
-    bool rescanned = false;
-    if (!(k < pmin)) {
-      // A pending row could hold the lowest key: rescan the previous phase's
-      // rows now, settle every pending row, and select again from records
-      // that hold no pending row (two extra barriers; rare).
-      rescans(listCount, spilled, -1, g);
-      if (!gridBarrier(s.bar, generation, &barrierOk))
-        return;
-      install(older);
-      unsigned long long k2 = kEmptyKey, p2 = kEmptyKey;
-      settledMin(k2, p2, -1);
-      publish(k2, p2, kEmptyKey, older, kEmptyKey, -1);
-      if (!gridBarrier(s.bar, generation, &barrierOk))
-        return;
-      k = kEmptyKey;
-      p = kEmptyKey;
-      if (tid < G) {
-        const unsigned long long *r = recordsOf((published - 1) & 1) + (size_t)tid * kRecordWords;
-        k = r[0];
-        p = r[1];
+    if (tid < G && sel[0] != kEmptyKey) {
+      const int r = headRank[tid];
+      if (r < kMaxBatch) {
+#pragma unroll
+        for (int q = 0; q < kTop; ++q) {
+          cand[r * kTop + q] = sel[q];
+          candCol[r * kTop + q] = col[q];
+        }
       }
-      blockMinPair(k, p, redK, redP);
-      rescanned = true;
     }
-    const int a = k == kEmptyKey ? -1 : keyIndex(k);
-    const int b = p == kEmptyKey ? -1 : keyIndex(p);
-    if (a < 0 || b <= a || b >= n) {
+    __syncthreads();
+    if (wave == 0) {
+      const unsigned long long key = cand[lane];
+      // Nor any key above the last of the chosen heads: a workgroup that is
+      // not among them may have a lower one.
+      guard = minKey(guard, cand[(kMaxBatch - 1) * kTop]);
+      int rank = 0;
+#pragma unroll 8
+      for (int j = 0; j < 64; ++j) {
+        const unsigned int lo = (unsigned)__builtin_amdgcn_readlane((int)(unsigned)key, j);
+        const unsigned int hi = (unsigned)__builtin_amdgcn_readlane((int)(unsigned)(key >> 32), j);
+        rank += (((unsigned long long)hi << 32) | lo) < key;
+      }
+      const int valid = min(kSorted, __popcll(__ballot(key != kEmptyKey)));
+      if (key != kEmptyKey && rank < kSorted) {
+        sorted[rank] = key;
+        sortedCol[rank] = candCol[lane];
+      }
+      waveSync();
+      // Lane t looks at the t-th lowest row. It ends the batch if its column
+      // is a slot of an earlier pair of the batch; if the row itself is an
+      // earlier pair's slot b, it retires with that merge and is passed over.
+      const bool have = lane < valid;
+      const unsigned long long k = have ? sorted[lane] : kEmptyKey;
+      const int i = keyIndex(k), j = have ? (int)sortedCol[lane] : -1;
+      unsigned long long stop = __ballot(!have || !(k < bound) || k > guard), retired = 0;
+      for (int t = 0; !(stop >> t & 1); ++t) { // lane 63 always stops
+        if (retired >> t & 1)
+          continue;
+        const int ti = __builtin_amdgcn_readlane(i, t), tj = __builtin_amdgcn_readlane(j, t);
+        const unsigned long long after = ~1ull << t;
+        stop |= (__ballot(j == ti) | __ballot(j == tj)) & after;
+        retired |= __ballot(i == tj) & after;
+      }
+      const unsigned long long inMask = ((stop & -stop) - 1) & ~retired;
+      const bool in = inMask >> lane & 1;
+      const int at = __popcll(inMask & ((1ull << lane) - 1));
+      if (in && at < s.batch) {
+        slotA[at] = i;
+        slotB[at] = j;
+        dist[at] = fromOrderedBits((unsigned)(k >> 32));
+        if (i >= mine0 && i < mine1)
+          ownSlot[i - mine0] = (signed char)at;
+        if (j >= mine0 && j < mine1)
+          ownSlot[j - mine0] = (signed char)(kMaxBatch + at);
+      }
+      if (lane == 0)
+        batchCount = valid == 0 && bound == kEmptyKey ? -1 : min(s.batch, __popcll(inMask));
+    } else {
+      // The pending rows are scanned again (no distance is written in this
+      // half), one column chunk per wave and step.
+      const unsigned int numItems = (unsigned)listCount * (unsigned)maxChunks;
+      for (unsigned int t = (unsigned)((wave - 1) * G + g); t < numItems;
+           t += (unsigned)((kWaves - 1) * G)) {
+        const unsigned int q = t / (unsigned)maxChunks;
+        const int r = listRow((int)q, spilled);
+        const int j0 = r + 1 + (int)(t - q * (unsigned)maxChunks) * kRescanCols;
+        if (j0 >= n)
+          continue;
+        const size_t base = condensedIndex(r, r + 1, n) - (size_t)(r + 1);
+        float v[kRescanPer];
+#pragma unroll
+        for (int u = 0; u < kRescanPer; ++u) {
+          const int j = j0 + lane + u * 64;
+          v[u] = j < n ? s.D[base + j] : 0.0f;
+        }
+        unsigned long long lowest = kEmptyKey, next = kEmptyKey;
+#pragma unroll
+        for (int u = 0; u < kRescanPer; ++u) {
+          const int j = j0 + lane + u * 64;
+          if (j < n && isActive(activeBits, j))
+            offer(lowest, next, denseKey(v[u], (unsigned)j));
+        }
+        waveLowest2(lowest, next);
+        if (lane == 0)
+          offerAtomic(&s.scanned[r], &s.scanned[n + r], lowest, next);
+      }
+    }
+    __syncthreads();
+    const int m = batchCount;
+    if (m < 0) {
       // No pair (non-finite distances): the remaining rows report -1. Every
       // workgroup reduced the same records, so all of them stop here.
       if (g == 0)
-        for (int r = step + tid; r < n - 1; r += kThreads)
+        for (int r = done + tid; r < n - 1; r += kThreads)
           for (int c = 0; c < 4; ++c)
             s.tree[(size_t)r * 4 + c] = -1.0;
       break;
     }
-    const float dab = fromOrderedBits((unsigned)(p >> 32));
-    // Sizes and ids in memory are at least one phase old; the previous
-    // merge's cluster is known here. Their loads join the update's loads.
-    const int na = a == prevA ? prevSize : s.size[a];
-    const int nb = b == prevA ? prevSize : s.size[b];
-    int ia = 0, ib = 0;
-    if (g == 0 && tid == 0) {
-      const int prevId = s.firstNewId + step - 1;
-      ia = a == prevA ? prevId : s.id[a];
-      ib = b == prevA ? prevId : s.id[b];
-    }
-    // The update skips b itself, so its bit is cleared without a barrier
-    // here (the next one, after the update, publishes it to the rescans).
-    if (tid == 0)
-      activeBits[b >> 5] &= ~(1u << (b & 31));
-    // The first rescan item of this workgroup: its loads are issued before
-    // the update (no entry it reads is written in this phase but D(row, a),
-    // which the scan leaves out).
-    const long long numItems = rescanned ? 0 : (long long)listCount * maxChunks;
-    int firstRow = -1, firstJ0 = n;
-    float firstV[kRescanPer];
-    if (g < numItems) {
-      firstRow = listRow(g / maxChunks, spilled);
-      firstJ0 = firstRow + 1 + (g % maxChunks) * kRescanChunk;
-      if (firstJ0 < n) {
-        const size_t base = condensedIndex(firstRow, firstRow + 1, n) - (size_t)(firstRow + 1);
-#pragma unroll
-        for (int u = 0; u < kRescanPer; ++u) {
-          const int j = firstJ0 + tid + u * kThreads;
-          firstV[u] = j < n && j < firstJ0 + kRescanChunk ? s.D[base + j] : 0.0f;
-        }
-      }
-    }
+    const int numInstall = pendCount;
     lap(0);
 
-    // Lance-Williams update of D(a, k) for this workgroup's k, its settled
-    // rows' fn, and its part of row a's new fn.
-    unsigned long long rowAMin = kEmptyKey, selK = kEmptyKey, selP = kEmptyKey;
-    const int fresh = older ^ 1;
-    // Rows in batches of kUpdatePer per thread, every load of a batch issued
-    // before the first is used: one memory round trip per batch.
-    for (int batch = mine0; batch < mine1; batch += kUpdatePer * kThreads) {
-      bool live[kUpdatePer];
-      size_t iakOf[kUpdatePer];
-      float dakOf[kUpdatePer], dbkOf[kUpdatePer];
+    // The new distances of this workgroup's rows, a wave per merge.
+    for (int t = wave; t < m; t += kWaves) {
+      const int a = slotA[t], b = slotB[t];
+      // The sizes (and, for the tree, the ids) arrive with the distances.
+      const int na = s.size[a], nb = s.size[b];
+      int ia = 0, ib = 0;
+      if (g == 0) {
+        ia = s.id[a];
+        ib = s.id[b];
+      }
+      const float dab = dist[t];
+      unsigned long long part = kEmptyKey, partNext = kEmptyKey;
+      unsigned int lowest = 0xffffffffu;
+      for (int base = lane; base < rows; base += 64 * kUpdatePer) {
+        bool live[kUpdatePer];
+        float dak[kUpdatePer], dbk[kUpdatePer];
 #pragma unroll
-      for (int u = 0; u < kUpdatePer; ++u) {
-        const int kk = batch + tid + u * kThreads;
-        live[u] = kk < mine1 && kk != a && kk != b && isActive(activeBits, kk);
-        if (live[u]) {
-          iakOf[u] = kk < a ? condensedIndex(kk, a, n) : condensedIndex(a, kk, n);
-          const size_t ibk = kk < b ? condensedIndex(kk, b, n) : condensedIndex(b, kk, n);
-          dakOf[u] = s.D[iakOf[u]];
-          dbkOf[u] = s.D[ibk];
+        for (int u = 0; u < kUpdatePer; ++u) {
+          const int r = base + 64 * u, k = mine0 + r;
+          // Slot b of an earlier merge has retired by this one; slot a of an
+          // earlier merge follows below.
+          const int slot = r < rows ? ownSlot[r] : 0;
+          live[u] = r < rows && k != a && k != b && isActive(activeBits, k) &&
+                    !(slot >= 0 && (slot & (kMaxBatch - 1)) < t);
+          if (live[u]) {
+            dak[u] = s.D[entry(a, k)];
+            dbk[u] = s.D[entry(b, k)];
+          }
+        }
+#pragma unroll
+        for (int u = 0; u < kUpdatePer; ++u) {
+          if (!live[u])
+            continue;
+          const int r = base + 64 * u, k = mine0 + r;
+          const float nd = lanceWilliams<LINKAGE>(dak[u], dbk[u], dab, na, nb, ownSize[r]);
+          if (ownSlot[r] < 0 && k > a)
+            offer(part, partNext, denseKey(nd, (unsigned)k));
+          newDist[t * per + r] = nd;
+          lowest = min(lowest, orderedBits(nd));
         }
       }
-#pragma unroll
-      for (int u = 0; u < kUpdatePer; ++u) {
-        if (!live[u])
-          continue;
-        const int kk = batch + tid + u * kThreads;
-        const size_t iak = iakOf[u];
-        const float dak = dakOf[u], dbk = dbkOf[u];
-        const unsigned long long f = ownFn[kk - mine0];
-        const float nd =
-            (float)lanceWilliams(s.linkage, dak, dbk, dab, na, nb, ownSize[kk - mine0]);
-        s.D[iak] = nd;
-        if (kk > a)
-          rowAMin = minKey(rowAMin, denseKey(nd, (unsigned)kk));
-        if (ownPending[kk - mine0]) {
-          // Being rescanned without column a: its new D(kk, a) joins here.
-          if (kk < a)
-            atomicMin(&s.fnRescan[kk], denseKey(nd, (unsigned)a));
-          continue;
-        }
-        unsigned long long nf = f;
-        bool rescan = false;
-        if (kk < a) {
-          // Every entry of row kk but D(kk, a) and D(kk, b) is unchanged.
-          const int fk = f == kEmptyKey ? -1 : keyIndex(f);
-          const unsigned long long cand = denseKey(nd, (unsigned)a);
-          if (fk == a || fk == b) {
-            // The other entries were >= the old minimum, and any equal one has
-            // a higher column than b: (nd, a) is the minimum if nd is no larger.
-            if (orderedBits(nd) <= (unsigned)(f >> 32))
-              nf = cand;
-            else
-              rescan = true;
-          } else if (cand < f) {
-            nf = cand;
-          }
-        } else if (kk < b && f != kEmptyKey && keyIndex(f) == b) {
-          rescan = true; // its nearest retired
-        }
-        if (rescan) {
-          // Pending until the next phase's rescan; its new key is at least
-          // the old one (every linkage here is reducible).
-          const int r = atomicAdd(&pendCount[fresh], 1);
-          pendRow[fresh][r] = kk;
-          pendKey[fresh][r] = selectionKey(f, kk);
-          ownPending[kk - mine0] = 1;
-          s.fnRescan[kk] = kEmptyKey;
-          nf = kEmptyKey;
-        } else {
-          pairMin(selK, selP, selectionKey(nf, kk), nf);
-        }
-        ownFn[kk - mine0] = nf;
+      waveLowest2(part, partNext);
+      lowest = waveMinBits(lowest);
+      if (lane == 0) {
+        sizeA[t] = na;
+        sizeB[t] = nb;
+        idA[t] = ia;
+        idB[t] = ib;
+        atomicMin(&newMin[t], lowest);
+        offerAtomic(&rowFn[t], &rowNext[t], part, partNext);
       }
     }
-    if (tid == 0 && b >= mine0 && b < mine1)
-      ownFn[b - mine0] = kEmptyKey;
-    if (g == 0 && tid == 0) {
-      double *row = s.tree + (size_t)step * 4;
-      row[0] = (double)min(ia, ib);
-      row[1] = (double)max(ia, ib);
-      row[2] = (double)dab;
-      row[3] = (double)(na + nb);
+    // Pairs of merges u < t with slot a_u among this workgroup's rows: merge
+    // u's distances to a_t and b_t first, then merge t's to a_u.
+    if (tid < kMaxBatch * kMaxBatch) {
+      const int t = tid / kMaxBatch, u = tid % kMaxBatch;
+      const int k = u < t && t < m ? slotA[u] : -1;
+      if (k >= mine0 && k < mine1) {
+        const int a = slotA[t], b = slotB[t], kb = slotB[u];
+        const int na = s.size[a], nb = s.size[b], ka = ownSize[k - mine0], kbSize = s.size[kb];
+        const float aa = s.D[entry(k, a)], ab = s.D[entry(k, b)];
+        const float ba = s.D[entry(kb, a)], bb = s.D[entry(kb, b)];
+        const float xa = lanceWilliams<LINKAGE>(aa, ba, dist[u], ka, kbSize, na);
+        const float xb = lanceWilliams<LINKAGE>(ab, bb, dist[u], ka, kbSize, nb);
+        const float nd = lanceWilliams<LINKAGE>(xa, xb, dist[t], na, nb, ka + kbSize);
+        newDist[t * per + k - mine0] = nd;
+        atomicMin(&newMin[t], orderedBits(nd));
+        offerAtomic(&rowFn[a < k ? t : u], &rowNext[a < k ? t : u],
+                    denseKey(nd, (unsigned)max(a, k)), kEmptyKey);
+      }
     }
     __syncthreads();
+    if (tid < m) {
+      s.partFn[tid * G + g] = rowFn[tid];
+      s.partNext[tid * G + g] = rowNext[tid];
+      s.partMin[tid * G + g] = newMin[tid];
+    }
     lap(1);
+    if (!gridBarrier(s.bar, generation, &barrierOk))
+      return;
+    lap(2);
 
-    // The first rescan item, loaded before the update (the same item for
-    // every thread of the workgroup); its minimum joins the record's
-    // reduction.
-    unsigned long long firstMin = kEmptyKey;
-    const bool firstLive = g < numItems && firstJ0 < n && isActive(activeBits, firstRow);
-    if (firstLive) {
-      const int j1 = min(n, firstJ0 + kRescanChunk);
+    // ---- Second half: the valid prefix, committed.
+    if (tid == 0)
+      pendCount = 0;
+    // Every load of the half's start is issued before the first is used.
+    const int installRow = tid < numInstall ? pendRow[tid] : -1;
+    const unsigned long long installFn = installRow >= 0 ? s.scanned[installRow] : kEmptyKey;
+    const unsigned long long installNext =
+        installRow >= 0 ? s.scanned[n + installRow] : kEmptyKey;
+    constexpr int kPerWave = kMaxBatch / kWaves;
+    unsigned long long fn[kPerWave], next[kPerWave];
+    unsigned int lowest[kPerWave];
 #pragma unroll
-      for (int u = 0; u < kRescanPer; ++u) {
-        const int j = firstJ0 + tid + u * kThreads;
-        if (j < j1 && j != a && isActive(activeBits, j))
-          firstMin = minKey(firstMin, denseKey(firstV[u], (unsigned)j));
+    for (int p = 0; p < kPerWave; ++p) {
+      fn[p] = kEmptyKey;
+      next[p] = kEmptyKey;
+      lowest[p] = 0xffffffffu;
+    }
+    for (int w0 = lane; w0 < G; w0 += 256) {
+      unsigned long long f[kPerWave][4], x[kPerWave][4];
+      unsigned int l[kPerWave][4];
+#pragma unroll
+      for (int p = 0; p < kPerWave; ++p)
+#pragma unroll
+        for (int u = 0; u < 4; ++u) {
+          const int t = wave + p * kWaves, w = w0 + 64 * u;
+          const bool in = t < m && w < G;
+          f[p][u] = in ? s.partFn[t * G + w] : kEmptyKey;
+          x[p][u] = in ? s.partNext[t * G + w] : kEmptyKey;
+          l[p][u] = in ? s.partMin[t * G + w] : 0xffffffffu;
+        }
+#pragma unroll
+      for (int p = 0; p < kPerWave; ++p)
+#pragma unroll
+        for (int u = 0; u < 4; ++u) {
+          offer(fn[p], next[p], f[p][u]);
+          next[p] = minKey(next[p], x[p][u]);
+          lowest[p] = min(lowest[p], l[p][u]);
+        }
+    }
+#pragma unroll
+    for (int p = 0; p < kPerWave; ++p) {
+      waveLowest2(fn[p], next[p]);
+      lowest[p] = waveMinBits(lowest[p]);
+      if (lane == 0) {
+        rowFn[wave + p * kWaves] = fn[p];
+        rowNext[wave + p * kWaves] = next[p];
+        newMin[wave + p * kWaves] = lowest[p];
       }
     }
-    // The rest of the previous phase's pending rows, rescanned by all
-    // workgroups.
-    if (!rescanned)
-      rescans(listCount, spilled, a, (long long)g + G);
-    publish(selK, selP, rowAMin, older, firstMin, firstLive ? firstRow : -1);
-    prevA = a;
-    prevSize = na + nb;
+    // Rows rescanned in the first half settle.
+    if (installRow >= 0) {
+      ownPending[installRow - mine0] = 0;
+      ownFn[installRow - mine0] = installFn;
+      ownNext[installRow - mine0] = installNext;
+    }
+    for (int i = kThreads + tid; i < numInstall; i += kThreads) {
+      const int r = pendRow[i];
+      ownPending[r - mine0] = 0;
+      ownFn[r - mine0] = s.scanned[r];
+      ownNext[r - mine0] = s.scanned[n + r];
+    }
+    __syncthreads();
+    // Merge t stands if it is below every new distance of the merges before
+    // it: lane t compares it with the minimum over lanes < t.
+    unsigned int before = lane < m ? newMin[lane] : 0xffffffffu;
+    const unsigned int own = lane < m ? orderedBits(dist[lane]) : 0xffffffffu;
+#pragma unroll
+    for (int d = 1; d < kMaxBatch; d <<= 1) {
+      const unsigned int v = __shfl_up(before, d, 64);
+      if (lane >= d)
+        before = min(before, v);
+    }
+    const unsigned int least = (unsigned int)__builtin_amdgcn_readlane((int)before, kMaxBatch - 1);
+    before = __shfl_up(before, 1, 64);
+    const unsigned long long cut = __ballot(lane >= m || (lane > 0 && !(own < before)));
+    const int valid = __ffsll((long long)cut) - 1; // m <= 16: lane 63 is cut
+    const bool whole = valid == m;
+    int slotsA[kMaxBatch], slotsB[kMaxBatch]; // uniform
+    {
+      const int laneA = lane < m ? slotA[lane] : 0, laneB = lane < m ? slotB[lane] : 0;
+#pragma unroll
+      for (int t = 0; t < kMaxBatch; ++t) {
+        slotsA[t] = __builtin_amdgcn_readlane(laneA, t);
+        slotsB[t] = __builtin_amdgcn_readlane(laneB, t);
+      }
+    }
+    for (int t = wave; t < valid; t += kWaves) {
+      const int a = slotA[t], b = slotB[t];
+      for (int r = lane; r < rows; r += 64) {
+        const int k = mine0 + r, slot = ownSlot[r];
+        if (k == a || k == b || !isActive(activeBits, k))
+          continue;
+        // Entries of slots that retire in the prefix are dead; entries
+        // between two merged slots are written for the later merge.
+        if (slot >= kMaxBatch ? slot - kMaxBatch < valid : slot > t && slot < valid)
+          continue;
+        s.D[entry(a, k)] = newDist[t * per + r];
+      }
+    }
+    for (int r = tid; r < rows; r += kThreads) {
+      const int k = mine0 + r, slot = ownSlot[r];
+      if (!isActive(activeBits, k))
+        continue;
+      if (slot >= kMaxBatch && slot - kMaxBatch < valid) {
+        ownFn[r] = kEmptyKey; // retired
+        ownPending[r] = 0;
+        continue;
+      }
+      unsigned long long f = ownFn[r], other = ownNext[r];
+      bool rescan = false;
+      if (slot >= 0 && slot < kMaxBatch && slot < valid) {
+        const int size = sizeA[slot] + sizeB[slot];
+        ownSize[r] = size;
+        s.size[k] = size;
+        // A cut batch: the parts leave out slots that stay, so the row is
+        // scanned again; no new distance of the batch is below the bound.
+        f = rowFn[slot];
+        other = rowNext[slot];
+        if (!whole) {
+          rescan = true;
+          other = (unsigned long long)least << 32;
+        }
+      } else {
+        // The merges that change this row's two lowest: those that take its
+        // nearest, and those whose new distance is below its bound (only the
+        // columns a > k and b > k are this row's).
+        float nd[kMaxBatch];
+#pragma unroll
+        for (int t = 0; t < kMaxBatch; ++t)
+          nd[t] = t < valid ? newDist[t * per + r] : 0.0f;
+        const int fk = f == kEmptyKey ? -1 : keyIndex(f);
+        const unsigned int otherBits = (unsigned)(other >> 32);
+        unsigned int changes = 0;
+#pragma unroll
+        for (int t = 0; t < kMaxBatch; ++t) {
+          const bool change = slotsA[t] == fk || slotsB[t] == fk ||
+                              (k < slotsA[t] && orderedBits(nd[t]) <= otherBits);
+          changes |= change && t < valid ? 1u << t : 0u;
+        }
+        for (; changes; changes &= changes - 1) {
+          const int t = __ffs(changes) - 1, a = slotA[t], b = slotB[t];
+          const unsigned long long c =
+              k < a ? denseKey(newDist[t * per + r], (unsigned)a) : kEmptyKey;
+          const int at = f == kEmptyKey ? -1 : keyIndex(f);
+          if (rescan) {
+            other = minKey(other, c);
+          } else if (at == a || at == b) {
+            // Its nearest is gone: the new distance replaces it if it is
+            // below all others; with no others, none is left.
+            if (c < other || other == kEmptyKey)
+              f = c;
+            else
+              rescan = true;
+          } else {
+            offer(f, other, c);
+          }
+        }
+      }
+      if (rescan) {
+        const int at = atomicAdd(&pendCount, 1);
+        pendRow[at] = k;
+        ownPending[r] = 1;
+        s.scanned[k] = kEmptyKey;
+        s.scanned[n + k] = kEmptyKey;
+      }
+      ownFn[r] = f;
+      ownNext[r] = other;
+    }
+    waveTop();
+    __syncthreads();
+    writeRecord();
+    if (tid >= 64 && tid < 64 + m) {
+      const int t = tid - 64, a = slotA[t], b = slotB[t];
+      if (t < valid)
+        atomicAnd(&activeBits[b >> 5], ~(1u << (b & 31)));
+      if (a >= mine0 && a < mine1)
+        ownSlot[a - mine0] = -1;
+      if (b >= mine0 && b < mine1)
+        ownSlot[b - mine0] = -1;
+      if (g == 0 && t < valid) {
+        double *row = s.tree + (size_t)(done + t) * 4;
+        row[0] = (double)min(idA[t], idB[t]);
+        row[1] = (double)max(idA[t], idB[t]);
+        row[2] = (double)dist[t];
+        row[3] = (double)(sizeA[t] + sizeB[t]);
+        s.id[a] = s.firstNewId + done + t;
+      }
+    }
+    if (pendCount > kInlineRows)
+      for (int i = tid; i < pendCount; i += kThreads)
+        s.pendingRows[(size_t)g * per + i] = pendRow[i];
+    done += valid;
     lap(3);
     if (!gridBarrier(s.bar, generation, &barrierOk))
       return;
@@ -773,7 +953,8 @@ __global__ void denseSetupKernel(DenseState s, const int *initialSize, const int
   for (int i = blockIdx.x * blockDim.x + threadIdx.x; i < s.n; i += gridDim.x * blockDim.x) {
     s.size[i] = initialSize ? initialSize[i] : 1;
     s.id[i] = initialId ? initialId[i] : i;
-    s.fnKey[i] = kEmptyKey;
+    s.scanned[i] = kEmptyKey;
+    s.scanned[s.n + i] = kEmptyKey;
   }
 }
 
@@ -799,12 +980,15 @@ int denseLinkageOnCondensed(float *D, int n, int linkage, const int *initialSize
                             const int *initialId, int firstNewId, double *hostTree) {
   if (n < 2)
     return 0;
-  const int G = numCUs();
+  // Fewer workgroups for small n: every barrier, record and part costs per
+  // workgroup, and a wave updates 64 rows at a time.
+  const int G = std::min(numCUs(), std::max(kMinGroups, (n + 63) / 64));
   if ((n + G - 1) / G > kMaxOwned || G > kThreads)
     return kErrInvalidShape; // beyond any condensed matrix that fits in HBM
   DenseState st{};
   DevArray<int> size, id;
-  DevArray<unsigned long long> fnKey, records, fnRescan;
+  DevArray<unsigned long long> scanned, records, partFn, partNext;
+  DevArray<unsigned int> partMin;
   DevArray<int> pendingRows;
   DevArray<int2> initItems;
   DevArray<double> tree;
@@ -815,25 +999,36 @@ int denseLinkageOnCondensed(float *D, int n, int linkage, const int *initialSize
   const long long initCount = (long long)(n - 1) * maxChunks;
   const int groups = (G + kGroup - 1) / kGroup;
   const size_t numBarrierWords = (size_t)kLineWords * (3 + groups);
-  // The merge kernel keeps one bit per slot in LDS beside its static arrays.
+  // The merge kernel keeps one bit per slot and the batch's new distances of
+  // its rows in LDS beside its static arrays.
   const size_t activeBytes = (size_t)(n + 31) / 32 * sizeof(unsigned int);
+  const int per = (n + G - 1) / G;
   int device = 0, maxLds = 0;
   s((int)hipGetDevice(&device));
   s((int)hipDeviceGetAttribute(&maxLds, hipDeviceAttributeMaxSharedMemoryPerBlock, device));
   if (!s.ok())
     return s.code;
+  const void *kernel = linkage == kSingle     ? (const void *)denseMergeKernel<kSingle>
+                       : linkage == kComplete ? (const void *)denseMergeKernel<kComplete>
+                       : linkage == kAverage  ? (const void *)denseMergeKernel<kAverage>
+                                              : (const void *)denseMergeKernel<kWard>;
   hipFuncAttributes attr{};
-  s((int)hipFuncGetAttributes(&attr, (const void *)denseMergeKernel));
+  s((int)hipFuncGetAttributes(&attr, kernel));
   if (!s.ok())
     return s.code;
-  if (activeBytes + attr.sharedSizeBytes > (size_t)maxLds)
+  if (activeBytes + per * sizeof(float) + attr.sharedSizeBytes > (size_t)maxLds)
     return kErrInvalidShape; // beyond any condensed matrix that fits in HBM
+  const int batch = (int)std::min<size_t>(
+      kMaxBatch, (maxLds - attr.sharedSizeBytes - activeBytes) / (per * sizeof(float)));
+  const size_t dynamicBytes = activeBytes + (size_t)batch * per * sizeof(float);
   s(size.alloc(n));
   s(id.alloc(n));
-  s(fnKey.alloc(n));
-  s(records.alloc((size_t)2 * G * kRecordWords));
-  s(fnRescan.alloc(n));
-  s(pendingRows.alloc((size_t)2 * G * kMaxOwned));
+  s(scanned.alloc((size_t)2 * n));
+  s(records.alloc((size_t)G * kRecordWords));
+  s(partFn.alloc((size_t)kMaxBatch * G));
+  s(partNext.alloc((size_t)kMaxBatch * G));
+  s(partMin.alloc((size_t)kMaxBatch * G));
+  s(pendingRows.alloc((size_t)G * per));
   s(initItems.alloc(initCount));
   s(tree.alloc((size_t)(n - 1) * 4));
   s(barrierWords.alloc(numBarrierWords));
@@ -841,13 +1036,16 @@ int denseLinkageOnCondensed(float *D, int n, int linkage, const int *initialSize
     return s.code;
   st.D = D;
   st.n = n;
-  st.linkage = linkage;
   st.firstNewId = firstNewId;
+  st.per = per;
+  st.batch = batch;
+  st.partFn = partFn;
+  st.partNext = partNext;
+  st.partMin = partMin;
   st.size = size;
   st.id = id;
-  st.fnKey = fnKey;
+  st.scanned = scanned;
   st.records = records;
-  st.fnRescan = fnRescan;
   st.pendingRows = pendingRows;
   st.items = initItems;
   st.tree = tree;
@@ -871,8 +1069,8 @@ int denseLinkageOnCondensed(float *D, int n, int linkage, const int *initialSize
   s((int)hipGetLastError());
   if (s.ok()) {
     void *args[] = {&st};
-    s((int)hipLaunchCooperativeKernel((const void *)denseMergeKernel, dim3(G), dim3(kThreads),
-                                      args, (unsigned int)activeBytes, stream()));
+    s((int)hipLaunchCooperativeKernel(kernel, dim3(G), dim3(kThreads),
+                                      args, (unsigned int)dynamicBytes, stream()));
   }
   s(sync());
   unsigned int aborted = 0;

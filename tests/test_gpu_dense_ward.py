@@ -75,6 +75,27 @@ def test_dense_star_many_rescans(method):
     np.testing.assert_array_equal(Z, oracle.dense_linkage(X, method))
 
 
+@pytest.mark.parametrize("method", ["single", "complete", "average", "ward"])
+@pytest.mark.parametrize("n", [63, 65, 511, 513, 1025])
+@pytest.mark.parametrize("data", ["lattice", "gaps", "pairs"])
+def test_dense_batches_of_merges(method, n, data):
+    # Several merges per batch, at the edges of the workgroups' row ranges (64
+    # rows): many equal distances (an integer lattice), merges that each take in
+    # the cluster just made (growing gaps: a batch keeps its first merge only),
+    # and independent ones (far pairs of close points: batches are full).
+    if data == "lattice":
+        X = np.random.default_rng(n).integers(0, 6, (n, 3))
+    elif data == "gaps":
+        X = np.stack([np.cumsum(np.arange(n)), np.zeros(n)], axis=1)
+    else:
+        rng = np.random.default_rng(n)
+        X = np.repeat(rng.normal(0, 100, (n // 2 + 1, 4)), 2, axis=0)[:n]
+        X = X + rng.normal(0, 0.1, X.shape)
+    X = X.astype(np.float32)
+    Z = cuhc.linkage(X, method=method, algorithm="dense")
+    np.testing.assert_array_equal(Z, oracle.dense_linkage(X, method))
+
+
 @pytest.mark.parametrize("n", [2, 3, 127, 128, 129, 600])
 @pytest.mark.parametrize("d", [1, 7, 64])
 def test_rnn_matches_scipy(n, d):
