@@ -4,7 +4,10 @@
 //
 // Layout: D(i, j), i < j, at i*n - i*(i+1)/2 + (j - i - 1): scipy's pdist order,
 // n (n - 1) / 2 floats (20 GB at n = 100k). Slot s holds one active cluster;
-// merging slots a < b puts the merged cluster in a and retires b.
+// merging slots a < b puts the merged cluster in a and retires b. (A square
+// matrix, whose merged rows are read in order, takes twice the memory and
+// gives nothing: the update's reads fell from 312 to 97 ms at n = 100k, and
+// writing the merged slots' columns rose from 29 to 190 ms.)
 //
 // Forward nearest cache: fn(i) = argmin over active j > i of (D(i, j), j). The
 // closest pair (lowest distance, then lowest i, then lowest j) is
@@ -341,7 +344,7 @@ __global__ void __launch_bounds__(kThreads) denseMergeKernel(DenseState s) {
   __shared__ unsigned long long rowFn[kMaxBatch], rowNext[kMaxBatch];
   __shared__ unsigned int newMin[kMaxBatch];
   __shared__ int batchCount; // merges in the batch, or -1: no pair is left
-  __shared__ unsigned long long waveKey[2 * kWaves];
+  __shared__ unsigned long long waveKey[3 * kWaves];
   __shared__ int waveInt[2 * kWaves];
   __shared__ __align__(16) unsigned long long topKey[kWaves * kTop];
   __shared__ int barrierOk;
@@ -372,13 +375,16 @@ __global__ void __launch_bounds__(kThreads) denseMergeKernel(DenseState s) {
   // This workgroup's kTop lowest settled rows, wave by wave (thread t looks
   // at rows t, t + kThreads, ...; keys are distinct, so the next lowest is the
   // lowest above the last).
-  auto waveTop = [&]() {
+  // Only the first `count` are looked for.
+  auto waveTop = [&](int count) {
     auto keyOf = [&](int r) {
       return r < rows && !ownPending[r] ? selectionKey(ownFn[r], mine0 + r) : kEmptyKey;
     };
     const unsigned long long first = keyOf(tid); // most workgroups own at most kThreads rows
+    if (lane >= count && lane < kTop)
+      topKey[wave * kTop + lane] = kEmptyKey;
     unsigned long long last = 0;
-    for (int q = 0; q < kTop; ++q) {
+    for (int q = 0; q < count; ++q) {
       unsigned long long best = q == 0 || first > last ? first : kEmptyKey;
       for (int r = tid + kThreads; r < rows; r += kThreads) {
         const unsigned long long key = keyOf(r);
@@ -463,7 +469,7 @@ __global__ void __launch_bounds__(kThreads) denseMergeKernel(DenseState s) {
   }
   if (tid == 0)
     pendCount = 0;
-  waveTop();
+  waveTop(kTop);
   __syncthreads();
   writeRecord();
   if (!gridBarrier(s.bar, generation, &barrierOk))
@@ -471,6 +477,11 @@ __global__ void __launch_bounds__(kThreads) denseMergeKernel(DenseState s) {
   if (clocked)
     t0 = wall_clock64();
 
+  // The batch's limit. Where each merge takes in the cluster just made (a
+  // chain), a batch is cut to its first merge and its row is scanned again: a
+  // batch of one costs less. So such a cut limits the next batches to one,
+  // twice as many of them as the cut before.
+  int limit = s.batch, hold = 0, holdNext = 1;
   for (int done = 0; done < n - 1;) {
     // ---- First half: select the batch.
     unsigned long long sel[kTop], bound = kEmptyKey;
@@ -524,9 +535,11 @@ __global__ void __launch_bounds__(kThreads) denseMergeKernel(DenseState s) {
         incl += v;
     }
     const bool spill = __ballot(cnt > kInlineRows) != 0;
+    unsigned long long lowestHead = limit == 1 ? waveMinKey(sel[0]) : kEmptyKey;
     if (lane == 0) {
       waveKey[wave] = bound;
       waveKey[kWaves + wave] = guard;
+      waveKey[2 * kWaves + wave] = lowestHead;
       waveInt[kWaves + wave] = spill;
     }
     if (lane == 63)
@@ -538,6 +551,7 @@ __global__ void __launch_bounds__(kThreads) denseMergeKernel(DenseState s) {
     for (int w = 0; w < kWaves; ++w) {
       bound = minKey(bound, waveKey[w]);
       guard = minKey(guard, waveKey[kWaves + w]);
+      lowestHead = minKey(lowestHead, waveKey[2 * kWaves + w]);
       start += w < wave ? waveInt[w] : 0;
       listCount += waveInt[w];
       spilled |= waveInt[kWaves + w] != 0;
@@ -552,7 +566,7 @@ __global__ void __launch_bounds__(kThreads) denseMergeKernel(DenseState s) {
       listStart[G] = listCount;
     // The kMaxBatch lowest heads' workgroups hold the kMaxBatch lowest keys:
     // each head's rank, by kThreads / G threads per head.
-    if (tid < rankers * G) {
+    if (limit > 1 && tid < rankers * G) {
       const int i = tid % G, lo = tid / G * rankSpan, hi = min(G, lo + rankSpan);
       const unsigned long long key = heads[i];
       int below = 0;
@@ -562,8 +576,22 @@ __global__ void __launch_bounds__(kThreads) denseMergeKernel(DenseState s) {
       if (below)
         atomicAdd(&headRank[i], below);
     }
+    auto take = [&](int at, int i, int j, unsigned long long key) {
+      slotA[at] = i;
+      slotB[at] = j;
+      dist[at] = fromOrderedBits((unsigned)(key >> 32));
+      if (i >= mine0 && i < mine1)
+        ownSlot[i - mine0] = (signed char)at;
+      if (j >= mine0 && j < mine1)
+        ownSlot[j - mine0] = (signed char)(kMaxBatch + at);
+    };
     __syncthreads();
-    if (tid < G && sel[0] != kEmptyKey) {
+    if (limit == 1) {
+      if (sel[0] == lowestHead && lowestHead < bound)
+        take(0, keyIndex(sel[0]), (int)col[0], sel[0]);
+      if (tid == 0)
+        batchCount = lowestHead < bound ? 1 : bound == kEmptyKey ? -1 : 0;
+    } else if (tid < G && sel[0] != kEmptyKey) {
       const int r = headRank[tid];
       if (r < kMaxBatch) {
 #pragma unroll
@@ -573,8 +601,9 @@ __global__ void __launch_bounds__(kThreads) denseMergeKernel(DenseState s) {
         }
       }
     }
-    __syncthreads();
-    if (wave == 0) {
+    if (limit > 1)
+      __syncthreads();
+    if (wave == 0 && limit > 1) {
       const unsigned long long key = cand[lane];
       // Nor any key above the last of the chosen heads: a workgroup that is
       // not among them may have a lower one.
@@ -610,18 +639,11 @@ __global__ void __launch_bounds__(kThreads) denseMergeKernel(DenseState s) {
       const unsigned long long inMask = ((stop & -stop) - 1) & ~retired;
       const bool in = inMask >> lane & 1;
       const int at = __popcll(inMask & ((1ull << lane) - 1));
-      if (in && at < s.batch) {
-        slotA[at] = i;
-        slotB[at] = j;
-        dist[at] = fromOrderedBits((unsigned)(k >> 32));
-        if (i >= mine0 && i < mine1)
-          ownSlot[i - mine0] = (signed char)at;
-        if (j >= mine0 && j < mine1)
-          ownSlot[j - mine0] = (signed char)(kMaxBatch + at);
-      }
+      if (in && at < limit)
+        take(at, i, j, k);
       if (lane == 0)
-        batchCount = valid == 0 && bound == kEmptyKey ? -1 : min(s.batch, __popcll(inMask));
-    } else {
+        batchCount = valid == 0 && bound == kEmptyKey ? -1 : min(limit, __popcll(inMask));
+    } else if (wave > 0) {
       // The pending rows are scanned again (no distance is written in this
       // half), one column chunk per wave and step.
       const unsigned int numItems = (unsigned)listCount * (unsigned)maxChunks;
@@ -788,6 +810,8 @@ __global__ void __launch_bounds__(kThreads) denseMergeKernel(DenseState s) {
     }
 #pragma unroll
     for (int p = 0; p < kPerWave; ++p) {
+      if (wave + p * kWaves >= m)
+        break;
       waveLowest2(fn[p], next[p]);
       lowest[p] = waveMinBits(lowest[p]);
       if (lane == 0) {
@@ -811,19 +835,34 @@ __global__ void __launch_bounds__(kThreads) denseMergeKernel(DenseState s) {
     __syncthreads();
     // Merge t stands if it is below every new distance of the merges before
     // it: lane t compares it with the minimum over lanes < t.
-    unsigned int before = lane < m ? newMin[lane] : 0xffffffffu;
-    const unsigned int own = lane < m ? orderedBits(dist[lane]) : 0xffffffffu;
+    int valid = m;
+    unsigned int least = newMin[0]; // the smallest new distance of the batch
+    if (m > 1) {
+      unsigned int before = lane < m ? newMin[lane] : 0xffffffffu;
+      const unsigned int own = lane < m ? orderedBits(dist[lane]) : 0xffffffffu;
 #pragma unroll
-    for (int d = 1; d < kMaxBatch; d <<= 1) {
-      const unsigned int v = __shfl_up(before, d, 64);
-      if (lane >= d)
-        before = min(before, v);
+      for (int d = 1; d < kMaxBatch; d <<= 1) {
+        const unsigned int v = __shfl_up(before, d, 64);
+        if (lane >= d)
+          before = min(before, v);
+      }
+      least = (unsigned int)__builtin_amdgcn_readlane((int)before, kMaxBatch - 1);
+      before = __shfl_up(before, 1, 64);
+      const unsigned long long cut = __ballot(lane >= m || (lane > 0 && !(own < before)));
+      valid = __ffsll((long long)cut) - 1; // m <= 16: lane 63 is cut
     }
-    const unsigned int least = (unsigned int)__builtin_amdgcn_readlane((int)before, kMaxBatch - 1);
-    before = __shfl_up(before, 1, 64);
-    const unsigned long long cut = __ballot(lane >= m || (lane > 0 && !(own < before)));
-    const int valid = __ffsll((long long)cut) - 1; // m <= 16: lane 63 is cut
     const bool whole = valid == m;
+    if (!whole && valid == 1) {
+      limit = 1;
+      hold = holdNext;
+      holdNext = min(2 * holdNext, 256);
+    } else if (hold > 0) {
+      --hold;
+    } else {
+      limit = s.batch;
+      if (valid > 1)
+        holdNext = 1;
+    }
     int slotsA[kMaxBatch], slotsB[kMaxBatch]; // uniform
     {
       const int laneA = lane < m ? slotA[lane] : 0, laneB = lane < m ? slotB[lane] : 0;
@@ -915,7 +954,7 @@ __global__ void __launch_bounds__(kThreads) denseMergeKernel(DenseState s) {
       ownFn[r] = f;
       ownNext[r] = other;
     }
-    waveTop();
+    waveTop(limit == 1 ? 1 : kTop);
     __syncthreads();
     writeRecord();
     if (tid >= 64 && tid < 64 + m) {
@@ -980,8 +1019,6 @@ int denseLinkageOnCondensed(float *D, int n, int linkage, const int *initialSize
                             const int *initialId, int firstNewId, double *hostTree) {
   if (n < 2)
     return 0;
-  // Fewer workgroups for small n: every barrier, record and part costs per
-  // workgroup, and a wave updates 64 rows at a time.
   const int G = std::min(numCUs(), std::max(kMinGroups, (n + 63) / 64));
   if ((n + G - 1) / G > kMaxOwned || G > kThreads)
     return kErrInvalidShape; // beyond any condensed matrix that fits in HBM
