@@ -101,3 +101,20 @@ def test_device_points_errors():
             cuhc.linkage(dev)
     finally:
         dev.free()
+
+
+@pytest.mark.parametrize("n, d", [(1, 1), (255, 1), (2049, 7), (513, 255), (300, 256), (5, 257),
+                                  (4097, 300)])
+def test_feature_ranges_shapes(n, d):
+    # Rows and features around the ranges kernel's workgroup (256 threads: whole
+    # rows up to 256 features, one row at a time above); the lowest and highest
+    # values in the last row and feature.
+    X = np.random.default_rng(n + d).normal(size=(n, d)).astype(np.float32)
+    X[-1, -1], X[0, 0] = -50.0, 60.0
+    X[-1, 0] += 70.0
+    low, high = np.empty(d, np.float32), np.empty(d, np.float32)
+    dev = _lib.DeviceArray(X)
+    _lib.check(_lib.lib.cuhc_feature_ranges_device(dev.ptr, n, d, _lib.float_ptr(low),
+                                                   _lib.float_ptr(high)))
+    np.testing.assert_array_equal(low, X.min(axis=0))
+    np.testing.assert_array_equal(high, X.max(axis=0))
