@@ -104,37 +104,92 @@ __global__ void layoutProbeKernel(int *bad) {
 // ---------------------------------------------------------------------------
 // Preparation: mean, scale, FP16 points and per-point bounds.
 
-__global__ void columnSumsKernel(const float *X, int n, int d, double *sums) {
-  // Each workgroup sums a contiguous chunk of rows; thread t owns feature t % d.
-  const int rowsPer = (n + gridDim.x - 1) / gridDim.x;
-  const int r0 = blockIdx.x * rowsPer, r1 = min(n, r0 + rowsPer);
-  const int lanes = (blockDim.x / d) * d;
-  if ((int)threadIdx.x >= lanes)
-    return;
-  const int f = threadIdx.x % d, group = threadIdx.x / d, groups = lanes / d;
-  double acc = 0.0;
-  for (int r = r0 + group; r < r1; r += groups)
-    acc += (double)X[(size_t)r * d + f];
-  atomicAdd(&sums[f], acc);
+// The set-up's kernels are bound by one read of the points at large n and by
+// launches and waiting at small: a workgroup ends with one atomic per result,
+// and only where it would change the word (one per wave, changed or not, from
+// 1,024 workgroups made the two maxima 150 us of a 4.1 ms tree of 20,000
+// points); the mean and the scale stay on the device.
+constexpr int kSetupThreads = 256;
+constexpr int kSetupAhead = 8; // rows loaded before the first is used
+
+// A monotone maximum: a stale read only costs an atomic.
+DEV void raiseMax(unsigned int *word, unsigned int bits) {
+  if (bits > __hip_atomic_load(word, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT))
+    atomicMax(word, bits);
 }
 
-__global__ void maxDevKernel(const float *X, int n, int d, const float *mu, unsigned int *maxBits) {
-  float local = 0.0f;
-  const size_t total = (size_t)n * d;
-  for (size_t e = blockIdx.x * (size_t)blockDim.x + threadIdx.x; e < total;
-       e += (size_t)gridDim.x * blockDim.x)
-    local = fmaxf(local, fabsf((float)((double)X[e] - (double)mu[e % d])));
+// The maximum over the workgroup, in every thread (non-negative floats).
+DEV float blockMaxFloat(float v, float *red) {
 #pragma unroll
   for (int m = 32; m > 0; m >>= 1)
-    local = fmaxf(local, __shfl_xor(local, m, 64));
+    v = fmaxf(v, __shfl_xor(v, m, 64));
+  __syncthreads();
   if ((threadIdx.x & 63) == 0)
-    atomicMax(maxBits, __float_as_uint(local));
+    red[threadIdx.x >> 6] = v;
+  __syncthreads();
+  return fmaxf(fmaxf(red[0], red[1]), fmaxf(red[2], red[3]));
 }
 
-__global__ void toHalfKernel(const float *X, int n, int d, int DP, const float *mu, double scale,
-                             _Float16 *xh, float *norm, float *R, float *rho,
-                             unsigned int *maxR, unsigned int *maxRho) {
+// Calls use(x) for the values of feature threadIdx.x % d (d <= 64) that fall
+// to this thread: whole rows per workgroup, kSetupAhead of them loaded at once.
+template <class Use> DEV void forFeature(const float *X, int n, int d, Use &&use) {
+  const int rows = kSetupThreads / d, f = threadIdx.x % d, r0 = threadIdx.x / d;
+  if (r0 >= rows)
+    return;
+  const long long step = (long long)gridDim.x * rows;
+  for (long long r = (long long)blockIdx.x * rows + r0; r < n; r += step * kSetupAhead) {
+    float v[kSetupAhead];
+#pragma unroll
+    for (int u = 0; u < kSetupAhead; ++u)
+      v[u] = r + u * step < n ? X[(size_t)(r + u * step) * d + f] : 0.0f;
+#pragma unroll
+    for (int u = 0; u < kSetupAhead; ++u)
+      if (r + u * step < n)
+        use(v[u]);
+  }
+}
+
+__global__ void __launch_bounds__(kSetupThreads)
+    columnSumsKernel(const float *X, int n, int d, double *sums) {
+  __shared__ double part[kSetupThreads];
+  double acc = 0.0;
+  forFeature(X, n, d, [&](float x) { acc += (double)x; });
+  part[threadIdx.x] = acc;
+  __syncthreads();
+  if ((int)threadIdx.x < d) {
+    for (int t = threadIdx.x + d; t < kSetupThreads / d * d; t += d)
+      acc += part[t];
+    atomicAdd(&sums[threadIdx.x], acc);
+  }
+}
+
+__global__ void meanKernel(const double *sums, int n, int d, float *mu) {
+  if ((int)threadIdx.x < d)
+    mu[threadIdx.x] = (float)(sums[threadIdx.x] / n);
+}
+
+__global__ void __launch_bounds__(kSetupThreads)
+    maxDevKernel(const float *X, int n, int d, const float *mu, unsigned int *maxBits) {
+  __shared__ float red[4];
+  const double m = (double)mu[threadIdx.x % d];
+  float local = 0.0f;
+  forFeature(X, n, d, [&](float x) { local = fmaxf(local, fabsf((float)((double)x - m))); });
+  local = blockMaxFloat(local, red);
+  if (threadIdx.x == 0)
+    raiseMax(maxBits, __float_as_uint(local));
+}
+
+// maxBits: the largest deviation from the mean, and (out) the largest R and rho.
+__global__ void __launch_bounds__(kSetupThreads)
+    toHalfKernel(const float *X, int n, int d, int DP, const float *mu, _Float16 *xh, float *norm,
+                 float *R, float *rho, unsigned int *maxBits) {
+  __shared__ float red[4];
   float lr = 0.0f, lrho = 0.0f;
+  // Power-of-two scale: max |x'| in (2^13, 2^14].
+  const float maxDev = __uint_as_float(maxBits[0]);
+  int exponent = 0;
+  (void)frexpf(maxDev > 0.0f && maxDev < INFINITY ? maxDev : 1.0f, &exponent);
+  const double scale = ldexp(1.0, 14 - exponent);
   // A thread converts one point, eight features at a time: the row is read in
   // 16-byte loads when X is 16-byte aligned and d is a multiple of 4 (every
   // row then is), and each eight halves leave in one 16-byte store.
@@ -179,14 +234,11 @@ __global__ void toHalfKernel(const float *X, int n, int d, int DP, const float *
     lr = fmaxf(lr, r);
     lrho = fmaxf(lrho, e);
   }
-#pragma unroll
-  for (int m = 32; m > 0; m >>= 1) {
-    lr = fmaxf(lr, __shfl_xor(lr, m, 64));
-    lrho = fmaxf(lrho, __shfl_xor(lrho, m, 64));
-  }
-  if ((threadIdx.x & 63) == 0) {
-    atomicMax(maxR, __float_as_uint(lr));
-    atomicMax(maxRho, __float_as_uint(lrho));
+  lr = blockMaxFloat(lr, red);
+  lrho = blockMaxFloat(lrho, red);
+  if (threadIdx.x == 0) {
+    raiseMax(&maxBits[1], __float_as_uint(lr));
+    raiseMax(&maxBits[2], __float_as_uint(lrho));
   }
 }
 
@@ -1217,26 +1269,20 @@ MixedPass *mixedPassCreate(const float *X, int n, int d, int *status) {
     s(fill(maxes, 0, 3 * sizeof(unsigned int)));
     s(fill(mp->stats, 0, 5 * sizeof(unsigned long long)));
     s(fill(mp->recheckStats, 0, mp->recheckStats.bytes()));
-    hipLaunchKernelGGL(columnSumsKernel, dim3(std::max(1, std::min(1024, n / 64 + 1))),
-                       dim3(256), 0, stream(), X, n, d, sums.get());
-    std::vector<double> hs(d);
-    s(download(hs.data(), sums, d * sizeof(double)));
-    std::vector<float> hmu(d);
-    for (int k = 0; k < d; ++k)
-      hmu[k] = (float)(hs[k] / n);
-    s(upload(mp->mu, hmu.data(), d * sizeof(float)));
-    hipLaunchKernelGGL(maxDevKernel, dim3(1024), dim3(256), 0, stream(), X, n, d, mp->mu.get(),
-                       maxes.get());
-    unsigned int mb = 0;
-    s(download(&mb, maxes, sizeof(mb)));
-    const float maxDev = floatOf(mb);
-    // Power-of-two scale: max |x'| in (2^13, 2^14].
-    int e = 0;
-    (void)std::frexp(maxDev > 0.0f && std::isfinite(maxDev) ? maxDev : 1.0f, &e);
-    const double scale = std::ldexp(1.0, 14 - e);
-    hipLaunchKernelGGL(toHalfKernel, dim3(1024), dim3(256), 0, stream(), X, n, d, mp->DP,
-                       mp->mu.get(), scale, mp->xh.get(), mp->norm.get(), mp->R.get(),
-                       mp->rho.get(), maxes.get() + 1, maxes.get() + 2);
+    // At most four workgroups per CU, each with rows for kSetupAhead loads.
+    const int rows = kSetupThreads / d;
+    const int blocks = (int)std::min<long long>(
+        4LL * numCUs(), ((long long)n + rows * kSetupAhead - 1) / (rows * kSetupAhead));
+    hipLaunchKernelGGL(columnSumsKernel, dim3(blocks), dim3(kSetupThreads), 0, stream(), X, n, d,
+                       sums.get());
+    hipLaunchKernelGGL(meanKernel, dim3(1), dim3(64), 0, stream(), sums.get(), n, d,
+                       mp->mu.get());
+    hipLaunchKernelGGL(maxDevKernel, dim3(blocks), dim3(kSetupThreads), 0, stream(), X, n, d,
+                       mp->mu.get(), maxes.get());
+    hipLaunchKernelGGL(toHalfKernel, dim3(std::min(1024, (n + 255) / 256)), dim3(kSetupThreads),
+                       0, stream(), X, n, d, mp->DP, mp->mu.get(), mp->xh.get(),
+                       mp->norm.get(), mp->R.get(), mp->rho.get(), maxes.get());
+    s((int)hipGetLastError());
     unsigned int rr[2] = {0, 0};
     s(download(rr, maxes.get() + 1, sizeof(rr)));
     mp->Rmax = floatOf(rr[0]);
