@@ -12,6 +12,7 @@
 #include "mst.hpp"
 
 #include <algorithm>
+#include <cmath>
 #include <numeric>
 
 namespace cuhc {
@@ -131,6 +132,24 @@ int boruvkaMst(const float *X, int n, int d, MetricSpec m, WeightSpec w, const M
   int numComponents = n;
   bool pruneThisPass = opt.prune;
   bool haveResult = false; // dNearest holds the last round's exact result
+  if (s.ok() && ct.small && !mixed && !opt.prune) {
+    // Few points: rounds cost launches and host reads, so as many as such
+    // inputs take (components fall to a quarter or less per round) are queued
+    // before the first read; rounds past the last find one component and end.
+    s(fill(dNearest, 0xff, n * sizeof(unsigned long long)));
+    int rounds = std::max(1, (int)std::ceil(std::log2((double)n) / 2));
+    while (s.ok() && numComponents > 1) {
+      for (int q = 0; q < rounds && s.ok(); ++q) {
+        s(nearestOtherSymmetric(X, n, d, m, w, dComp, opt.devOrig, dNearest, ct.state + 1));
+        PhaseTimer timer(kPhaseContract);
+        s(contractSmallQueue(ct, dNearest, dComp, opt.devOrig, posOf, true));
+      }
+      int added = 0;
+      if (s.ok())
+        s(contractState(ct, &numComponents, &added));
+      rounds = 1;
+    }
+  }
   while (s.ok() && numComponents > 1) {
     if (mixed) {
       s(mixedPassRun(mixed, dComp, numComponents, m.id == kSqEuclidean, !haveResult, dNearest));

@@ -205,7 +205,10 @@ __global__ void __launch_bounds__(256, 3) // three waves per SIMD (at most 168 V
     nearestOtherSymmetricKernel(const float *__restrict__ X, int n, int d, Metric metric,
                                 Weight weight, const int *__restrict__ comp,
                                 const int *__restrict__ orig,
-                                unsigned long long *__restrict__ nearest, long long numPairs) {
+                                unsigned long long *__restrict__ nearest, long long numPairs,
+                                const int *__restrict__ numComp) {
+  if (numComp && *numComp <= 1)
+    return; // queued ahead of the host: one component is left
   constexpr int TR = T::TR;
   // With an accumulator bound, a pair is finished (sqrt, weight, keys) only
   // when its raw accumulator is within the limit of its row point or of its
@@ -910,7 +913,8 @@ int condensedMatrix(const float *X, int n, int d, MetricSpec m, float *out) {
 }
 
 int nearestOtherSymmetric(const float *X, int n, int d, MetricSpec m, WeightSpec w,
-                          const int *comp, const int *orig, unsigned long long *nearest) {
+                          const int *comp, const int *orig, unsigned long long *nearest,
+                          const int *numComp) {
   if (w.kind == kWeightWard) {
     if (m.id != kSqEuclidean)
       return kErrInvalidMetric;
@@ -920,7 +924,7 @@ int nearestOtherSymmetric(const float *X, int n, int d, MetricSpec m, WeightSpec
       const long long tiles = (n + T::DIM - 1) / T::DIM, pairs = tiles * (tiles + 1) / 2;
       hipLaunchKernelGGL((nearestOtherSymmetricKernel<T, SqEuclidean, WardWeight>),
                          dim3(persistentBlocks(pairs, 8)), dim3(256), 0, stream(), X, n, d,
-                         SqEuclidean{}, ward, comp, orig, nearest, pairs);
+                         SqEuclidean{}, ward, comp, orig, nearest, pairs, numComp);
       return (int)hipGetLastError();
     });
   }
@@ -935,7 +939,7 @@ int nearestOtherSymmetric(const float *X, int n, int d, MetricSpec m, WeightSpec
         addUnits(kPhaseDistanceTiles, (long long)n * (n + 1) / 2);
         hipLaunchKernelGGL((nearestOtherSymmetricKernel<T, Metric, Weight>),
                            dim3(persistentBlocks(pairs, 8)), dim3(256), 0, stream(), X, n, d,
-                           metric, weight, comp, orig, nearest, pairs);
+                           metric, weight, comp, orig, nearest, pairs, numComp);
         return (int)hipGetLastError();
       });
     });

@@ -27,11 +27,12 @@ struct DevicePoints {
   std::vector<float> hostCopy;
 };
 
-// Edges of a spanning forest in device memory (original indices, u < v).
-struct DeviceEdges {
-  DevArray<int> u, v;
-  DevArray<float> w;
-  int count = 0;
+// Edges of a spanning forest in device memory (original indices, u < v): u, v
+// and w are consecutive arrays of capacity entries.
+struct EdgeArrays {
+  int *u = nullptr, *v = nullptr;
+  float *w = nullptr;
+  int capacity = 0, count = 0;
 };
 
 // Device state of Boruvka's contraction (contract.hip).
@@ -39,10 +40,14 @@ struct Contraction {
   int n = 0;
   DevArray<unsigned long long> best1;
   DevArray<unsigned int> best2;
-  DevArray<int> parent, root, flags, newId, changed, counters;
+  DevArray<int> parent, root, flags, newId;
   DevArray<unsigned char> scanTemp;
-  size_t scanBytes = 0;
-  DeviceEdges edges;
+  // Edges in the forest, components, an error flag (a cycle), a flag for a
+  // round that found no edge.
+  DevArray<int> state;
+  DevArray<int> storage; // the edges
+  EdgeArrays edges;
+  bool small = false; // contractSmallQueue applies
   int alloc(int points);
 };
 
@@ -54,11 +59,19 @@ int resetComponents(int *comp, int n);
 // ct.edges, comp relabelled to 0..newNumComp-1. orig maps positions to
 // original indices and posOf back (both null: identity). *added = edges
 // appended this round.
-int contractRound(Contraction &ct, const unsigned long long *nearest, int *comp, const int *orig,
+int contractRound(Contraction &ct, unsigned long long *nearest, int *comp, const int *orig,
                   const int *posOf, int numComp, int *newNumComp, int *added);
 
+// For ct.small: a contraction queued without waiting for its result (nothing
+// happens once one component is left; empty: nearest[] is emptied for the next
+// pass), and the host's read of the result of
+// all contractions queued: kErrDisconnected if one of them found no edge.
+int contractSmallQueue(Contraction &ct, unsigned long long *nearest, int *comp, const int *orig,
+                       const int *posOf, bool empty);
+int contractState(Contraction &ct, int *numComp, int *added);
+
 // Sorts device edges into the global order and writes the scipy-format tree.
-int treeFromDeviceEdges(const DeviceEdges &edges, int n, double *tree);
+int treeFromDeviceEdges(const EdgeArrays &edges, int n, double *tree);
 
 // The learned method's candidate lists, kept for the Boruvka rounds of
 // mutual reachability. List row r (the points' order at the gather) holds

@@ -38,9 +38,11 @@ int condensedMatrix(const float *X, int n, int d, MetricSpec m, float *out);
 // nearest[i] = min over j with comp[j] != comp[i] of packKey(weight(i, j), id(j)),
 // combined by atomicMin, so nearest[] must start at kEmptyKey. Each unordered
 // pair is computed once (tiles I <= J). id(j) = orig[j] (device) for points in
-// spatial order, else j (orig == nullptr).
+// spatial order, else j (orig == nullptr). numComp (device, nullable): nothing
+// is computed when it holds 1 (passes queued ahead of the host).
 int nearestOtherSymmetric(const float *X, int n, int d, MetricSpec m, WeightSpec w,
-                          const int *comp, const int *orig, unsigned long long *nearest);
+                          const int *comp, const int *orig, unsigned long long *nearest,
+                          const int *numComp = nullptr);
 
 // ---------------------------------------------------------------------------
 // Spatial pruning (reference src/spatial.cuh)

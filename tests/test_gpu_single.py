@@ -24,6 +24,20 @@ def run(X, metric="euclidean", precision="fp32", pruning="never", p=2.0):
         _lib.set_pruning("auto")
 
 
+@pytest.mark.parametrize("data", ["lattice", "gaps"])
+@pytest.mark.parametrize("n", [2, 1024, 1025, 4096, 4098, 7168, 7169, 9000])
+def test_contraction_forms(data, n):
+    # Around the largest input that one workgroup contracts (7,168 points, 1,024
+    # threads) and the fewest edges sorted on the device (4,096): many tied
+    # edges, and growing gaps, where every point hooks onto the one before it (a
+    # chain of n hooks in the first round).
+    if data == "lattice":
+        X = np.random.default_rng(n).integers(0, 30, (n, 3)).astype(np.float32)
+    else:
+        X = np.cumsum(np.arange(n)).astype(np.float32)[:, None]
+    np.testing.assert_array_equal(run(X, "manhattan"), oracle.single_linkage(X, "manhattan"))
+
+
 @pytest.mark.parametrize("metric", ["euclidean", "sqeuclidean", "manhattan", "chebyshev",
                                     "cosine"])
 @pytest.mark.parametrize("n", [2, 3, 127, 128, 129, 300])
