@@ -13,13 +13,23 @@
 
 #include <algorithm>
 #include <cmath>
-#include <numeric>
 
 namespace cuhc {
 
+int DevicePoints::arrange(const float *X, int n, int d) {
+  Status s;
+  s(orig.alloc(n));
+  if (s.ok())
+    s(spatialOrder(X, d, nullptr, n, orig));
+  if (s.ok())
+    s(gatherRows(X, orig, n, d, points));
+  inOrder = s.ok();
+  return s.code;
+}
+
 // Both entry paths check the coordinates first (kErrNonFinite for NaN or
 // infinity): the FP16 candidate kernels are compiled without NaN semantics and
-// the host k-d order needs ordered comparisons.
+// the k-d order needs ordered comparisons.
 int DevicePoints::upload(const float *hostPoints, int n, int d, bool spatial) {
   const size_t count = (size_t)n * d;
   Status s;
@@ -33,17 +43,10 @@ int DevicePoints::upload(const float *hostPoints, int n, int d, bool spatial) {
   }
   DevArray<float> raw;
   s(raw.alloc(count));
-  s(orig.alloc(n));
   s(cuhc::upload(raw, hostPoints, count * sizeof(float)));
   s(checkFinite(raw, count));
-  if (!s.ok())
-    return s.code;
-  order = spatialOrder(hostPoints, n, d);
-  host = hostPoints;
-  s(cuhc::upload(orig, order.data(), n * sizeof(int)));
   if (s.ok())
-    s(gatherRows(raw, orig, n, d, points));
-  s(sync());
+    s(arrange(raw, n, d));
   return s.code;
 }
 
@@ -60,18 +63,9 @@ int DevicePoints::adopt(const float *devicePoints, int n, int d, bool spatial) {
     external = devicePoints;
     return 0;
   }
-  hostCopy.resize(count);
-  s(download(hostCopy.data(), devicePoints, count * sizeof(float)));
-  if (!s.ok())
-    return s.code;
-  host = hostCopy.data();
-  order = spatialOrder(host, n, d);
   s(points.alloc(count));
-  s(orig.alloc(n));
-  s(cuhc::upload(orig, order.data(), n * sizeof(int)));
   if (s.ok())
-    s(gatherRows(devicePoints, orig, n, d, points));
-  s(sync());
+    s(arrange(devicePoints, n, d));
   return s.code;
 }
 
@@ -222,41 +216,6 @@ int singleLinkageMst(const DevicePoints &pts, int n, int d, MetricSpec m, bool p
   return status;
 }
 
-namespace {
-
-// Spatial order stratified by core distance: the points above the 90th
-// percentile of core distances (noise, in sparse regions) get their own k-d
-// order after the others'. A pruned pass skips a column tile when its bound
-// exceeds the largest current best of the row tile, and one sparse point's
-// large mutual-reachability weight would otherwise hold that bound up for the
-// dense points it shares a tile with. Returns the new order (original
-// indices) and new position -> old position, or empty vectors when one
-// class would be empty.
-void coreStratifiedOrder(const DevicePoints &pts, int n, int d, const std::vector<float> &core,
-                         std::vector<int> &order, std::vector<int> &newToOld) {
-  std::vector<float> sorted(core);
-  const size_t q = (size_t)(0.9 * n);
-  std::nth_element(sorted.begin(), sorted.begin() + q, sorted.end());
-  const float threshold = sorted[q];
-  std::vector<int> low, high; // original indices
-  for (int p = 0; p < n; ++p)
-    (core[p] > threshold ? high : low).push_back(pts.order[p]);
-  if (low.size() < 128 || high.size() < 128)
-    return;
-  spatialOrderIndices(pts.host, d, low.data(), (int)low.size());
-  spatialOrderIndices(pts.host, d, high.data(), (int)high.size());
-  order = low;
-  order.insert(order.end(), high.begin(), high.end());
-  std::vector<int> oldPos(n);
-  for (int p = 0; p < n; ++p)
-    oldPos[pts.order[p]] = p;
-  newToOld.resize(n);
-  for (int p = 0; p < n; ++p)
-    newToOld[p] = oldPos[order[p]];
-}
-
-} // namespace
-
 int hdbscanTree(const DevicePoints &pts, int n, int d, MetricSpec m, int minSamples, float alpha,
                 int coreMethod, bool prune, PassStats *stats, double *tree, float *hostCore) {
   DevArray<float> core;
@@ -278,22 +237,17 @@ int hdbscanTree(const DevicePoints &pts, int n, int d, MetricSpec m, int minSamp
   // on the order).
   const float *X = pts.data();
   const int *devOrig = pts.ordered() ? pts.orig.get() : nullptr;
-  const std::vector<int> *order = &pts.order;
-  std::vector<int> stratified, newToOld;
+  bool stratified = false;
   DevArray<float> sPoints, sCore;
   DevArray<int> sOrig, sMap;
-  if (s.ok() && prune && pts.ordered() && pts.host && n >= 1024) {
-    std::vector<float> hc(n);
-    s(download(hc.data(), core, n * sizeof(float)));
+  if (s.ok() && prune && pts.ordered() && n >= 1024) {
+    s(sOrig.alloc(n));
+    s(sMap.alloc(n));
     if (s.ok())
-      coreStratifiedOrder(pts, n, d, hc, stratified, newToOld);
-    if (s.ok() && !stratified.empty()) {
+      s(coreStratifiedOrder(X, n, d, core, devOrig, sMap, sOrig, &stratified));
+    if (s.ok() && stratified) {
       s(sPoints.alloc((size_t)n * d));
       s(sCore.alloc(n));
-      s(sOrig.alloc(n));
-      s(sMap.alloc(n));
-      s(upload(sOrig, stratified.data(), n * sizeof(int)));
-      s(upload(sMap, newToOld.data(), n * sizeof(int)));
       if (s.ok()) {
         s(gatherRows(X, sMap, n, d, sPoints));
         s(gatherRows(core, sMap, n, 1, sCore));
@@ -301,7 +255,6 @@ int hdbscanTree(const DevicePoints &pts, int n, int d, MetricSpec m, int minSamp
       if (s.ok()) {
         X = sPoints;
         devOrig = sOrig;
-        order = &stratified;
       }
       if (s.ok() && keepLists) {
         // List rows stay in the old order (rowMap = new -> old); partners
@@ -324,16 +277,20 @@ int hdbscanTree(const DevicePoints &pts, int n, int d, MetricSpec m, int minSamp
   opt.lists = keepLists && lists.pos.get() ? &lists : nullptr;
   WeightSpec w;
   w.kind = kWeightMReach;
-  w.core = stratified.empty() ? core.get() : sCore.get();
+  w.core = stratified ? sCore.get() : core.get();
   w.alpha = alpha;
   Contraction ct;
   if (s.ok())
     s(boruvkaMst(X, n, d, m, w, opt, ct));
   if (s.ok() && hostCore) {
-    std::vector<float> c(n);
-    s(download(c.data(), w.core, n * sizeof(float)));
-    for (int i = 0; i < n; ++i)
-      hostCore[pts.ordered() ? (*order)[i] : i] = c[i];
+    DevArray<float> byIndex; // in original order
+    if (devOrig) {
+      s(byIndex.alloc(n));
+      if (s.ok())
+        s(scatterFloats(w.core, devOrig, n, byIndex));
+    }
+    if (s.ok())
+      s(download(hostCore, devOrig ? byIndex.get() : w.core, n * sizeof(float)));
   }
   if (s.ok())
     s(treeFromDeviceEdges(ct.edges, n, tree));

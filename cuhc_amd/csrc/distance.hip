@@ -11,9 +11,6 @@
 #include "tile.hpp"
 
 #include <algorithm>
-#include <atomic>
-#include <thread>
-#include <numeric>
 #include <type_traits>
 
 namespace cuhc {
@@ -952,91 +949,6 @@ bool shouldPrune(int mode, int metricId, int n, int d) {
       d > kPruneHardMaxFeatures)
     return false;
   return mode == kPruneAlways || (n >= kPruneMinPoints && d <= kPruneMaxFeatures);
-}
-
-// k-d order: split each range at a tile boundary near its middle along the
-// feature with the widest spread (estimated from a sample), until each range
-// is one tile (the behaviour of reference src/spatial.cuh:48-91). The order
-// inside the partitions of nth_element is implementation-defined; ties between
-// equal weights always break by original index, so results do not depend on it.
-// The top levels run on one thread until there are enough ranges, then the
-// ranges are finished on up to 16 threads (disjoint ranges: the same order).
-void spatialOrderIndices(const float *pts, int d, int *idx, int count) {
-  constexpr int kTile = 128, kSample = 64;
-  struct Range {
-    int begin, end;
-  };
-  auto split = [&](Range range, std::vector<Range> &out) {
-    const int length = range.end - range.begin;
-    if (length <= kTile)
-      return;
-    int feature = 0;
-    float widest = -1.0f;
-    const int step = std::max(1, length / kSample);
-    for (int f = 0; f < d; ++f) {
-      float lo = INFINITY, hi = -INFINITY;
-      for (int i = range.begin; i < range.end; i += step) {
-        const float v = pts[(size_t)idx[i] * d + f];
-        lo = std::min(lo, v);
-        hi = std::max(hi, v);
-      }
-      if (hi - lo > widest) {
-        widest = hi - lo;
-        feature = f;
-      }
-    }
-    const int tiles = (length + kTile - 1) / kTile;
-    const int middle = range.begin + tiles / 2 * kTile;
-    std::nth_element(idx + range.begin, idx + middle, idx + range.end, [&](int x, int y) {
-      return pts[(size_t)x * d + feature] < pts[(size_t)y * d + feature];
-    });
-    out.push_back({range.begin, middle});
-    out.push_back({middle, range.end});
-  };
-  auto finish = [&](Range range) {
-    std::vector<Range> stack{range};
-    while (!stack.empty()) {
-      const Range r = stack.back();
-      stack.pop_back();
-      split(r, stack);
-    }
-  };
-  const unsigned threads = std::max(1u, std::min(16u, std::thread::hardware_concurrency()));
-  // Runs job(i) for i < count on the pool (disjoint ranges of idx).
-  auto parallel = [&](size_t jobs, auto &&job) {
-    std::atomic<size_t> cursor{0};
-    auto worker = [&]() {
-      for (size_t i = cursor++; i < jobs; i = cursor++)
-        job(i);
-    };
-    std::vector<std::thread> pool;
-    for (unsigned t = 1; t < std::min<size_t>(threads, jobs); ++t)
-      pool.emplace_back(worker);
-    worker();
-    for (auto &t : pool)
-      t.join();
-  };
-  // Breadth first, one level at a time, each level's ranges in parallel,
-  // until there are enough ranges to finish them depth first in parallel.
-  std::vector<Range> level{{0, count}};
-  while (level.size() < 4 * threads) {
-    std::vector<std::vector<Range>> children(level.size());
-    parallel(level.size(), [&](size_t i) { split(level[i], children[i]); });
-    std::vector<Range> next;
-    for (const auto &c : children)
-      next.insert(next.end(), c.begin(), c.end());
-    if (next.empty())
-      return; // every range is one tile (ranges of one tile are final)
-    level.swap(next);
-  }
-  parallel(level.size(), [&](size_t i) { finish(level[i]); });
-}
-
-std::vector<int> spatialOrder(const float *pts, int n, int d) {
-  std::vector<int> order(n);
-  std::iota(order.begin(), order.end(), 0);
-  spatialOrderIndices(pts, d, order.data(), n);
-  return order;
 }
 
 int gatherRows(const float *src, const int *order, int n, int d, float *dst) {

@@ -8,23 +8,21 @@
 
 namespace cuhc {
 
-// Points on the device, possibly in spatial order (order[i] = original index
-// of position i; empty = identity).
+// Points on the device, possibly in spatial order (orig[i] = original index
+// of position i).
 struct DevicePoints {
   DevArray<float> points;
-  DevArray<int> orig; // device copy of order (only when ordered)
-  std::vector<int> order;
-  bool ordered() const { return !order.empty(); }
+  DevArray<int> orig; // only when ordered
+  bool inOrder = false;
+  bool ordered() const { return inOrder; }
   // Uploads hostPoints (n x d), in spatial order if spatial is set.
   int upload(const float *hostPoints, int n, int d, bool spatial);
   // Adopts device-resident points (no copy unless spatial order is wanted).
   int adopt(const float *devicePoints, int n, int d, bool spatial);
+  // The spatial order of X into orig and points.
+  int arrange(const float *X, int n, int d);
   const float *data() const { return external ? external : points.get(); }
   const float *external = nullptr;
-  // Host coordinates in original order while ordered (the caller's array, or
-  // hostCopy for device-resident input).
-  const float *host = nullptr;
-  std::vector<float> hostCopy;
 };
 
 // Edges of a spanning forest in device memory (original indices, u < v): u, v

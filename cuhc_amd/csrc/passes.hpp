@@ -55,10 +55,22 @@ enum PruneMode : int { kPruneAuto = 0, kPruneAlways = 1, kPruneNever = 2 };
 
 bool shouldPrune(int mode, int metricId, int n, int d);
 
-// k-d order on the host: order[i] = original index of the point at position i.
-std::vector<int> spatialOrder(const float *hostPoints, int n, int d);
-// The same order of the listed points (indices into hostPoints), in place.
-void spatialOrderIndices(const float *hostPoints, int d, int *idx, int count);
+// k-d order of the listed points (indices into X; null: all of the first
+// count), all arrays on the device: order[i] = index of the point at position i.
+int spatialOrder(const float *X, int d, const int *list, int count, int *order);
+// The order of mutual-reachability passes over X (n points in k-d order, orig:
+// position -> original index): the points above the 90th percentile of core
+// distances (noise, in sparse regions) get their own k-d order after the
+// others'. A pruned pass skips a column tile when its bound exceeds the
+// largest current best of the row tile, and one sparse point's large
+// mutual-reachability weight would otherwise hold that bound up for the dense
+// points it shares a tile with. newToOld: new position -> position in X;
+// newOrig: new position -> original index. Left alone (*stratified false)
+// when one class would have less than a tile.
+int coreStratifiedOrder(const float *X, int n, int d, const float *core, const int *orig,
+                        int *newToOld, int *newOrig, bool *stratified);
+// dst[to[i]] = src[i].
+int scatterFloats(const float *src, const int *to, int n, float *dst);
 
 // dst[i] = src[order[i]] (rows of d floats).
 int gatherRows(const float *src, const int *order, int n, int d, float *dst);

@@ -38,6 +38,20 @@ def test_contraction_forms(data, n):
     np.testing.assert_array_equal(run(X, "manhattan"), oracle.single_linkage(X, "manhattan"))
 
 
+@pytest.mark.parametrize("n, d", [(129, 1), (257, 3), (1025, 65), (4000, 2), (20001, 5)])
+@pytest.mark.parametrize("spread", ["even", "outlier", "constant"])
+def test_spatial_order_shapes(n, d, spread):
+    # Pruned passes over the device's k-d order: last tiles of one point, more
+    # features than a wave samples rows, one value far from the others (every
+    # quantised value but its own in one bucket), and a feature that is constant.
+    X = np.random.default_rng(n + d).normal(size=(n, d)).astype(np.float32)
+    if spread == "outlier":
+        X[n // 2] = 1e6
+    elif spread == "constant":
+        X[:, 0] = 1.0
+    np.testing.assert_array_equal(run(X, pruning="always"), oracle.single_linkage(X))
+
+
 @pytest.mark.parametrize("metric", ["euclidean", "sqeuclidean", "manhattan", "chebyshev",
                                     "cosine"])
 @pytest.mark.parametrize("n", [2, 3, 127, 128, 129, 300])
