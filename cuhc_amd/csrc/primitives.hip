@@ -23,11 +23,21 @@ namespace {
 constexpr int kThreads = 256;
 constexpr int kPerThread = 16;
 constexpr int kTile = kThreads * kPerThread;
+// Items per workgroup of a radix pass: a workgroup places its items 256 at a
+// time, each step behind three barriers, so small sorts take 1,024 (four
+// steps, 16 to 6 us per scatter of 100,000 items, @@) and sorts that fill the device
+// anyway 4,096 (fewer digit counts to scan).
+constexpr int kSmallPerThread = 4;
+constexpr int kSmallSort = 1 << 19;
 constexpr int kRadixBits = 8;
 constexpr int kDigits = 1 << kRadixBits;
 
 size_t align256(size_t bytes) { return (bytes + 255) / 256 * 256; }
 int tilesOf(int count) { return (count + kTile - 1) / kTile; }
+int sortTiles(int count) {
+  const long long tile = (count <= kSmallSort ? kSmallPerThread : kPerThread) * kThreads;
+  return (int)((count + tile - 1) / tile);
+}
 
 DEV int waveSum(int v) {
 #pragma unroll
@@ -95,16 +105,16 @@ __global__ void __launch_bounds__(kThreads)
   }
 }
 
-template <class Key>
+template <int PER, class Key>
 __global__ void __launch_bounds__(kThreads)
     digitCountsKernel(const Key *__restrict__ keys, int count, int shift, unsigned int digitMask,
                       int tiles, int *__restrict__ counts) {
   __shared__ int hist[kDigits];
   hist[threadIdx.x] = 0;
   __syncthreads();
-  const size_t base = (size_t)blockIdx.x * kTile;
+  const size_t base = (size_t)blockIdx.x * PER * kThreads;
 #pragma unroll 4
-  for (int j = 0; j < kPerThread; ++j) {
+  for (int j = 0; j < PER; ++j) {
     const size_t i = base + (size_t)j * kThreads + threadIdx.x;
     if (i < (size_t)count)
       atomicAdd(&hist[(unsigned int)(keys[i] >> shift) & digitMask], 1);
@@ -113,7 +123,7 @@ __global__ void __launch_bounds__(kThreads)
   counts[(size_t)threadIdx.x * tiles + blockIdx.x] = hist[threadIdx.x];
 }
 
-template <class Key, class Value>
+template <int PER, class Key, class Value>
 __global__ void __launch_bounds__(kThreads)
     scatterKernel(const Key *__restrict__ keysIn, const Value *__restrict__ valuesIn,
                   Key *__restrict__ keysOut, Value *__restrict__ valuesOut, int count, int shift,
@@ -127,8 +137,8 @@ __global__ void __launch_bounds__(kThreads)
     waveCount[w][threadIdx.x] = 0;
   __syncthreads();
   const unsigned long long below = (1ull << lane) - 1ull;
-  const size_t base = (size_t)blockIdx.x * kTile;
-  for (int j = 0; j < kPerThread; ++j) {
+  const size_t base = (size_t)blockIdx.x * PER * kThreads;
+  for (int j = 0; j < PER; ++j) {
     const size_t i = base + (size_t)j * kThreads + threadIdx.x;
     const bool valid = i < (size_t)count;
     Key key = 0;
@@ -171,7 +181,7 @@ __global__ void __launch_bounds__(kThreads)
 }
 
 template <class Key, class Value> size_t sortTempBytes(int count) {
-  const int tiles = std::max(1, tilesOf(count));
+  const int tiles = std::max(1, sortTiles(count));
   const int countsLen = kDigits * tiles;
   return align256((size_t)count * sizeof(Key)) + align256((size_t)count * sizeof(Value)) +
          2 * align256((size_t)countsLen * sizeof(int)) + scanTempBytes(countsLen);
@@ -191,7 +201,7 @@ int sortPairs(const Key *keysIn, Key *keysOut, const Value *valuesIn, Value *val
                           hipMemcpyDeviceToDevice, stream()));
     return s.code;
   }
-  const int tiles = tilesOf(count);
+  const int tiles = sortTiles(count);
   const int countsLen = kDigits * tiles;
   char *t = static_cast<char *>(temp);
   Key *keysAlt = reinterpret_cast<Key *>(t);
@@ -213,12 +223,16 @@ int sortPairs(const Key *keysIn, Key *keysOut, const Value *valuesIn, Value *val
     const int shift = p * kRadixBits;
     const int width = std::min(kRadixBits, bits - shift);
     const unsigned int mask = (1u << width) - 1u;
-    hipLaunchKernelGGL((digitCountsKernel<Key>), dim3(tiles), dim3(kThreads), 0, stream(), srcK,
-                       count, shift, mask, tiles, counts);
+    const bool smallSort = count <= kSmallSort;
+    hipLaunchKernelGGL((smallSort ? digitCountsKernel<kSmallPerThread, Key>
+                                  : digitCountsKernel<kPerThread, Key>),
+                       dim3(tiles), dim3(kThreads), 0, stream(), srcK, count, shift, mask, tiles,
+                       counts);
     s((int)hipGetLastError());
     s(exclusiveScan(counts, offsets, countsLen, scanTemp));
-    hipLaunchKernelGGL((scatterKernel<Key, Value>), dim3(tiles), dim3(kThreads), 0, stream(),
-                       srcK, srcV, dstK, dstV, count, shift, mask, tiles, offsets);
+    hipLaunchKernelGGL((smallSort ? scatterKernel<kSmallPerThread, Key, Value>
+                                  : scatterKernel<kPerThread, Key, Value>),
+                       dim3(tiles), dim3(kThreads), 0, stream(), srcK, srcV, dstK, dstV, count, shift, mask, tiles, offsets);
     s((int)hipGetLastError());
     srcK = dstK;
     srcV = dstV;
