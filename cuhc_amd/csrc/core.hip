@@ -5,9 +5,11 @@
 // fused (k <= 64): one workgroup per row tile walks the column tiles nearest
 //   first and keeps each row's k smallest distances sorted in LDS. After each
 //   tile the 16 lanes of a row mark the distances that beat the row's k-th,
-//   and the row's lowest lane with work inserts one value per step (64-bit
-//   ballot over the wave: 4 rows insert in parallel). Optional box pruning for
-//   points in spatial order.
+//   and insert them together, one value per step (64-bit ballot over the
+//   wave: 4 rows insert in parallel). Optional box pruning for points in
+//   spatial order, per wave: one box and one largest k-th distance over 128
+//   rows computed 47% of the pairs of 100,000 points of 8 features, by 32 rows
+//   26% (10^6 points, k = 25: core pass 159 to 135 ms, 100,000: 11.6 to 7.6).
 // radix: distances of a block of rows into a bounded buffer, then per row a
 //   4-pass MSB-first byte radix select over the FP32 bit patterns with
 //   per-wave LDS histograms.
@@ -22,13 +24,10 @@ namespace cuhc {
 
 namespace {
 
-// Column tile boxes (low/high per tile, numTiles > 0 turns pruning on), and
-// for gathered rows the boxes of their row tiles (rowLow/rowHigh; null: the
-// rows are the points themselves and share the column tiles' boxes).
+// Column tile boxes (low/high per tile; numTiles > 0 turns pruning on).
 struct CoreBoxes {
   const float *low = nullptr, *high = nullptr;
   int numTiles = 0;
-  const float *rowLow = nullptr, *rowHigh = nullptr;
 };
 
 DEV int walkTileCore(int rowTile, int step, int numTiles) {
@@ -50,30 +49,36 @@ DEV float coreBoxBound(const Metric &metric, const float *lowA, const float *hig
   return metric.finish(acc);
 }
 
-// Inserts v into the ascending list[0..k), dropping the largest, if v beats list[k-1].
-DEV void insertSorted(float *list, int k, float v) {
-  if (!(v < list[k - 1]))
-    return;
-  int pos = k - 1;
-  while (pos > 0 && list[pos - 1] > v) {
-    list[pos] = list[pos - 1];
-    --pos;
+// Inserts v into the ascending list[0..k), dropping the largest, by the 16
+// lanes of a tile row (lane16 = 0..15) together: entry s keeps its value up to
+// v, and above v takes the larger of v and its predecessor. One LDS round trip;
+// one lane shifting the entries took one per entry (k = 25: 2,003 points
+// unpruned 3.3 ms, now 0.96; 24,000 points of 20 features 6.9 ms, now 3.6).
+DEV void insertSorted(float *list, int k, int lane16, float v) {
+  // From the last 16 entries to the first: an entry's predecessor is read
+  // before it is written.
+#pragma unroll 1
+  for (int s = (k - 1) / 16 * 16 + lane16; s >= 0; s -= 16) {
+    if (s < k) {
+      const float cur = list[s], prev = s > 0 ? list[s - 1] : -INFINITY;
+      list[s] = cur > v ? fmaxf(prev, v) : cur;
+    }
+    __builtin_amdgcn_wave_barrier();
   }
-  list[pos] = v;
 }
 
 // Rows are the points themselves (rowsX null: row tile blockIdx.x of X, or
 // tile tileList[blockIdx.x] with a list) or listed points (rowsX: numRows
 // gathered rows, rowPos their positions in X, for the exact search of
 // selected points).
-// Four waves per SIMD for the one-fill tiles (d <= 8) of the squared-sum
-// metrics: the pass waits on tile loads, and the extra wave hides more of them
-// than its few spills cost (1M points, d = 8: 195 to 168 ms). The other folds
-// would spill far more at 128 VGPRs.
+// Three waves per SIMD for the one-fill tiles (d <= 8) of the squared-sum
+// metrics: the pass waits on tile loads, and 160 VGPRs hold it without spills
+// (at four, 62 registers spill: 10^6 points, d = 8, 225 ms against 166 before
+// the rows were bounded by wave).
 template <class T, class Metric> constexpr int coreMinWaves() {
   return T::FILL <= 8 &&
                  (std::is_same<Metric, Euclidean>::value || std::is_same<Metric, SqEuclidean>::value)
-             ? 4
+             ? 3
              : 1;
 }
 
@@ -83,34 +88,44 @@ __global__ void __launch_bounds__(256, (coreMinWaves<T, Metric>()))
                           float *__restrict__ core, CoreBoxes boxes, int stepLimit,
                           const float *__restrict__ rowsX, int numRows,
                           const int *__restrict__ rowPos, const int *__restrict__ tileList) {
-  constexpr int TR = T::TR;
-  constexpr int kBatch = 64; // walk steps whose box bounds wave 0 computes at once
+  constexpr int TR = T::TR, kWaves = T::THREADS / 64, kWaveRows = T::WAVE_ROWS;
+  constexpr int kBatch = 64; // walk steps whose box bounds are computed at once
   __shared__ __align__(16) TileSmem<T> sm;
-  __shared__ float lowerBound[kBatch];
-  __shared__ float largestKth; // the largest k-th distance over the tile's rows
-  __shared__ int inserted;     // a row's list changed in the current tile
-  extern __shared__ float lists[]; // [DIM][k], then the row tile's box (2d) if pruning
+  // Per wave: the bounds of the batch's steps, the steps within its largest
+  // k-th distance when the batch began, and that distance now.
+  __shared__ float lowerBound[kWaves][kBatch];
+  __shared__ unsigned long long within[kWaves];
+  __shared__ float largestKth[kWaves];
+  extern __shared__ float lists[]; // [DIM][k], then the waves' row boxes [kWaves][2 d] if pruning
 
   const int rowTile = tileList ? tileList[blockIdx.x] : (int)blockIdx.x;
   const int row0 = rowTile * T::DIM;
   const float *A = rowsX ? rowsX : X;
   const int nA = rowsX ? numRows : n;
+  const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
   for (int i = threadIdx.x; i < T::DIM * k; i += T::THREADS)
     lists[i] = INFINITY;
   const bool prune = boxes.numTiles > 0;
-  float *rowBox = lists + T::DIM * k;
+  float *rowBox = lists + T::DIM * k + wave * 2 * d;
   if (prune) {
-    const float *rl = boxes.rowLow ? boxes.rowLow : boxes.low;
-    const float *rh = boxes.rowHigh ? boxes.rowHigh : boxes.high;
-    for (int f = threadIdx.x; f < d; f += T::THREADS) {
-      rowBox[f] = rl[(size_t)rowTile * d + f];
-      rowBox[d + f] = rh[(size_t)rowTile * d + f];
+    const int row = row0 + wave * kWaveRows + (lane & (kWaveRows - 1));
+    for (int f = 0; f < d; ++f) {
+      const float v = row < nA ? A[(size_t)row * d + f] : 0.0f;
+      float lo = row < nA ? v : INFINITY, hi = row < nA ? v : -INFINITY;
+#pragma unroll
+      for (int m = kWaveRows / 2; m > 0; m >>= 1) {
+        lo = fminf(lo, __shfl_xor(lo, m, 64));
+        hi = fmaxf(hi, __shfl_xor(hi, m, 64));
+      }
+      if (lane == 0) {
+        rowBox[f] = lo;
+        rowBox[d + f] = hi;
+      }
     }
   }
-  if (threadIdx.x == 0) {
-    largestKth = INFINITY; // every list starts empty
-    inserted = 0;
-  }
+  // A wave without rows needs no tile; the others' lists start empty.
+  if (lane == 0)
+    largestKth[wave] = row0 + wave * kWaveRows < nA ? INFINITY : -1.0f;
   // The 8-feature tiles serve d <= 8 only (one fill): the row slice is
   // staged once for every tile.
   constexpr bool kRowsResident = T::FILL == 8;
@@ -119,7 +134,6 @@ __global__ void __launch_bounds__(256, (coreMinWaves<T, Metric>()))
   __syncthreads();
   const float slack = 1.0f - coreBoxSlack(d);
   const int numTiles = (n + T::DIM - 1) / T::DIM;
-  const int lane = threadIdx.x & 63;
   const unsigned long long groupMask = 0xffffull << (lane & 48);
   // Listed rows have no home tile: the walk starts anywhere and covers all;
   // with pruning (rows listed in point order) it starts at the column tile of
@@ -127,120 +141,139 @@ __global__ void __launch_bounds__(256, (coreMinWaves<T, Metric>()))
   const int homeTile =
       rowsX ? (prune ? rowPos[row0] / T::DIM : (int)(blockIdx.x % numTiles)) : rowTile;
 
-  // A step is skipped when the box bound between the row tile and its column
-  // tile exceeds the largest k-th distance of the tile's rows: wave 0 computes
-  // the bounds of 64 steps at once into LDS, and the largest k-th distance
-  // is refreshed only after a tile that changed a list, so skipped steps and
-  // unchanged tiles cost no barrier.
+  // A wave leaves out a step when the box bound between its rows and the
+  // column tile exceeds the largest k-th distance of those rows, and the
+  // workgroup skips it when every wave does. Every wave computes its bounds of
+  // 64 steps at once; only the steps some wave still had within reach when
+  // the batch began are looked at again.
   const int steps = min(2 * numTiles, stepLimit);
   for (int base = 0; base < steps; base += kBatch) {
-    if (prune) {
-      if (threadIdx.x < kBatch) {
-        const int step = base + (int)threadIdx.x;
-        const int colTile = step < steps ? walkTileCore(homeTile, step, numTiles) : -1;
-        lowerBound[threadIdx.x] =
-            colTile >= 0 ? coreBoxBound(metric, rowBox, rowBox + d, boxes.low + (size_t)colTile * d,
-                                        boxes.high + (size_t)colTile * d, d) * slack
-                         : 0.0f;
-      }
-      __syncthreads();
-    }
-    const int batchEnd = min(steps, base + kBatch);
-    for (int step = base; step < batchEnd; ++step) {
-      const int colTile = walkTileCore(homeTile, step, numTiles);
-      if (colTile < 0)
-        continue;
+    unsigned long long todo;
+    {
+      const int step = base + lane;
+      const int colTile = step < steps ? walkTileCore(homeTile, step, numTiles) : -1;
+      float lb = 0.0f;
+      if (prune && colTile >= 0)
+        lb = coreBoxBound(metric, rowBox, rowBox + d, boxes.low + (size_t)colTile * d,
+                          boxes.high + (size_t)colTile * d, d) * slack;
+      todo = __ballot(colTile >= 0 && !(prune && lb > largestKth[wave]));
       if (prune) {
-        const float largest = largestKth; // uniform: LDS, written only between barriers
-        if (largest != INFINITY && lowerBound[step - base] > largest)
+        lowerBound[wave][lane] = lb;
+        if (lane == 0)
+          within[wave] = todo;
+        __syncthreads();
+        todo = 0;
+#pragma unroll
+        for (int w = 0; w < kWaves; ++w)
+          todo |= within[w];
+      }
+    }
+    for (; todo; todo &= todo - 1) {
+      const int j = __ffsll((long long)todo) - 1;
+      // Uniform: written before the barrier after the last computed tile.
+      bool active = true;
+      if (prune) {
+        bool any = false;
+#pragma unroll
+        for (int w = 0; w < kWaves; ++w) {
+          const bool reach = !(lowerBound[w][j] > largestKth[w]);
+          any |= reach;
+          if (w == wave)
+            active = reach;
+        }
+        if (!any)
           continue;
       }
-      const int col0 = colTile * T::DIM;
+      const int col0 = walkTileCore(homeTile, base + j, numTiles) * T::DIM;
       // With an accumulator bound the tile holds raw accumulators, and only the
       // pairs within the bound of the row's current k-th distance are finished
       // (most pairs of a tile are not, which skips their sqrt).
       constexpr bool kFilter = Metric::kAccFilter;
       float v[TR][TR];
-      computeTile<T, Metric, !kFilter, kRowsResident>(sm, A, nA, X, n, d, metric, row0, col0, v);
+      computeTile<T, Metric, !kFilter, kRowsResident, true>(sm, A, nA, X, n, d, metric, row0,
+                                                            col0, v, NoExtraStage{}, active);
+      if (active) {
+        unsigned long long changed = 0;
 #pragma unroll
-      for (int r = 0; r < TR; ++r) {
-        const int rit = T::rowInTile(r);
-        const int row = row0 + rit;
-        float *list = lists + rit * k;
-        unsigned int pending = 0;
-        if (row < nA) {
-          const float kth = list[k - 1];
-          const int self = rowsX ? rowPos[row] : row;
-          if constexpr (kFilter) {
-            const float limit = metric.accBound(kth);
+        for (int r = 0; r < TR; ++r) {
+          int rit = T::rowInTile(r);
+          asm volatile("" : "+v"(rit)); // computed here, not kept for every row
+          const int row = row0 + rit;
+          float *list = lists + rit * k;
+          unsigned int pending = 0;
+          if (row < nA) {
+            const float kth = list[k - 1];
+            const int self = rowsX ? rowPos[row] : row;
+            if constexpr (kFilter) {
+              const float limit = metric.accBound(kth);
 #pragma unroll
-            for (int c = 0; c < TR; ++c) {
-              const int col = col0 + T::colInTile(c);
-              const float acc = v[r][c];
-              if (col < n && !(acc > limit)) {
-                const float value = col == self ? 0.0f : fmaxf(metric.finish(acc), 0.0f);
-                v[r][c] = value;
-                if (value < kth)
+              for (int c = 0; c < TR; ++c) {
+                const int col = col0 + T::colInTile(c);
+                const float acc = v[r][c];
+                if (col < n && !(acc > limit)) {
+                  const float value = col == self ? 0.0f : fmaxf(metric.finish(acc), 0.0f);
+                  v[r][c] = value;
+                  if (value < kth)
+                    pending |= 1u << c;
+                }
+              }
+            } else {
+#pragma unroll
+              for (int c = 0; c < TR; ++c) {
+                const int col = col0 + T::colInTile(c);
+                // The point itself is distance 0 (drops float noise such as cosine's 1e-7).
+                v[r][c] = col == self ? 0.0f : fmaxf(v[r][c], 0.0f);
+                if (col < n && v[r][c] < kth)
                   pending |= 1u << c;
               }
             }
-          } else {
+          }
+          // One insertion per row per step until no lane of the wave has work;
+          // all lanes stay converged for the ballot. The row's lowest lane with
+          // work gives its value, the row's 16 lanes insert it, and every lane
+          // drops the values that no longer beat the k-th.
+          while (true) {
+            const unsigned long long work = __ballot(pending != 0);
+            if (work == 0)
+              break;
+            changed |= work;
+            const unsigned long long mine = work & groupMask;
+            const int source = mine ? __ffsll((long long)mine) - 1 : lane;
+            float value = 0.0f;
+            const int first = __ffs(pending) - 1;
 #pragma unroll
-            for (int c = 0; c < TR; ++c) {
-              const int col = col0 + T::colInTile(c);
-              // The point itself is distance 0 (drops float noise such as cosine's 1e-7).
-              v[r][c] = col == self ? 0.0f : fmaxf(v[r][c], 0.0f);
-              if (col < n && v[r][c] < kth)
-                pending |= 1u << c;
+            for (int cc = 0; cc < TR; ++cc)
+              if (cc == first)
+                value = v[r][cc];
+            value = __shfl(value, source, 64);
+            if (lane == source)
+              pending &= pending - 1;
+            if (mine)
+              insertSorted(list, k, lane & 15, value);
+            __builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront");
+            __builtin_amdgcn_wave_barrier();
+            __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "wavefront");
+            if (pending) {
+              const float kth = list[k - 1];
+#pragma unroll
+              for (int c = 0; c < TR; ++c)
+                if (!(v[r][c] < kth))
+                  pending &= ~(1u << c);
             }
           }
         }
-        // One insertion per row per step until no lane of the wave has work;
-        // all lanes stay converged for the ballot.
-        while (true) {
-          const unsigned long long work = __ballot(pending != 0);
-          if (work == 0)
-            break;
-          const unsigned long long mine = work & groupMask;
-          if (mine != 0 && lane == __ffsll((long long)mine) - 1) {
-            const int c = __ffs(pending) - 1;
-            pending &= pending - 1;
-            float value = 0.0f;
+        // The wave's rows are its own: it refreshes their largest k-th itself.
+        if (prune && changed) {
+          const int i = wave * kWaveRows + (lane & (kWaveRows - 1));
+          float largest = row0 + i < nA ? lists[i * k + k - 1] : -1.0f;
 #pragma unroll
-            for (int cc = 0; cc < TR; ++cc)
-              if (cc == c)
-                value = v[r][cc];
-            insertSorted(list, k, value);
-            if (prune)
-              inserted = 1;
-          }
-          __builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront");
-          __builtin_amdgcn_wave_barrier();
-          __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "wavefront");
+          for (int m = kWaveRows / 2; m > 0; m >>= 1)
+            largest = fmaxf(largest, __shfl_xor(largest, m, 64));
+          if (lane == 0)
+            largestKth[wave] = largest;
         }
       }
-      if (prune) {
-        __syncthreads(); // insertions done
-        // Every wave reads the flag after the barrier above; it is cleared
-        // after the barrier below and set again only after the next tile's
-        // first barrier, so every wave takes the same branch.
-        if (inserted) {
-          if (threadIdx.x < 64) {
-            float largest = 0.0f;
-            for (int i = threadIdx.x; i < T::DIM; i += 64)
-              if (row0 + i < nA)
-                largest = fmaxf(largest, lists[i * k + k - 1]);
-#pragma unroll
-            for (int m = 32; m > 0; m >>= 1)
-              largest = fmaxf(largest, __shfl_xor(largest, m, 64));
-            if (threadIdx.x == 0)
-              largestKth = largest;
-          }
-          __syncthreads();
-          if (threadIdx.x == 0)
-            inserted = 0;
-        }
-      }
+      __syncthreads(); // the tile is consumed, the largest k-th distances are current
     }
     if (prune)
       __syncthreads(); // lowerBound is rewritten by the next batch
@@ -296,18 +329,40 @@ __global__ void __launch_bounds__(256)
         atomicAdd(&hist[wave][(bits >> shift) & 0xffu], 1u);
     }
     __syncthreads();
-    if (threadIdx.x == 0) {
-      unsigned int below = 0, bin = 0;
-      while (true) {
-        const unsigned int count = hist[0][bin] + hist[1][bin] + hist[2][bin] + hist[3][bin];
-        if (below + count >= remaining || bin == 255)
-          break;
-        below += count;
-        ++bin;
+    // The first bin that reaches `remaining`: one wave, four bins per lane (one
+    // thread stepping through the bins took 14 us per digit).
+    if (wave == 0) {
+      const int lane = threadIdx.x;
+      unsigned int count[4], sum = 0;
+#pragma unroll
+      for (int q = 0; q < 4; ++q) {
+        const int bin = 4 * lane + q;
+        count[q] = hist[0][bin] + hist[1][bin] + hist[2][bin] + hist[3][bin];
+        sum += count[q];
       }
-      remaining -= below;
-      prefix |= bin << shift;
-      prefixMask |= 0xffu << shift;
+      unsigned int upTo = sum;
+#pragma unroll
+      for (int m = 1; m < 64; m <<= 1) {
+        const unsigned int up = __shfl_up(upTo, m, 64);
+        if (lane >= m)
+          upTo += up;
+      }
+      const unsigned long long reached = __ballot(upTo >= remaining);
+      // Every value is finite: some bin reaches it.
+      const int first = reached ? __ffsll((long long)reached) - 1 : 63;
+      if (lane == first) {
+        unsigned int below = upTo - sum;
+        int q = 0;
+#pragma unroll
+        for (int b = 0; b < 3; ++b)
+          if (q == b && below + count[b] < remaining) {
+            below += count[b];
+            ++q;
+          }
+        remaining -= below;
+        prefix |= (unsigned int)(4 * lane + q) << shift;
+        prefixMask |= 0xffu << shift;
+      }
     }
     __syncthreads();
   }
@@ -347,7 +402,7 @@ int coreFused(const float *X, int n, int d, MetricSpec m, int k, float *core, bo
         hipLaunchKernelGGL(coreBoxesKernel, dim3(tiles), dim3(64), 0, stream(), X, n, d, T::DIM,
                            low.get(), high.get());
         boxes = CoreBoxes{low, high, tiles};
-        smem += 2 * d * sizeof(float);
+        smem += (T::THREADS / 64) * 2 * d * sizeof(float);
       }
       PhaseTimer timer(kPhaseCore);
       hipLaunchKernelGGL((kthNearestFusedKernel<T, Metric>), dim3(tileList ? numListed : tiles),
@@ -428,22 +483,18 @@ int coreForRowsFused(const float *X, int n, int d, MetricSpec m, int k, const in
       const int rowTiles = (numRows + T::DIM - 1) / T::DIM;
       size_t smem = (size_t)T::DIM * k * sizeof(float);
       CoreBoxes boxes;
-      DevArray<float> low, high, rowLow, rowHigh;
+      DevArray<float> low, high;
       Status st;
       if (prune && Metric::kBoxBound) {
         const int tiles = (n + T::DIM - 1) / T::DIM;
         st(low.alloc((size_t)tiles * d));
         st(high.alloc((size_t)tiles * d));
-        st(rowLow.alloc((size_t)rowTiles * d));
-        st(rowHigh.alloc((size_t)rowTiles * d));
         if (!st.ok())
           return st.code;
         hipLaunchKernelGGL(coreBoxesKernel, dim3(tiles), dim3(64), 0, stream(), X, n, d, T::DIM,
                            low.get(), high.get());
-        hipLaunchKernelGGL(coreBoxesKernel, dim3(rowTiles), dim3(64), 0, stream(),
-                           rowData.get(), numRows, d, T::DIM, rowLow.get(), rowHigh.get());
-        boxes = CoreBoxes{low, high, tiles, rowLow, rowHigh};
-        smem += 2 * d * sizeof(float);
+        boxes = CoreBoxes{low, high, tiles};
+        smem += (T::THREADS / 64) * 2 * d * sizeof(float);
       }
       PhaseTimer timer(kPhaseCore);
       hipLaunchKernelGGL((kthNearestFusedKernel<T, Metric>), dim3(rowTiles), dim3(256), smem,

@@ -344,13 +344,10 @@ struct Boxes {
   int numTiles = 0;
 };
 
-// Boxes of the tiles of X (n points of d features, tileDim per tile). The
-// weight values and components of point p are those of position pos[p]
-// (pos null: p), for rows gathered out of the full order.
+// Boxes of the tiles of X (n points of d features, tileDim per tile).
 template <class Weight>
 __global__ void buildBoxesKernel(const float *__restrict__ X, int n, int d, int tileDim,
-                                 Weight weight, const int *__restrict__ comp,
-                                 const int *__restrict__ pos, Boxes boxes) {
+                                 Weight weight, const int *__restrict__ comp, Boxes boxes) {
   const int tile = blockIdx.x;
   const int first = tile * tileDim, last = min(n, first + tileDim);
   for (int f = threadIdx.x; f < d; f += blockDim.x) {
@@ -368,9 +365,8 @@ __global__ void buildBoxesKernel(const float *__restrict__ X, int n, int d, int 
     float mv = INFINITY;
     int cmin = 0x7fffffff, cmax = -1;
     for (int p = first + (int)threadIdx.x; p < last; p += 64) {
-      const int q = pos ? pos[p] : p;
-      mv = fminf(mv, (float)weight.value(q));
-      const int c = comp ? comp[q] : 0;
+      mv = fminf(mv, (float)weight.value(p));
+      const int c = comp ? comp[p] : 0;
       cmin = min(cmin, c);
       cmax = max(cmax, c);
     }
@@ -450,28 +446,37 @@ template <class Weight> struct ColumnStage {
 };
 
 // One workgroup per row tile walks the column tiles outward from its own
-// (walkTile order). Lower bounds of the weight between the two boxes are
-// computed 64 steps at a time by wave 0, one step per lane, into LDS; a step
-// is skipped when its bound exceeds every row's need. A row needs candidates
-// below min(its current best, its component's best known edge): Boruvka only
-// uses each component's smallest outgoing edge, so once any point of the
-// component has found an edge of weight b, no row of that component needs a
-// candidate above b (compBest, shared by all workgroups through atomicMin on
-// the weight bits; null disables it). The row that holds the component's
-// smallest edge always finds it exactly; other rows may stop early, and their
-// results are then only upper bounds, which the contraction never prefers.
-// The same need filters single pairs: wave 0 publishes each row's need in
-// LDS, and for metrics with an accumulator bound a pair is finished (sqrt,
-// weight, key) only when its raw accumulator is within the row's need and
-// it crosses components; the pairs filtered out weigh more than the need.
+// (walkTile order). Each wave owns 32 consecutive rows and computes the lower
+// bounds of the weight between their box and the column tiles' boxes 64 steps
+// at a time, one step per lane; it leaves out a step whose bound exceeds every
+// one of its rows' need, and the workgroup skips the step when all waves do. A
+// row needs candidates below min(its current best, its component's best known
+// edge): Boruvka only uses each component's smallest outgoing edge, so once any
+// point of the component has found an edge of weight b, no row of that
+// component needs a candidate above b (compBest, shared by all workgroups
+// through atomicMin on the weight bits; null disables it). The row that holds
+// the component's smallest edge always finds it exactly; other rows may stop
+// early, and their results are then only upper bounds, which the contraction
+// never prefers. The same need filters single pairs: every row's is published
+// in LDS, and for metrics with an accumulator bound a pair is finished (sqrt,
+// weight, key) only when its raw accumulator is within the row's need and it
+// crosses components; the pairs filtered out weigh more than the need.
+// A row belongs to one wave, so its best, need and list change without a
+// barrier; the tile needs two (its data staged; consumed, with the waves' bounds
+// current, on which all waves decide the next step alike).
+// Bound by FP32 VALU work at large n, by the longest row tile's walk where all
+// row tiles are resident at once. One box and one bound per 128-row tile
+// computed nearly twice the pairs (47% of all pairs of 100,000 points of 8
+// features against 26% by 32 rows). HDBSCAN's passes over 10^6 points of 8
+// features took 290 ms; by wave 235, and with the sparse tiles first 202.
+
 // The rows of a compact walk: n rows gathered into X (d features each) from
-// positions pos[0 .. n) of the full order (ascending), in tiles with their
-// own boxes; center[t] is the full-order tile around which row tile t walks.
+// positions pos[0 .. n) of the full order (ascending); center[t] is the
+// full-order tile around which row tile t walks.
 struct RowSet {
   const float *X = nullptr;
   int n = 0;
   const int *pos = nullptr;
-  Boxes boxes;
   const int *center = nullptr;
 };
 
@@ -483,8 +488,8 @@ struct RowSet {
 constexpr int kKeptKeys = 4;
 
 // The keeping walk runs the first round only; three waves per SIMD hide its
-// waits better than two despite 5 spilled registers (C3's four Borůvka walks:
-// 298 ms with two waves, 265 ms with three).
+// waits better than two (C3's four Borůvka walks: 298 ms with two waves, 265 ms
+// with three).
 template <class T, class Metric, class Weight, bool COMPACT = false, bool KEEP = false>
 __global__ void __launch_bounds__(256, (KEEP ? 3 : 1))
     nearestOtherWalkKernel(const float *__restrict__ X, int n, int d, Metric metric,
@@ -492,79 +497,93 @@ __global__ void __launch_bounds__(256, (KEEP ? 3 : 1))
                            const int *__restrict__ orig, Boxes boxes,
                            unsigned int *__restrict__ compBest,
                            unsigned long long *__restrict__ nearest,
-                           unsigned long long *tilesComputed, int rowTileStride,
+                           unsigned long long *wavesComputed, int rowTileStride,
                            int computeSteps, const int *__restrict__ skipComp,
                            const unsigned char *__restrict__ closedRows, RowSet rows,
                            unsigned long long *__restrict__ kept) {
-  constexpr int TR = T::TR;
+  constexpr int TR = T::TR, kWaves = T::THREADS / 64, kWaveRows = T::WAVE_ROWS;
+  constexpr int kBatch = 64;
+  static_assert(TR == 8 && kWaveRows == 32, "a wave's rows are its lower 32 lanes");
   __shared__ unsigned long long rowTop[KEEP ? T::DIM * kKeptKeys : 1];
   // Rows: the full order's tiles, or (COMPACT) the gathered rows, whose
   // position in the full order indexes comp, the weight values, closedRows
   // and nearest.
   const float *__restrict__ rowX = COMPACT ? rows.X : X;
   const int nRows = COMPACT ? rows.n : n;
-  const Boxes &rowBoxes = COMPACT ? rows.boxes : boxes;
   auto posOf = [&](int row) { return COMPACT ? rows.pos[row] : row; };
-  constexpr int kBatch = 64;
   __shared__ __align__(16) TileSmem<T> sm;
   __shared__ unsigned long long rowBest[T::DIM];
   __shared__ float rowNeed[T::DIM]; // -1: no row
-  __shared__ float lowerBound[kBatch];
-  __shared__ float bound;
-  __shared__ int tileImproved; // a row's best improved in the current tile
+  // Per wave: the batch's bounds, the steps within its reach when the batch
+  // began, and its largest need now (-1: no open row).
+  __shared__ float lowerBound[kWaves][kBatch];
+  __shared__ unsigned long long within[kWaves];
+  __shared__ float bound[kWaves];
   __shared__ int sColComp[T::DIM];
   __shared__ typename Weight::Value sColVal[T::DIM];
   __shared__ unsigned int sColIdx[T::DIM];
-  extern __shared__ float rowBox[]; // low[d], high[d]
+  extern __shared__ float rowBoxes[]; // per wave low[d], high[d]
   constexpr bool kFilter = Metric::kAccFilter && Weight::kDistBound;
 
-  const int rowTile = blockIdx.x * rowTileStride, numTiles = boxes.numTiles;
+  // Last tiles first: in the order by core distance they hold the sparse points,
+  // whose walks are the longest.
+  const int rowTile = (int)(gridDim.x - 1 - blockIdx.x) * rowTileStride;
+  const int numTiles = boxes.numTiles;
   const int row0 = rowTile * T::DIM;
   const int center = COMPACT ? rows.center[rowTile] : rowTile;
-  // Rows of the skipped component are closed; a tile of only such rows has
-  // nothing to do (uniform: every thread reads the same values).
-  const int skip = skipComp ? *skipComp : -1;
-  if (skip >= 0 && rowBoxes.minComp[rowTile] == skip && rowBoxes.maxComp[rowTile] == skip)
-    return;
+  const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
   // A row is open unless it lies past the end, in the skipped component, or
   // is closed (its exact answer is already in nearest[]).
+  const int skip = skipComp ? *skipComp : -1;
   auto isOpen = [&](int row) {
     if (row >= nRows)
       return false;
     const int p = posOf(row);
     return comp[p] != skip && !(closedRows && closedRows[p]);
   };
-  int anyOpen = 0;
+  // Lanes 0..31 own the wave's rows: whether open, component, and the
+  // component's best known edge (refreshed once per batch).
+  const int own = wave * kWaveRows + (lane & (kWaveRows - 1)), ownRow = row0 + own;
+  const bool open = lane < kWaveRows && isOpen(ownRow);
+  const int ownComp = open ? comp[posOf(ownRow)] : 0;
+  float cap = INFINITY;
+  if (!__syncthreads_or(open))
+    return; // uniform: every row of the tile is settled
   if (KEEP)
     for (int i = threadIdx.x; i < T::DIM * kKeptKeys; i += T::THREADS)
       rowTop[i] = kEmptyKey;
-  for (int i = threadIdx.x; i < T::DIM; i += T::THREADS) {
-    rowBest[i] = kEmptyKey;
-    const bool open = isOpen(row0 + i);
-    rowNeed[i] = open ? INFINITY : -1.0f;
-    anyOpen |= open;
+  if (lane < kWaveRows) {
+    rowBest[own] = kEmptyKey;
+    rowNeed[own] = open ? INFINITY : -1.0f;
   }
-  if (!__syncthreads_or(anyOpen))
-    return; // uniform: every row of the tile is settled
-  for (int k = threadIdx.x; k < d; k += T::THREADS) {
-    rowBox[k] = rowBoxes.low[(size_t)rowTile * d + k];
-    rowBox[d + k] = rowBoxes.high[(size_t)rowTile * d + k];
+  if (lane == 0)
+    bound[wave] = INFINITY;
+  // The box, smallest weight value and components of the wave's open rows.
+  float *rowBox = rowBoxes + wave * 2 * d;
+  for (int f = 0; f < d; ++f) {
+    const float v = open ? rowX[(size_t)ownRow * d + f] : 0.0f;
+    float lo = open ? v : INFINITY, hi = open ? v : -INFINITY;
+#pragma unroll
+    for (int m = kWaveRows / 2; m > 0; m >>= 1) {
+      lo = fminf(lo, __shfl_xor(lo, m, 64));
+      hi = fmaxf(hi, __shfl_xor(hi, m, 64));
+    }
+    if (lane == 0) {
+      rowBox[f] = lo;
+      rowBox[d + f] = hi;
+    }
   }
-  // Wave 0 owns rows lane and lane + 64 for the bound: their components and
-  // the components' best known edges (refreshed once per batch).
-  const int ra = row0 + (int)(threadIdx.x & 63), rb = ra + 64;
-  const bool open0 = threadIdx.x < 64 && isOpen(ra);
-  const bool open1 = threadIdx.x < 64 && isOpen(rb);
-  const int comp0 = open0 ? comp[posOf(ra)] : 0, comp1 = open1 ? comp[posOf(rb)] : 0;
-  float cap0 = INFINITY, cap1 = INFINITY;
+  float rowMinValue = open && Weight::kHasValue ? (float)weight.value(posOf(ownRow)) : INFINITY;
+  int compLow = open ? ownComp : 0x7fffffff, compHigh = open ? ownComp : -1;
+#pragma unroll
+  for (int m = 32; m > 0; m >>= 1) {
+    rowMinValue = fminf(rowMinValue, __shfl_xor(rowMinValue, m, 64));
+    compLow = min(compLow, __shfl_xor(compLow, m, 64));
+    compHigh = max(compHigh, __shfl_xor(compHigh, m, 64));
+  }
+  if (!Weight::kHasValue)
+    rowMinValue = 0.0f;
   auto capOf = [&](unsigned int bits) { return bits == 0xffffffffu ? INFINITY : floatOf(bits); };
-  if (threadIdx.x == 0) {
-    bound = INFINITY;
-    tileImproved = 0;
-  }
-  const bool rowTilePure = rowBoxes.minComp[rowTile] == rowBoxes.maxComp[rowTile];
-  const int rowCompTile = rowBoxes.minComp[rowTile];
-  const float rowMinValue = rowBoxes.minValue[rowTile];
   const float slack = 1.0f - boxSlack(d);
 
   int rowComp[TR];
@@ -583,73 +602,74 @@ __global__ void __launch_bounds__(256, (KEEP ? 3 : 1))
     stageRows<T>(sm, rowX, nRows, d, row0);
   __syncthreads();
 
-  // The bound: the largest need over the open rows (inf while a row of a
-  // component without a known edge has no candidate yet). Wave 0 only; it
-  // also publishes each row's need.
+  // The wave's bound: the largest need over its open rows (inf while a row of
+  // a component without a known edge has no candidate yet, -1 without open
+  // rows). Publishes each row's need.
   auto newBound = [&]() {
-    float need = 0.0f;
-    if (open0) {
+    float need = -1.0f;
+    if (open) {
       const unsigned long long k =
-          KEEP ? rowTop[threadIdx.x * kKeptKeys + kKeptKeys - 1] : rowBest[threadIdx.x];
+          KEEP ? rowTop[own * kKeptKeys + kKeptKeys - 1] : rowBest[own];
       const float w = k == kEmptyKey ? INFINITY : keyWeight(k);
-      if (compBest && w < cap0) {
-        atomicMin(&compBest[comp0], bitsOf(w));
-        cap0 = w;
+      if (compBest && w < cap) {
+        atomicMin(&compBest[ownComp], bitsOf(w));
+        cap = w;
       }
-      need = fminf(w, cap0);
-      rowNeed[threadIdx.x] = need;
-    }
-    if (open1) {
-      const unsigned long long k = KEEP ? rowTop[(threadIdx.x + 64) * kKeptKeys + kKeptKeys - 1]
-                                        : rowBest[threadIdx.x + 64];
-      const float w = k == kEmptyKey ? INFINITY : keyWeight(k);
-      if (compBest && w < cap1) {
-        atomicMin(&compBest[comp1], bitsOf(w));
-        cap1 = w;
-      }
-      const float need1 = fminf(w, cap1);
-      rowNeed[threadIdx.x + 64] = need1;
-      need = fmaxf(need, need1);
+      need = fminf(w, cap);
+      rowNeed[own] = need;
     }
 #pragma unroll
-    for (int m = 32; m > 0; m >>= 1)
+    for (int m = kWaveRows / 2; m > 0; m >>= 1)
       need = fmaxf(need, __shfl_xor(need, m, 64));
-    return need;
+    if (lane == 0)
+      bound[wave] = need;
+    return __shfl(need, 0, 64);
   };
 
   const int steps = 2 * numTiles;
   for (int base = 0; base < steps; base += kBatch) {
-    if (threadIdx.x < kBatch) {
-      if (compBest) {
-        // Other workgroups may have found better edges for these components.
-        if (open0)
-          cap0 = fminf(cap0, capOf(compBest[comp0]));
-        if (open1)
-          cap1 = fminf(cap1, capOf(compBest[comp1]));
-        const float b = newBound();
-        if (threadIdx.x == 0)
-          bound = b;
-      }
-      // -1: never computed (outside the grid, or both tiles wholly one component).
-      const int step = base + (int)threadIdx.x;
+    // Other workgroups may have found better edges for these components.
+    if (compBest && open)
+      cap = fminf(cap, capOf(compBest[ownComp]));
+    const float reach = newBound();
+    {
+      // -1: never computed (outside the grid, or both sides wholly one component).
+      const int step = base + lane;
       const int colTile = step < steps ? walkTile(center, step, numTiles) : -1;
       float lb = -1.0f;
-      if (colTile >= 0 &&
-          !(rowTilePure && boxes.minComp[colTile] == boxes.maxComp[colTile] &&
-            boxes.minComp[colTile] == rowCompTile)) {
+      if (colTile >= 0 && !(compLow == compHigh && boxes.minComp[colTile] == compLow &&
+                            boxes.maxComp[colTile] == compLow)) {
         const float db = boxLowerBound(metric, rowBox, rowBox + d, boxes.low + (size_t)colTile * d,
                                        boxes.high + (size_t)colTile * d, d);
         lb = weight(db, rowMinValue, boxes.minValue[colTile]) * slack;
       }
-      lowerBound[threadIdx.x] = lb;
+      lowerBound[wave][lane] = lb;
+      const unsigned long long mask = __ballot(lb >= 0.0f && !(lb > reach));
+      if (lane == 0)
+        within[wave] = mask;
     }
     __syncthreads();
-    for (int j = 0; j < kBatch; ++j) {
-      const float lb = lowerBound[j];
-      if (lb < 0.0f || lb > bound)
-        continue; // uniform: lowerBound and bound are shared
+    unsigned long long todo = 0;
+#pragma unroll
+    for (int w = 0; w < kWaves; ++w)
+      todo |= within[w];
+    for (; todo; todo &= todo - 1) {
+      const int j = __ffsll((long long)todo) - 1;
+      // Uniform: written before the barrier after the last computed tile.
+      bool active = false;
+      int activeWaves = 0;
+#pragma unroll
+      for (int w = 0; w < kWaves; ++w) {
+        const float lb = lowerBound[w][j];
+        const bool in = lb >= 0.0f && !(lb > bound[w]);
+        activeWaves += in;
+        if (w == wave)
+          active = in;
+      }
+      if (activeWaves == 0)
+        continue;
       const int colTile = walkTile(center, base + j, numTiles);
-      ++computed;
+      computed += activeWaves;
       if (base + j >= computeSteps)
         continue; // estimate: counted against the bound reached so far, not computed
       const int col0 = colTile * T::DIM;
@@ -658,52 +678,57 @@ __global__ void __launch_bounds__(256, (KEEP ? 3 : 1))
       // computeTile's barriers; rewritten only after this tile's last barrier).
       const ColumnStage<Weight> stage{comp, orig, weight, col0, n, T::DIM,
                                       sColComp, sColVal, sColIdx};
-      computeTile<T, Metric, !kFilter, kRowsResident>(sm, rowX, nRows, X, n, d, metric, row0,
-                                                      col0, w, stage);
-      int colComp[TR];
-      typename Weight::Value colVal[TR];
-      unsigned int colIdx[TR];
+      computeTile<T, Metric, !kFilter, kRowsResident, true>(sm, rowX, nRows, X, n, d, metric,
+                                                            row0, col0, w, stage, active);
+      if (active) {
+        bool improved = false; // a row's best (or list) of this wave
+        int colComp[TR];
+        typename Weight::Value colVal[TR];
+        unsigned int colIdx[TR];
 #pragma unroll
-      for (int c = 0; c < TR; ++c) {
-        const int i = T::colInTile(c);
-        colComp[c] = sColComp[i];
-        colVal[c] = sColVal[i];
-        colIdx[c] = sColIdx[i];
-      }
-      if constexpr (KEEP) {
-        const int lane = threadIdx.x & 63;
-        const unsigned long long groupMask = 0xffffull << (lane & 48);
+        for (int c = 0; c < TR; ++c) {
+          const int i = T::colInTile(c);
+          colComp[c] = sColComp[i];
+          colVal[c] = sColVal[i];
+          colIdx[c] = sColIdx[i];
+        }
+        if constexpr (KEEP) {
+          const unsigned long long groupMask = 0xffffull << (lane & 48);
 #pragma unroll
-        for (int r = 0; r < TR; ++r) {
-          const int i = T::rowInTile(r);
-          unsigned long long *top = rowTop + i * kKeptKeys;
-          // Pairs that can enter the row's list (a stale last key only adds
-          // pairs that the insertion then rejects).
-          const float need = rowNeed[i];
-          const float limit = need < 0.0f ? -INFINITY
-                              : kFilter   ? metric.accBound(weight.distBound(need))
-                                          : INFINITY;
-          const unsigned long long last = top[kKeptKeys - 1];
-          unsigned int pending = 0;
+          for (int r = 0; r < TR; ++r) {
+            int i = T::rowInTile(r);
+            asm volatile("" : "+v"(i)); // computed here, not kept for every row
+            unsigned long long *top = rowTop + i * kKeptKeys;
+            // Pairs that can enter the row's list.
+            const float need = rowNeed[i];
+            const float limit = need < 0.0f ? -INFINITY
+                                : kFilter   ? metric.accBound(weight.distBound(need))
+                                            : INFINITY;
+            const unsigned long long last = top[kKeptKeys - 1];
+            unsigned int pending = 0;
 #pragma unroll
-          for (int c = 0; c < TR; ++c) {
-            const float acc = w[r][c];
-            if (!(acc > limit) && colComp[c] != rowComp[r] && rowComp[r] >= 0 && colComp[c] >= 0) {
-              const float ww = weight(kFilter ? metric.finish(acc) : acc, rowVal[r], colVal[c]);
-              w[r][c] = ww;
-              if (ww != INFINITY && packKey(ww, colIdx[c]) < last)
-                pending |= 1u << c;
+            for (int c = 0; c < TR; ++c) {
+              const float acc = w[r][c];
+              if (!(acc > limit) && colComp[c] != rowComp[r] && rowComp[r] >= 0 &&
+                  colComp[c] >= 0) {
+                const float ww = weight(kFilter ? metric.finish(acc) : acc, rowVal[r], colVal[c]);
+                w[r][c] = ww;
+                if (ww != INFINITY && packKey(ww, colIdx[c]) < last)
+                  pending |= 1u << c;
+              }
             }
-          }
-          // One insertion per row group at a time; the lanes stay converged.
-          while (true) {
-            const unsigned long long work = __ballot(pending != 0);
-            if (work == 0)
-              break;
-            const unsigned long long mine = work & groupMask;
-            if (mine != 0 && lane == __ffsll((long long)mine) - 1) {
+            // One insertion per row group at a time; the lanes stay converged.
+            // The row's lowest lane with work gives its key, and its 16 lanes
+            // insert it: entry q takes the larger of the key and its
+            // predecessor where it is above the key.
+            while (true) {
+              const unsigned long long work = __ballot(pending != 0);
+              if (work == 0)
+                break;
+              improved = true;
+              const unsigned long long mine = work & groupMask;
+              const int source = mine ? __ffsll((long long)mine) - 1 : lane;
               const int c = __ffs(pending) - 1;
-              pending &= pending - 1;
               float wv = 0.0f;
               unsigned int idx = 0;
 #pragma unroll
@@ -712,78 +737,76 @@ __global__ void __launch_bounds__(256, (KEEP ? 3 : 1))
                   wv = w[r][cc];
                   idx = colIdx[cc];
                 }
-              unsigned long long key = packKey(wv, idx);
-              if (key < top[kKeptKeys - 1]) {
-#pragma unroll
-                for (int q = 0; q < kKeptKeys; ++q) {
-                  const unsigned long long cur = top[q];
-                  top[q] = key < cur ? key : cur;
-                  key = key < cur ? cur : key;
-                }
-                tileImproved = 1;
+              if (lane == source)
+                pending &= pending - 1;
+              const unsigned long long key =
+                  packKey(__shfl(wv, source, 64), (unsigned int)__shfl((int)idx, source, 64));
+              const int q = lane & 15;
+              if (mine && q < kKeptKeys) {
+                const unsigned long long cur = top[q], prev = q > 0 ? top[q - 1] : 0;
+                if (cur > key)
+                  top[q] = prev > key ? prev : key;
               }
-            }
-            __builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront");
-            __builtin_amdgcn_wave_barrier();
-            __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "wavefront");
-          }
-        }
-      } else {
+              __builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront");
+              __builtin_amdgcn_wave_barrier();
+              __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "wavefront");
+              if (pending) {
+                const unsigned long long now = top[kKeptKeys - 1];
 #pragma unroll
-      for (int r = 0; r < TR; ++r) {
-        unsigned long long best = kEmptyKey;
-        if constexpr (kFilter) {
-          // rowNeed was published before this tile's barriers.
-          const float need = rowNeed[T::rowInTile(r)];
-          const float limit = need < 0.0f ? -INFINITY : metric.accBound(weight.distBound(need));
-#pragma unroll
-          for (int c = 0; c < TR; ++c) {
-            const float acc = w[r][c];
-            if (!(acc > limit) && colComp[c] != rowComp[r]) {
-              const float ww = weight(metric.finish(acc), rowVal[r], colVal[c]);
-              if (rowComp[r] >= 0 && colComp[c] >= 0 && ww != INFINITY)
-                best = minKey(best, packKey(ww, colIdx[c]));
+                for (int cc = 0; cc < TR; ++cc)
+                  if (!(packKey(w[r][cc], colIdx[cc]) < now))
+                    pending &= ~(1u << cc);
+              }
             }
           }
         } else {
 #pragma unroll
-          for (int c = 0; c < TR; ++c) {
-            const float ww = weight(w[r][c], rowVal[r], colVal[c]);
-            const bool counts = rowComp[r] >= 0 && colComp[c] >= 0 &&
-                                colComp[c] != rowComp[r] && ww != INFINITY;
-            if (counts)
-              best = minKey(best, packKey(ww, colIdx[c]));
-          }
-        }
-        // Wave-uniform: most rows of most tiles have no candidate.
-        if (__ballot(best != kEmptyKey) != 0) {
-          best = rowGroupMin(best);
-          if (T::tc() == 0 && best != kEmptyKey) {
-            const int i = T::rowInTile(r);
-            if (best < rowBest[i]) {
-              rowBest[i] = best;
-              tileImproved = 1;
+          for (int r = 0; r < TR; ++r) {
+            unsigned long long best = kEmptyKey;
+            if constexpr (kFilter) {
+              const float need = rowNeed[T::rowInTile(r)];
+              const float limit = need < 0.0f ? -INFINITY : metric.accBound(weight.distBound(need));
+#pragma unroll
+              for (int c = 0; c < TR; ++c) {
+                const float acc = w[r][c];
+                if (!(acc > limit) && colComp[c] != rowComp[r]) {
+                  const float ww = weight(metric.finish(acc), rowVal[r], colVal[c]);
+                  if (rowComp[r] >= 0 && colComp[c] >= 0 && ww != INFINITY)
+                    best = minKey(best, packKey(ww, colIdx[c]));
+                }
+              }
+            } else {
+#pragma unroll
+              for (int c = 0; c < TR; ++c) {
+                const float ww = weight(w[r][c], rowVal[r], colVal[c]);
+                const bool counts = rowComp[r] >= 0 && colComp[c] >= 0 &&
+                                    colComp[c] != rowComp[r] && ww != INFINITY;
+                if (counts)
+                  best = minKey(best, packKey(ww, colIdx[c]));
+              }
+            }
+            // Wave-uniform: most rows of most tiles have no candidate.
+            if (__ballot(best != kEmptyKey) != 0) {
+              best = rowGroupMin(best);
+              if (T::tc() == 0 && best != kEmptyKey) {
+                const int i = T::rowInTile(r);
+                if (best < rowBest[i]) {
+                  rowBest[i] = best;
+                  improved = true;
+                }
+              }
             }
           }
         }
-      }
-      }
-      __syncthreads();
-      // The needs and the bound change only with a row's best: a tile that
-      // improved none skips the update and its barrier. Every wave reads the
-      // flag after the barrier above; it is cleared only after the barrier
-      // below (all reads done) and set again only after the next tile's
-      // first barrier, so every wave takes the same branch.
-      if (tileImproved) {
-        if (threadIdx.x < 64) {
-          const float b = newBound();
-          if (threadIdx.x == 0)
-            bound = b;
+        // The needs and the bound change only with a row's best.
+        if (__ballot(improved) != 0) {
+          __builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront");
+          __builtin_amdgcn_wave_barrier();
+          __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "wavefront");
+          (void)newBound();
         }
-        __syncthreads();
-        if (threadIdx.x == 0)
-          tileImproved = 0;
       }
+      __syncthreads(); // the tile is consumed, the waves' bounds are current
     }
     __syncthreads(); // lowerBound is rewritten by the next batch
   }
@@ -799,8 +822,8 @@ __global__ void __launch_bounds__(256, (KEEP ? 3 : 1))
   for (int i = threadIdx.x; i < T::DIM; i += T::THREADS)
     if (row0 + i < nRows && rowBest[i] != kEmptyKey)
       atomicMin(&nearest[posOf(row0 + i)], rowBest[i]);
-  if (tilesComputed && threadIdx.x == 0)
-    atomicAdd(tilesComputed, computed);
+  if (wavesComputed && threadIdx.x == 0)
+    atomicAdd(wavesComputed, computed);
 }
 
 // Seeds each component's best known edge weight for the next pass from the
@@ -980,6 +1003,11 @@ struct DeviceBoxes {
 // overestimate of the pruned share: the bound would keep shrinking).
 constexpr int kEstimateSteps = 64;
 
+// Dynamic LDS of the walk: a row box per wave.
+template <class T> size_t walkBoxBytes(int d) {
+  return (size_t)(T::THREADS / 64) * 2 * d * sizeof(float);
+}
+
 template <class T, class Metric, class Weight>
 int runWalk(const float *X, int n, int d, const Metric &metric, const Weight &weight,
             const int *comp, const int *orig, unsigned int *compBest,
@@ -996,7 +1024,7 @@ int runWalk(const float *X, int n, int d, const Metric &metric, const Weight &we
     return s.code;
   s(fill(counter, 0, sizeof(unsigned long long)));
   hipLaunchKernelGGL((buildBoxesKernel<Weight>), dim3(tiles), dim3(64), 0, stream(), X, n, d,
-                     T::DIM, weight, comp, nullptr, boxes.view);
+                     T::DIM, weight, comp, boxes.view);
   s((int)hipGetLastError());
   const int sampled = (tiles + stride - 1) / stride;
   {
@@ -1005,7 +1033,7 @@ int runWalk(const float *X, int n, int d, const Metric &metric, const Weight &we
     if constexpr (Weight::kHasValue) {
       if (kept) {
         hipLaunchKernelGGL((nearestOtherWalkKernel<T, Metric, Weight, false, true>),
-                           dim3(sampled), dim3(256), 2 * d * sizeof(float), stream(), X, n, d,
+                           dim3(sampled), dim3(256), walkBoxBytes<T>(d), stream(), X, n, d,
                            metric, weight, comp, orig, boxes.view, nullptr, nearest,
                            counter.get(), stride, stride > 1 ? kEstimateSteps : 0x7fffffff,
                            skipComp, closedRows, RowSet{}, kept);
@@ -1014,7 +1042,7 @@ int runWalk(const float *X, int n, int d, const Metric &metric, const Weight &we
     }
     if (!launched)
       hipLaunchKernelGGL((nearestOtherWalkKernel<T, Metric, Weight>), dim3(sampled), dim3(256),
-                         2 * d * sizeof(float), stream(), X, n, d, metric, weight, comp, orig,
+                         walkBoxBytes<T>(d), stream(), X, n, d, metric, weight, comp, orig,
                          boxes.view, compBest, nearest, counter.get(), stride,
                          stride > 1 ? kEstimateSteps : 0x7fffffff, skipComp, closedRows,
                          RowSet{}, nullptr);
@@ -1022,11 +1050,13 @@ int runWalk(const float *X, int n, int d, const Metric &metric, const Weight &we
   }
   unsigned long long computed = 0;
   s(download(&computed, counter, sizeof(computed)));
+  // The kernel counts quarter tiles (a wave's rows).
+  constexpr int kWaves = T::THREADS / 64;
   const unsigned long long total = (unsigned long long)sampled * tiles;
-  *share = total ? (double)computed / (double)total : 1.0;
-  addUnits(kPhaseDistanceTiles, (long long)computed * T::DIM * T::DIM);
+  *share = total ? (double)computed / (double)(total * kWaves) : 1.0;
+  addUnits(kPhaseDistanceTiles, (long long)computed * T::WAVE_ROWS * T::DIM);
   if (stats && s.ok()) {
-    stats->tilesComputed += computed;
+    stats->tilesComputed += (computed + kWaves - 1) / kWaves;
     stats->tilesTotal += total;
   }
   return s.code;
@@ -1095,12 +1125,11 @@ int runWalkOpen(const float *X, int n, int d, const Metric &metric, const Weight
   hipLaunchKernelGGL(openRowListKernel, dim3(blocks), dim3(256), 0, stream(), flags.get(),
                      index.get(), n, rowPos.get());
   const int rowTiles = (nOpen + T::DIM - 1) / T::DIM;
-  DeviceBoxes colBoxes, rowBoxes;
+  DeviceBoxes colBoxes;
   DevArray<float> rowX;
   DevArray<int> center;
   DevArray<unsigned long long> counter;
   s(colBoxes.alloc(tiles, d));
-  s(rowBoxes.alloc(rowTiles, d));
   s(rowX.alloc((size_t)nOpen * d));
   s(center.alloc(rowTiles));
   s(counter.alloc(1));
@@ -1109,9 +1138,7 @@ int runWalkOpen(const float *X, int n, int d, const Metric &metric, const Weight
   s(fill(counter, 0, sizeof(unsigned long long)));
   s(gatherRows(X, rowPos, nOpen, d, rowX));
   hipLaunchKernelGGL((buildBoxesKernel<Weight>), dim3(tiles), dim3(64), 0, stream(), X, n, d,
-                     T::DIM, weight, comp, nullptr, colBoxes.view);
-  hipLaunchKernelGGL((buildBoxesKernel<Weight>), dim3(rowTiles), dim3(64), 0, stream(),
-                     rowX.get(), nOpen, d, T::DIM, weight, comp, rowPos.get(), rowBoxes.view);
+                     T::DIM, weight, comp, colBoxes.view);
   hipLaunchKernelGGL(rowTileCentersKernel, dim3((rowTiles + 255) / 256), dim3(256), 0, stream(),
                      rowPos.get(), nOpen, T::DIM, rowTiles, center.get());
   s((int)hipGetLastError());
@@ -1119,12 +1146,11 @@ int runWalkOpen(const float *X, int n, int d, const Metric &metric, const Weight
   rows.X = rowX;
   rows.n = nOpen;
   rows.pos = rowPos;
-  rows.boxes = rowBoxes.view;
   rows.center = center;
   {
     PhaseTimer timer(kPhaseDistanceTiles);
     hipLaunchKernelGGL((nearestOtherWalkKernel<T, Metric, Weight, true>), dim3(rowTiles),
-                       dim3(256), 2 * d * sizeof(float), stream(), X, n, d, metric, weight, comp,
+                       dim3(256), walkBoxBytes<T>(d), stream(), X, n, d, metric, weight, comp,
                        orig, colBoxes.view, compBest, nearest, counter.get(), 1, 0x7fffffff,
                        skipComp, closedRows, rows, nullptr);
     s((int)hipGetLastError());
@@ -1132,10 +1158,11 @@ int runWalkOpen(const float *X, int n, int d, const Metric &metric, const Weight
   unsigned long long computed = 0;
   s(download(&computed, counter, sizeof(computed)));
   const unsigned long long total = (unsigned long long)tiles * tiles;
-  *share = (double)computed / (double)total;
-  addUnits(kPhaseDistanceTiles, (long long)computed * T::DIM * T::DIM);
+  constexpr int kWaves = T::THREADS / 64; // the kernel counts quarter tiles
+  *share = (double)computed / (double)(total * kWaves);
+  addUnits(kPhaseDistanceTiles, (long long)computed * T::WAVE_ROWS * T::DIM);
   if (stats && s.ok()) {
-    stats->tilesComputed += computed;
+    stats->tilesComputed += (computed + kWaves - 1) / kWaves;
     stats->tilesTotal += total;
   }
   return s.code;

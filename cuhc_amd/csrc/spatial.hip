@@ -1,16 +1,16 @@
 // The spatial order of the pruned passes, on the device: each range of points
 // is split at a tile boundary near its middle along its widest feature, until
-// each range is one tile (the behaviour of reference src/spatial.cuh:48-91,
-// which does it on the host). Ties between equal weights always break by
-// original index, so results do not depend on the order; it only decides how
-// much a pass can skip.
+// each range is one tile, and tiles into their waves' 32 rows (down to the tile
+// the behaviour of reference src/spatial.cuh:48-91, which does it on the host).
+// Ties between equal weights always break by original index, so results do
+// not depend on the order; it only decides how much a pass can skip.
 //
 // One level at a time, every range of the level together: a wave per range
 // finds the widest feature of a sample, every point's key is (range, value of
-// that feature quantised to 16 bits (fewer above 8 million points) over the sample's spread), and one stable
-// radix sort of the keys splits all ranges at their middles. A range is named
-// by its path (a bit per level), which orders ranges as they lie and needs no
-// more bits than there are levels.
+// that feature quantised to 16 bits over the sample's spread; fewer bits above
+// a million points), and one stable radix sort of the keys splits all ranges at
+// their middles. A range is named by its path (a bit per level), which orders
+// ranges as they lie and needs no more bits than there are levels.
 // Bound by launches up to some 10^5 points, then by the sorts' passes. With the
 // order made on the host (16 threads; points on the device were copied there
 // first) whole calls took: single linkage, manhattan, 50,021 x 10, 18.9 ms, now
@@ -28,16 +28,26 @@ namespace cuhc {
 namespace {
 
 constexpr int kTilePoints = 128;
+constexpr int kUnitPoints = 32; // a wave's rows of a tile: the finest ranges
+constexpr int kTileUnits = kTilePoints / kUnitPoints;
 constexpr int kSample = 64;      // sampled points per range: one per lane
 constexpr int kMaxValueBits = 16;
 
-// Tiles [lo, hi) of a range of the level, from its path; the range of a path
-// that takes the right half of a single tile is empty.
-DEV void rangeOfPath(unsigned int path, int level, int tiles, int &lo, int &hi) {
+// Where the units [lo, hi) split: between tiles while there is more than one,
+// then between units; a single unit has an empty right half.
+DEV int middleOf(int lo, int hi) {
+  const int units = hi - lo;
+  if (units > kTileUnits)
+    return lo + (units + kTileUnits - 1) / kTileUnits / 2 * kTileUnits;
+  return units > 1 ? lo + (units + 1) / 2 : hi;
+}
+
+// Units [lo, hi) of a range of the level, from its path.
+DEV void rangeOfPath(unsigned int path, int level, int units, int &lo, int &hi) {
   lo = 0;
-  hi = tiles;
+  hi = units;
   for (int l = level - 1; l >= 0; --l) {
-    const int mid = hi - lo > 1 ? lo + (hi - lo) / 2 : hi;
+    const int mid = middleOf(lo, hi);
     if (path >> l & 1)
       lo = mid;
     else
@@ -45,12 +55,12 @@ DEV void rangeOfPath(unsigned int path, int level, int tiles, int &lo, int &hi) 
   }
 }
 
-DEV unsigned int pathOfTile(int tile, int level, int tiles) {
-  int lo = 0, hi = tiles;
+DEV unsigned int pathOfUnit(int unit, int level, int units) {
+  int lo = 0, hi = units;
   unsigned int path = 0;
   for (int l = 0; l < level; ++l) {
-    const int mid = hi - lo > 1 ? lo + (hi - lo) / 2 : hi;
-    const bool right = tile >= mid;
+    const int mid = middleOf(lo, hi);
+    const bool right = unit >= mid;
     path = path << 1 | (right ? 1u : 0u);
     if (right)
       lo = mid;
@@ -62,17 +72,17 @@ DEV unsigned int pathOfTile(int tile, int level, int tiles) {
 
 struct Split {
   int feature;
-  float low, scale; // quantised value = (v - low) scale; scale 0: a single tile
+  float low, scale; // quantised value = (v - low) scale; scale 0: a single unit
 };
 
 __global__ void __launch_bounds__(64)
     splitsKernel(const float *__restrict__ X, int d, const int *__restrict__ order, int count,
-                 int level, int tiles, int valueBits, Split *__restrict__ splits) {
+                 int level, int units, int valueBits, Split *__restrict__ splits) {
   int lo, hi;
-  rangeOfPath(blockIdx.x, level, tiles, lo, hi);
+  rangeOfPath(blockIdx.x, level, units, lo, hi);
   Split best{0, 0.0f, 0.0f};
   if (hi - lo > 1) {
-    const int begin = lo * kTilePoints, end = min(count, hi * kTilePoints);
+    const int begin = lo * kUnitPoints, end = min(count, hi * kUnitPoints);
     const long long at = begin + (long long)(end - begin) * threadIdx.x / kSample;
     const float *row = X + (size_t)order[at] * d;
     float widest = -1.0f;
@@ -96,12 +106,12 @@ __global__ void __launch_bounds__(64)
 }
 
 __global__ void keysKernel(const float *__restrict__ X, int d, const int *__restrict__ order,
-                           int count, int level, int tiles, int valueBits,
+                           int count, int level, int units, int valueBits,
                            const Split *__restrict__ splits, unsigned int *__restrict__ keys) {
   const int p = blockIdx.x * blockDim.x + threadIdx.x;
   if (p >= count)
     return;
-  const unsigned int path = pathOfTile(p / kTilePoints, level, tiles);
+  const unsigned int path = pathOfUnit(p / kUnitPoints, level, units);
   const Split s = splits[path];
   unsigned int q = 0;
   if (s.scale > 0.0f) {
@@ -162,10 +172,13 @@ inline dim3 gridFor(long long count) { return dim3((unsigned)((count + 255) / 25
 
 int spatialOrder(const float *X, int d, const int *list, int count, int *order) {
   hipLaunchKernelGGL(startKernel, gridFor(count), dim3(256), 0, stream(), list, count, order);
+  const int units = (count + kUnitPoints - 1) / kUnitPoints;
   const int tiles = (count + kTilePoints - 1) / kTilePoints;
   int levels = 0;
   while ((1LL << levels) < tiles)
     ++levels;
+  for (int u = std::min(units, kTileUnits); u > 1; u = (u + 1) / 2)
+    ++levels; // inside the tiles
   // Paths and values share 32 bits (2^24 tiles are 2^31 points).
   const int valueBits = std::min(kMaxValueBits, 32 - levels);
   Status s;
@@ -181,9 +194,9 @@ int spatialOrder(const float *X, int d, const int *list, int count, int *order) 
   int *from = order, *to = other.get();
   for (int level = 0; level < levels && s.ok(); ++level) {
     hipLaunchKernelGGL(splitsKernel, dim3(1u << level), dim3(64), 0, stream(), X, d, from, count,
-                       level, tiles, valueBits, splits.get());
+                       level, units, valueBits, splits.get());
     hipLaunchKernelGGL(keysKernel, gridFor(count), dim3(256), 0, stream(), X, d, from, count,
-                       level, tiles, valueBits, splits.get(), keys.get());
+                       level, units, valueBits, splits.get(), keys.get());
     s((int)hipGetLastError());
     s(radixSortPairs(keys.get(), keysOut.get(), from, to, count, level + valueBits, temp));
     std::swap(from, to);

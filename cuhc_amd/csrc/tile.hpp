@@ -2,10 +2,12 @@
 //
 // A workgroup of 256 threads (4 waves) owns a DIM x DIM tile of the distance
 // matrix, DIM = 16 * TR. Thread t = (tr, tc) = (t / 16, t % 16) owns TR x TR
-// outputs: tile rows (r / 4) * 64 + 4 tr + r % 4 and the same pattern for
-// columns. The 16 threads of one tile row are 16 consecutive lanes of one wave,
-// so row reductions are xor-shuffles inside a 16-lane group, and the 4 threads
-// of a wave that share a column tc are lanes tc, tc+16, tc+32, tc+48.
+// outputs: columns (c / 4) * 64 + 4 tc + c % 4, and of the 4 TR consecutive
+// rows of its wave the rows (r / 4) * 16 + 4 (tr % 4) + r % 4, so that a wave
+// can leave out a tile that none of its rows needs. The 16 threads of one tile
+// row are 16 consecutive lanes of one wave, so row reductions are xor-shuffles
+// inside a 16-lane group, and the 4 threads of a wave that share a column tc
+// are lanes tc, tc+16, tc+32, tc+48.
 //
 // Features are staged in LDS transposed (feature-major, rows padded to DIM + 4
 // floats so the transposed stores spread over the banks) FILL features at a
@@ -30,7 +32,10 @@ template <int TR_, int FILL_> struct Tile {
 
   DEV static int tr() { return threadIdx.x >> 4; }
   DEV static int tc() { return threadIdx.x & 15; }
-  DEV static int rowInTile(int r) { return (r >> 2) * 64 + 4 * tr() + (r & 3); }
+  static constexpr int WAVE_ROWS = 4 * TR; // consecutive rows of a wave
+  DEV static int rowInTile(int r) {
+    return WAVE_ROWS * (tr() >> 2) + (r >> 2) * 16 + 4 * (tr() & 3) + (r & 3);
+  }
   DEV static int colInTile(int c) { return (c >> 2) * 64 + 4 * tc() + (c & 3); }
 };
 
@@ -90,12 +95,15 @@ struct NoExtraStage {
 // its barrier: per-tile data the caller stages in LDS shares the fill's
 // memory round trip. With kRowsResident (only for d <= T::FILL: one fill)
 // sm.a already holds the row slice (stageRows) and only the columns are
-// staged.
+// staged. A wave with active false stages its share and leaves its outputs
+// unset. With kFenced the caller has a barrier between its last use of sm (and
+// of extra's data) and every call: the first and last barriers are left out.
 template <class T, class Metric, bool kFinish = true, bool kRowsResident = false,
-          class Extra = NoExtraStage>
+          bool kFenced = false, class Extra = NoExtraStage>
 DEV void computeTile(TileSmem<T> &sm, const float *__restrict__ A, int nA,
                      const float *__restrict__ B, int nB, int d, const Metric &metric, int rowA0,
-                     int colB0, float (&out)[T::TR][T::TR], const Extra &extra = Extra{}) {
+                     int colB0, float (&out)[T::TR][T::TR], const Extra &extra = Extra{},
+                     bool active = true) {
   constexpr int TR = T::TR;
   using Acc = typename Metric::Acc;
   Acc acc[TR][TR];
@@ -105,11 +113,12 @@ DEV void computeTile(TileSmem<T> &sm, const float *__restrict__ A, int nA,
     for (int c = 0; c < TR; ++c)
       acc[r][c] = metric.init();
 
-  const int tr4 = 4 * T::tr(), tc4 = 4 * T::tc();
+  const int row4 = T::rowInTile(0), tc4 = 4 * T::tc();
   for (int f0 = 0; f0 < d; f0 += T::FILL) {
     const int nf = min(T::FILL, d - f0);
     const int nf8 = (nf + 7) & ~7;
-    __syncthreads(); // previous fill fully consumed
+    if (!kFenced || f0 > 0)
+      __syncthreads(); // previous fill fully consumed
     typename Extra::Value ev{};
     if (f0 == 0)
       ev = extra.load();
@@ -119,14 +128,14 @@ DEV void computeTile(TileSmem<T> &sm, const float *__restrict__ A, int nA,
     if (f0 == 0)
       extra.store(ev);
     __syncthreads();
-    for (int k0 = 0; k0 < nf8; k0 += 8) {
+    for (int k0 = 0; k0 < nf8 && active; k0 += 8) {
 #pragma unroll
       for (int kk = 0; kk < 8; ++kk) {
         const int k = k0 + kk;
         float av[TR], bv[TR];
 #pragma unroll
         for (int h = 0; h < TR / 4; ++h) {
-          const float4 a4 = *reinterpret_cast<const float4 *>(&sm.a[k][h * 64 + tr4]);
+          const float4 a4 = *reinterpret_cast<const float4 *>(&sm.a[k][row4 + h * 16]);
           const float4 b4 = *reinterpret_cast<const float4 *>(&sm.b[k][h * 64 + tc4]);
           av[4 * h + 0] = a4.x; av[4 * h + 1] = a4.y; av[4 * h + 2] = a4.z; av[4 * h + 3] = a4.w;
           bv[4 * h + 0] = b4.x; bv[4 * h + 1] = b4.y; bv[4 * h + 2] = b4.z; bv[4 * h + 3] = b4.w;
@@ -139,7 +148,8 @@ DEV void computeTile(TileSmem<T> &sm, const float *__restrict__ A, int nA,
       }
     }
   }
-  __syncthreads(); // LDS free for the caller / next tile
+  if (!kFenced)
+    __syncthreads(); // LDS free for the caller / next tile
 #pragma unroll
   for (int r = 0; r < TR; ++r)
 #pragma unroll
