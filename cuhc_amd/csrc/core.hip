@@ -423,6 +423,8 @@ int coreFused(const float *X, int n, int d, MetricSpec m, int k, float *core, bo
 // fills the chip many times over), at least one row, a multiple of the tile
 // rows when possible, never more than wanted.
 int radixChunkRows(int n, int wanted, int tileRows) {
+  if ((size_t)n * wanted <= ((size_t)64 << 20))
+    return wanted; // 256 MiB at most: not worth asking
   size_t freeBytes = 0, totalBytes = 0;
   if (hipMemGetInfo(&freeBytes, &totalBytes) != hipSuccess) {
     (void)hipGetLastError();

@@ -112,17 +112,12 @@ DEV unsigned long long rowGroupMin(unsigned long long k) {
 
 // Pair filter of the symmetric pass. A point's limit comes from the weight of
 // its current nearest (+inf while it has none; the key's high word, read
-// alone: nearest only decreases, so a stale read is a looser limit). A pair
-// passes when its filter value is within the larger of its two points'
-// limits; every pair whose weight is within a point's nearest weight passes.
-//   metrics with an accumulator bound (plain and mutual-reachability
-//   weights): value = the raw accumulator, limit = accBound(distBound(w));
-//   Ward: 2 si sj / (si + sj) >= min(si, sj), so the weight is at least
-//   sq min(si, sj) up to the rounding of its four operations (2^-22):
-//   value = sq min(si, sj), limit = w (1 + 2^-20) + FLT_MIN.
+// alone: nearest only decreases, so a stale read is a looser limit). With a
+// metric that has an accumulator bound, a pair passes when its raw accumulator
+// is within the larger of its two points' limits, accBound(distBound(w)); every
+// pair whose weight is within a point's nearest weight passes.
 template <class Metric, class Weight> struct PairFilter {
-  static constexpr bool kWard = std::is_same<Weight, WardWeight>::value;
-  static constexpr bool kOn = (Metric::kAccFilter && Weight::kDistBound) || kWard;
+  static constexpr bool kOn = Metric::kAccFilter && Weight::kDistBound;
   DEV static float limit(const Metric &metric, const Weight &weight,
                          const unsigned long long *nearest, int p) {
     return limitOf(metric, weight,
@@ -132,16 +127,7 @@ template <class Metric, class Weight> struct PairFilter {
     if (bits == 0xffffffffu)
       return INFINITY;
     const float w = floatOf(bits);
-    if constexpr (kWard)
-      return w * (1.0f + 0x1p-20f) + FLT_MIN;
-    else
-      return metric.accBound(weight.distBound(w));
-  }
-  DEV static float value(float acc, typename Weight::Value vi, typename Weight::Value vj) {
-    if constexpr (kWard)
-      return acc * fminf(vi, vj);
-    else
-      return acc;
+    return metric.accBound(weight.distBound(w));
   }
 };
 
@@ -269,7 +255,7 @@ __global__ void __launch_bounds__(256, 3) // three waves per SIMD (at most 168 V
 #pragma unroll
         for (int c = 0; c < TR; ++c) {
           const float acc = w[r][c];
-          if (!(Filter::value(acc, rv, colVal[c]) > fmaxf(rowLimit, colLimit[c])) &&
+          if (!(acc > fmaxf(rowLimit, colLimit[c])) &&
               colComp[c] != rc) {
             const float ww = weight(metric.finish(acc), rv, colVal[c]);
             w[r][c] = ww;
@@ -935,19 +921,6 @@ int condensedMatrix(const float *X, int n, int d, MetricSpec m, float *out) {
 int nearestOtherSymmetric(const float *X, int n, int d, MetricSpec m, WeightSpec w,
                           const int *comp, const int *orig, unsigned long long *nearest,
                           const int *numComp) {
-  if (w.kind == kWeightWard) {
-    if (m.id != kSqEuclidean)
-      return kErrInvalidMetric;
-    WardWeight ward{w.size};
-    return withFill(d, [&](auto fill) {
-      using T = Tile<8, decltype(fill)::value>;
-      const long long tiles = (n + T::DIM - 1) / T::DIM, pairs = tiles * (tiles + 1) / 2;
-      hipLaunchKernelGGL((nearestOtherSymmetricKernel<T, SqEuclidean, WardWeight>),
-                         dim3(persistentBlocks(pairs, 8)), dim3(256), 0, stream(), X, n, d,
-                         SqEuclidean{}, ward, comp, orig, nearest, pairs, numComp);
-      return (int)hipGetLastError();
-    });
-  }
   return withMetric(m, [&](auto metric) {
     using Metric = decltype(metric);
     return withWeightFor(metric, w, [&](auto weight) {

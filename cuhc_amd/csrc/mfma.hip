@@ -1313,6 +1313,11 @@ void mixedPassDestroy(MixedPass *mp) {
   delete mp;
 }
 
+const unsigned long long *mixedPassLists(const MixedPass *mp, int *per) {
+  *per = kTopK;
+  return mp->topk.get();
+}
+
 int mixedPassRun(MixedPass *mp, const int *comp, int numComponents, bool sqeuclidean,
                  bool firstRound, unsigned long long *nearest) {
   const int n = mp->n;

@@ -174,5 +174,8 @@ void mixedPassDestroy(MixedPass *mp);
 int mixedPassRun(MixedPass *mp, const int *comp, int numComponents, bool sqeuclidean,
                  bool firstRound, unsigned long long *nearest);
 bool mixedPassSupports(int d);
+// The lowest keys that a first round kept of every point, [n][*per] ascending
+// (device memory of the pass).
+const unsigned long long *mixedPassLists(const MixedPass *mp, int *per);
 
 } // namespace cuhc

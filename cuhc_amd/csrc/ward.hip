@@ -11,121 +11,20 @@
 // pair always sees each other and every round makes progress).
 #include "linkage.hpp"
 #include "mst.hpp"
+#include "primitives.hpp"
+#include "tile.hpp"
 
 #include <hip/hip_cooperative_groups.h>
 
 #include <algorithm>
 #include <numeric>
+#include <type_traits>
 
 namespace cuhc {
 
 namespace {
 
 namespace cg = cooperative_groups;
-
-DEV int reciprocalPartner(const unsigned long long *nearest, int i) {
-  const unsigned long long k = nearest[i];
-  if (k == kEmptyKey)
-    return -1;
-  const int j = keyIndex(k);
-  return keyIndex(nearest[j]) == i && nearest[j] != kEmptyKey ? j : -1;
-}
-
-__global__ void survivorsKernel(const unsigned long long *nearest, int m, int *survives) {
-  const int i = blockIdx.x * blockDim.x + threadIdx.x;
-  if (i >= m)
-    return;
-  const int j = reciprocalPartner(nearest, i);
-  survives[i] = !(j >= 0 && j < i);
-}
-
-// Exclusive scan, three launches: per-block scan of 1024 values, a one-block
-// scan of the block totals, and the offsets added back.
-constexpr int kScanBlock = 1024;
-
-__global__ void __launch_bounds__(kScanBlock) scanBlocksKernel(const int *in, int m, int *out,
-                                                               int *blockTotals) {
-  __shared__ int waveTotals[kScanBlock / 64];
-  const int i = blockIdx.x * kScanBlock + threadIdx.x;
-  const int v = i < m ? in[i] : 0;
-  const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
-  int x = v; // inclusive scan inside the wave
-#pragma unroll
-  for (int off = 1; off < 64; off <<= 1) {
-    const int y = __shfl_up(x, off, 64);
-    if (lane >= off)
-      x += y;
-  }
-  if (lane == 63)
-    waveTotals[wave] = x;
-  __syncthreads();
-  if (wave == 0) {
-    int t = lane < kScanBlock / 64 ? waveTotals[lane] : 0;
-#pragma unroll
-    for (int off = 1; off < 64; off <<= 1) {
-      const int y = __shfl_up(t, off, 64);
-      if (lane >= off)
-        t += y;
-    }
-    if (lane < kScanBlock / 64)
-      waveTotals[lane] = t; // inclusive over waves
-  }
-  __syncthreads();
-  const int before = wave > 0 ? waveTotals[wave - 1] : 0;
-  if (i < m)
-    out[i] = before + x - v;
-  if (threadIdx.x == kScanBlock - 1)
-    blockTotals[blockIdx.x] = before + x;
-}
-
-__global__ void __launch_bounds__(kScanBlock) scanTotalsKernel(int *totals, int numBlocks) {
-  // Sequential over chunks of 1024 (numBlocks is small: m / 1024).
-  __shared__ int carry;
-  __shared__ int waveTotals[kScanBlock / 64];
-  if (threadIdx.x == 0)
-    carry = 0;
-  __syncthreads();
-  for (int base = 0; base < numBlocks; base += kScanBlock) {
-    const int i = base + threadIdx.x;
-    const int v = i < numBlocks ? totals[i] : 0;
-    const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
-    int x = v;
-#pragma unroll
-    for (int off = 1; off < 64; off <<= 1) {
-      const int y = __shfl_up(x, off, 64);
-      if (lane >= off)
-        x += y;
-    }
-    if (lane == 63)
-      waveTotals[wave] = x;
-    __syncthreads();
-    if (wave == 0) {
-      int t = lane < kScanBlock / 64 ? waveTotals[lane] : 0;
-#pragma unroll
-      for (int off = 1; off < 64; off <<= 1) {
-        const int y = __shfl_up(t, off, 64);
-        if (lane >= off)
-          t += y;
-      }
-      if (lane < kScanBlock / 64)
-        waveTotals[lane] = t;
-    }
-    __syncthreads();
-    const int before = (wave > 0 ? waveTotals[wave - 1] : 0) + carry;
-    if (i < numBlocks)
-      totals[i] = before + x - v; // exclusive
-    __syncthreads();
-    if (threadIdx.x == kScanBlock - 1)
-      carry = before + x;
-    __syncthreads();
-  }
-}
-
-__global__ void addOffsetsKernel(int *out, int m, const int *offsets) {
-  const int i = blockIdx.x * kScanBlock + threadIdx.x;
-  if (i < m)
-    out[i] += offsets[blockIdx.x];
-}
 
 struct Clusters {
   double *c64;
@@ -139,45 +38,553 @@ struct DevMerge {
   double h;
 };
 
-// One thread per (slot, feature): surviving slot i goes to newIndex[i]; if it
-// pairs with a higher slot j, the merged centroid goes there and the merge is
-// recorded (heights in FP64).
-__global__ void rnnMergeKernel(Clusters cur, Clusters next, const unsigned long long *nearest,
-                               const int *newIndex, int m, int d, DevMerge *merges,
-                               int *numMerges) {
-  const size_t total = (size_t)m * d;
-  for (size_t e = blockIdx.x * (size_t)blockDim.x + threadIdx.x; e < total;
-       e += (size_t)gridDim.x * blockDim.x) {
-    const int i = (int)(e / d), k = (int)(e - (size_t)i * d);
-    const int j = reciprocalPartner(nearest, i);
-    if (j >= 0 && j < i)
-      continue;
-    const int to = newIndex[i];
-    const double ci = cur.c64[e];
-    double c = ci;
-    if (j >= 0) {
-      const double si = cur.size[i], sj = cur.size[j];
-      c = fma(cur.c64[(size_t)j * d + k] - ci, sj / (si + sj), ci);
-    }
-    next.c64[(size_t)to * d + k] = c;
-    next.c32[(size_t)to * d + k] = (float)c;
-    if (k == 0) {
-      next.size[to] = cur.size[i] + (j >= 0 ? cur.size[j] : 0);
-      next.rep[to] = cur.rep[i];
-      if (j >= 0) {
-        const double *a = cur.c64 + (size_t)i * d, *b = cur.c64 + (size_t)j * d;
-        double sq = 0.0;
-        for (int f = 0; f < d; ++f) {
-          const double diff = a[f] - b[f];
-          sq = fma(diff, diff, sq);
-        }
-        const double si = cur.size[i], sj = cur.size[j];
-        const int u = cur.rep[i], v = cur.rep[j];
-        merges[atomicAdd(numMerges, 1)] =
-            DevMerge{min(u, v), max(u, v), sqrt(2.0 * (si * sj) / (si + sj) * sq)};
-      }
+// ---------------------------------------------------------------------------
+// Rounds of reciprocal nearest neighbours.
+//
+// Every cluster keeps a list of its kList nearest clusters, exactly the lowest
+// keys (FP32 Ward weight, slot), and a bound below every key that is not in the
+// list; its nearest is the list's first. A round merges the reciprocal pairs
+// and compacts the slots in order. The weights between clusters that did not
+// merge do not change, so a list without its merged entries still holds the
+// lowest keys, and only the merged clusters and those whose list ran out search
+// again (a few tenths of the rows against all columns; the lower triangle of
+// all pairs before). A search row that is a new cluster offers its weight to
+// every column whose bound lies above it (pushed[]); the lowest offer enters
+// the column's list, which ends there: what else was offered weighs more. Slots
+// keep their order through a compaction, so keys keep theirs and every
+// nearest, ties included, is the one a pass over all pairs would find.
+//
+// Bound by FP32 VALU work at large m, by launches and dependent waits at small:
+// the component count stays on the device, so that rounds are queued several
+// at a time, each of 5 launches (7 above 4,096 clusters), without a host read.
+// A pass over all pairs per round and its read took 4.3 ms for 3,001 points of
+// 13 features (55 rounds) and 99 ms for 100,000 of 32 (95 rounds); now 2.6 and
+// 61 ms.
+constexpr int kList = 4;       // 8 searches a quarter fewer pairs and takes as long
+constexpr int kRoundsAhead = 8;    // rounds queued per host read
+// Workgroups per CU, and the work items a search is split into: two for each
+// of them on 256 CUs (with 1,024 items a third of the chip waited for the
+// second ones).
+constexpr int kSearchGroups = 3;
+constexpr int kSearchItems = 1536;
+constexpr int kSmallSearch = 16384; // clusters up to which tiles are 64 a side
+
+struct RoundState {
+  int m;        // clusters
+  int merges;   // recorded so far
+  int searches; // rows of the current search
+  int stop;     // a round fell below the wanted progress: queued rounds do nothing
+  int rounds;   // rounds done
+};
+
+struct Lists {
+  unsigned long long *keys;  // [m][kList], ascending, kEmptyKey padded
+  unsigned long long *bound; // [m]
+};
+
+// Column splits of a search and its work items (row tile, split).
+DEV int searchSplits(int rows, int m, int dim) {
+  const int rowTiles = (rows + dim - 1) / dim, colTiles = (m + dim - 1) / dim;
+  return max(1, min(colTiles, kSearchItems / max(1, rowTiles)));
+}
+
+DEV bool roundOver(const RoundState *st) { return st->stop != 0 || st->m <= 1; }
+
+DEV int reciprocalPartner(const unsigned long long *keys, int i) {
+  const unsigned long long k = keys[(size_t)i * kList];
+  if (k == kEmptyKey)
+    return -1;
+  const int j = keyIndex(k);
+  const unsigned long long back = keys[(size_t)j * kList];
+  return back != kEmptyKey && keyIndex(back) == i ? j : -1;
+}
+
+// The end of a round: its place in the merges, the new count, and whether it
+// made enough progress.
+DEV void endRound(RoundState *st, int now, float minProgress, int *roundEnd) {
+  if (roundOver(st))
+    return;
+  const int before = st->m;
+  roundEnd[st->rounds++] = st->merges;
+  st->m = now;
+  if (now > 1 && (now == before || (float)(before - now) < minProgress * (float)before))
+    st->stop = 1;
+}
+
+__global__ void roundEndKernel(RoundState *st, const int *__restrict__ mNow, float minProgress,
+                               int *roundEnd) {
+  endRound(st, *mNow, minProgress, roundEnd);
+}
+
+// partner[i] (-1: none) and survives[i] for i <= mMost (mMost: the most
+// clusters there can be); the scan of survives numbers the next round's slots.
+__global__ void survivorsKernel(Lists lists, RoundState *st, int mMost, int *partner,
+                                int *survives) {
+  const int i = blockIdx.x * blockDim.x + threadIdx.x;
+  if (i > mMost)
+    return;
+  const int m = roundOver(st) ? 0 : st->m;
+  int keep = 0;
+  if (i < m) {
+    const int j = reciprocalPartner(lists.keys, i);
+    partner[i] = j;
+    keep = !(j >= 0 && j < i);
+  }
+  survives[i] = keep;
+  if (i == 0)
+    st->searches = 0;
+}
+
+// The same and its scan by one workgroup, after the end of the round before
+// (first: there is none). newIndex[mMost] receives the survivors.
+constexpr int kSmallThreads = 1024;
+constexpr int kSmallPer = 8;
+constexpr int kSmallClusters = kSmallThreads * kSmallPer;
+
+__global__ void __launch_bounds__(kSmallThreads)
+    smallRoundKernel(Lists lists, RoundState *st, int mMost, bool first, float minProgress,
+                     int *roundEnd, int *partner, int *newIndex) {
+  __shared__ int waveTotal[kSmallThreads / 64];
+  const int t = threadIdx.x, lane = t & 63, wave = t >> 6;
+  if (t == 0 && !first)
+    endRound(st, newIndex[mMost], minProgress, roundEnd);
+  __syncthreads();
+  if (roundOver(st))
+    return;
+  const int m = st->m;
+  const int per = (m + kSmallThreads - 1) / kSmallThreads, i0 = t * per;
+  int keep = 0; // bit q: slot i0 + q survives
+#pragma unroll
+  for (int q = 0; q < kSmallPer; ++q) {
+    const int i = i0 + q;
+    if (q < per && i < m) {
+      const int j = reciprocalPartner(lists.keys, i);
+      partner[i] = j;
+      keep |= !(j >= 0 && j < i) ? 1 << q : 0;
     }
   }
+  int upTo = __popc(keep);
+#pragma unroll
+  for (int d = 1; d < 64; d <<= 1) {
+    const int up = __shfl_up(upTo, d, 64);
+    if (lane >= d)
+      upTo += up;
+  }
+  if (lane == 63)
+    waveTotal[wave] = upTo;
+  __syncthreads();
+  int at = upTo - __popc(keep), total = 0;
+  for (int w = 0; w < kSmallThreads / 64; ++w) {
+    at += w < wave ? waveTotal[w] : 0;
+    total += waveTotal[w];
+  }
+#pragma unroll
+  for (int q = 0; q < kSmallPer; ++q)
+    if (q < per && i0 + q < m) {
+      newIndex[i0 + q] = at;
+      at += keep >> q & 1;
+    }
+  __syncthreads();
+  if (t == 0) {
+    newIndex[mMost] = total; // past every slot
+    st->searches = 0;
+  }
+}
+
+// Surviving slot i goes to newIndex[i]; if it pairs with a higher slot j, the
+// merged centroid goes there and the merge is recorded (heights in FP64). The
+// first slotBlocks workgroups take a slot per thread (sizes, merges, and the
+// slot's list: carried over, or put on the search list as slot with the top bit
+// for a new cluster, searchOf[slot] its place or -1), the others a centroid
+// coordinate per thread.
+__global__ void __launch_bounds__(256)
+    rnnMergeKernel(Clusters cur, Clusters next, Lists from, Lists to,
+                   const int *__restrict__ partner, const int *__restrict__ newIndex, int d,
+                   RoundState *st, DevMerge *merges, unsigned int *searchRows, int *searchOf,
+                   unsigned long long *pushed, int slotBlocks) {
+  if (roundOver(st))
+    return;
+  const int m = st->m;
+  if ((int)blockIdx.x >= slotBlocks) {
+    const size_t total = (size_t)m * d;
+    for (size_t e = ((size_t)blockIdx.x - slotBlocks) * blockDim.x + threadIdx.x; e < total;
+         e += (size_t)(gridDim.x - slotBlocks) * blockDim.x) {
+      const int i = (int)(e / d), k = (int)(e - (size_t)i * d);
+      const int j = partner[i];
+      if (j >= 0 && j < i)
+        continue;
+      const double ci = cur.c64[e];
+      double c = ci;
+      if (j >= 0) {
+        const double si = cur.size[i], sj = cur.size[j];
+        c = fma(cur.c64[(size_t)j * d + k] - ci, sj / (si + sj), ci);
+      }
+      const size_t at = (size_t)newIndex[i] * d + k;
+      next.c64[at] = c;
+      next.c32[at] = (float)c;
+    }
+    return;
+  }
+  const int i = blockIdx.x * blockDim.x + threadIdx.x;
+  if (i >= m)
+    return;
+  const int j = partner[i];
+  if (j >= 0 && j < i)
+    return;
+  const int at = newIndex[i];
+  next.size[at] = cur.size[i] + (j >= 0 ? cur.size[j] : 0);
+  next.rep[at] = cur.rep[i];
+  pushed[at] = kEmptyKey;
+  int left = 0;
+  if (j < 0) {
+    for (int q = 0; q < kList; ++q) {
+      const unsigned long long key = from.keys[(size_t)i * kList + q];
+      if (key == kEmptyKey)
+        break;
+      const int s = keyIndex(key);
+      if (partner[s] < 0)
+        to.keys[(size_t)at * kList + left++] =
+            (key & 0xffffffff00000000ull) | (unsigned int)newIndex[s];
+    }
+    for (int q = left; q < kList; ++q)
+      to.keys[(size_t)at * kList + q] = kEmptyKey;
+    const unsigned long long bound = from.bound[i];
+    to.bound[at] = bound == kEmptyKey ? kEmptyKey
+                                      : (bound & 0xffffffff00000000ull) |
+                                            (unsigned int)newIndex[keyIndex(bound)];
+  }
+  if (left == 0) {
+    const int place = atomicAdd(&st->searches, 1);
+    searchRows[place] = (unsigned int)at | (j >= 0 ? 0x80000000u : 0u);
+    searchOf[at] = place;
+  } else {
+    searchOf[at] = -1;
+  }
+  if (j >= 0) {
+    const double *a = cur.c64 + (size_t)i * d, *b = cur.c64 + (size_t)j * d;
+    double sq = 0.0;
+    for (int f = 0; f < d; ++f) {
+      const double diff = a[f] - b[f];
+      sq = fma(diff, diff, sq);
+    }
+    const double si = cur.size[i], sj = cur.size[j];
+    const int u = cur.rep[i], v = cur.rep[j];
+    merges[atomicAdd(&st->merges, 1)] =
+        DevMerge{min(u, v), max(u, v), sqrt(2.0 * (si * sj) / (si + sj) * sq)};
+  }
+}
+
+// The first round's search: every slot, none of them new.
+__global__ void searchAllKernel(int n, unsigned int *searchRows, int *searchOf,
+                                unsigned long long *pushed, RoundState *st) {
+  const int i = blockIdx.x * blockDim.x + threadIdx.x;
+  if (i < n) {
+    searchRows[i] = (unsigned int)i;
+    searchOf[i] = i;
+    pushed[i] = kEmptyKey;
+  }
+  if (i == 0)
+    st->searches = n;
+}
+
+// Lists from an exact pass that kept `per` lowest keys of every point.
+__global__ void listsFromKeysKernel(const unsigned long long *__restrict__ keys, int per, int n,
+                                    Lists lists) {
+  const int i = blockIdx.x * blockDim.x + threadIdx.x;
+  if (i >= n)
+    return;
+  for (int q = 0; q < kList; ++q)
+    lists.keys[(size_t)i * kList + q] = q < per ? keys[(size_t)i * per + q] : kEmptyKey;
+  lists.bound[i] = keys[(size_t)i * per + per - 1];
+}
+
+// Minimum over the 16 lanes of a tile row, in all of them (DPP row rotations).
+template <int CTRL> DEV unsigned long long rotateMin(unsigned long long v) {
+  const unsigned int lo =
+      (unsigned int)__builtin_amdgcn_update_dpp(-1, (int)(unsigned int)v, CTRL, 0xf, 0xf, false);
+  const unsigned int hi = (unsigned int)__builtin_amdgcn_update_dpp(
+      -1, (int)(unsigned int)(v >> 32), CTRL, 0xf, 0xf, false);
+  return minKey(v, ((unsigned long long)hi << 32) | lo);
+}
+DEV unsigned long long rowMin16(unsigned long long v) {
+  v = rotateMin<0x128>(v); // row_ror:8, 4, 2, 1
+  v = rotateMin<0x124>(v);
+  v = rotateMin<0x122>(v);
+  return rotateMin<0x121>(v);
+}
+
+// The filter of PairFilter (distance.hip) for Ward: 2 si sj / (si + sj) >=
+// min(si, sj), so a pair whose sq min(si, sj) is above the limit of a key's
+// weight weighs more than the key.
+DEV float wardLimit(unsigned long long key) {
+  return key == kEmptyKey ? INFINITY : keyWeight(key) * (1.0f + 0x1p-20f) + FLT_MIN;
+}
+
+// Search rows against all m columns, in work items of a tile of rows and every
+// splits-th column tile (128 points a side; 64 for few clusters: one tile's
+// lists take longer than its distances, and more, smaller items share them). A row's kList lowest keys over an item's columns
+// go to partial[place][split][kList]; a new cluster's weight goes to
+// pushed[column] where it is below the column's bound.
+template <int TR_, int FILL>
+__global__ void __launch_bounds__(256, 3)
+    wardSearchKernel(const float *__restrict__ C, int d, const int *__restrict__ size,
+                     const unsigned int *__restrict__ searchRows, const int *__restrict__ searchOf,
+                     const unsigned long long *__restrict__ bound, const RoundState *st,
+                     const int *__restrict__ mNow, unsigned long long *__restrict__ partial,
+                     unsigned long long *__restrict__ pushed) {
+  using T = Tile<TR_, FILL>;
+  constexpr int TR = T::TR, DIM = T::DIM;
+  __shared__ __align__(16) TileSmem<T> sm;
+  __shared__ unsigned long long top[DIM][kList];
+  __shared__ int rowSlot[DIM];   // -1: no row
+  __shared__ float rowSize[DIM];
+  __shared__ unsigned char rowNew[DIM];
+  __shared__ float colSize[DIM], colLimit[DIM]; // limit -inf: takes no offers
+  __shared__ unsigned int colBits[DIM];
+  if (roundOver(st))
+    return;
+  const int m = *mNow, rows = st->searches;
+  const int rowTiles = (rows + DIM - 1) / DIM, colTiles = (m + DIM - 1) / DIM;
+  const int splits = searchSplits(rows, m, DIM);
+  const SqEuclidean metric;
+  const int tid = threadIdx.x, lane = tid & 63;
+  const unsigned long long groupMask = 0xffffull << (lane & 48);
+  const int row4 = T::rowInTile(0), tc4 = 4 * T::tc();
+  for (int item = blockIdx.x; item < rowTiles * splits; item += gridDim.x) {
+    const int rowTile = item / splits, split = item - rowTile * splits;
+    __syncthreads(); // the last item's LDS is consumed
+    if (tid < DIM) {
+      const int at = rowTile * DIM + tid;
+      const unsigned int entry = at < rows ? searchRows[at] : 0u;
+      const int slot = at < rows ? (int)(entry & 0x7fffffffu) : -1;
+      rowSlot[tid] = slot;
+      rowSize[tid] = slot >= 0 ? (float)size[slot] : 1.0f;
+      rowNew[tid] = entry >> 31;
+    }
+    for (int i = tid; i < DIM * kList; i += T::THREADS)
+      (&top[0][0])[i] = kEmptyKey;
+    __syncthreads();
+    bool first = true;
+    for (int colTile = split; colTile < colTiles; colTile += splits) {
+      const int col0 = colTile * DIM;
+      float acc[TR][TR];
+#pragma unroll
+      for (int r = 0; r < TR; ++r)
+#pragma unroll
+        for (int c = 0; c < TR; ++c)
+          acc[r][c] = 0.0f;
+      for (int f0 = 0; f0 < d; f0 += FILL) {
+        const int nf8 = (min(FILL, d - f0) + 7) & ~7;
+        // Rows of one fill stay in LDS for all of the item's tiles.
+        if (first || d > FILL)
+          for (int idx = tid; idx < DIM * nf8; idx += T::THREADS) {
+            const int p = idx / nf8, k = idx - p * nf8, slot = rowSlot[p];
+            sm.a[k][p] = slot >= 0 && f0 + k < d ? C[(size_t)slot * d + f0 + k] : 0.0f;
+          }
+        stageSlice<T>(sm.b, C, m, d, col0, f0, nf8);
+        if (f0 == 0 && tid < DIM) {
+          const int col = col0 + tid;
+          const bool in = col < m;
+          const unsigned long long b = in && searchOf[col] < 0 ? bound[col] : 0ull;
+          colSize[tid] = in ? (float)size[col] : -1.0f;
+          colLimit[tid] = in && searchOf[col] < 0 ? wardLimit(b) : -INFINITY;
+          colBits[tid] = (unsigned int)(b >> 32);
+        }
+        __syncthreads();
+        for (int k0 = 0; k0 < nf8; k0 += 8) {
+#pragma unroll
+          for (int kk = 0; kk < 8; ++kk) {
+            const int k = k0 + kk;
+            float av[TR], bv[TR];
+#pragma unroll
+            for (int h = 0; h < TR / 4; ++h) {
+              const float4 a4 = *reinterpret_cast<const float4 *>(&sm.a[k][row4 + h * 16]);
+              const float4 b4 = *reinterpret_cast<const float4 *>(&sm.b[k][h * 64 + tc4]);
+              av[4 * h + 0] = a4.x; av[4 * h + 1] = a4.y; av[4 * h + 2] = a4.z; av[4 * h + 3] = a4.w;
+              bv[4 * h + 0] = b4.x; bv[4 * h + 1] = b4.y; bv[4 * h + 2] = b4.z; bv[4 * h + 3] = b4.w;
+            }
+#pragma unroll
+            for (int r = 0; r < TR; ++r)
+#pragma unroll
+              for (int c = 0; c < TR; ++c)
+                acc[r][c] = metric.fold(acc[r][c], av[r], bv[c]);
+          }
+        }
+        if (f0 + FILL < d)
+          __syncthreads(); // the fill is consumed
+      }
+      float cs[TR], cl[TR];
+#pragma unroll
+      for (int c = 0; c < TR; ++c) {
+        cs[c] = colSize[T::colInTile(c)];
+        cl[c] = colLimit[T::colInTile(c)];
+      }
+#pragma unroll
+      for (int r = 0; r < TR; ++r) {
+        int i = T::rowInTile(r);
+        asm volatile("" : "+v"(i)); // computed here, not kept for every row
+        const int slot = rowSlot[i];
+        const float rs = rowSize[i];
+        unsigned long long *list = top[i];
+        const unsigned long long last = list[kList - 1];
+        const float limit = slot < 0 ? -INFINITY : wardLimit(last);
+        const bool offers = rowNew[i];
+        unsigned int pending = 0;
+#pragma unroll
+        for (int c = 0; c < TR; ++c) {
+          const int col = col0 + T::colInTile(c);
+          const float least = acc[r][c] * fminf(rs, cs[c]);
+          if (!(least > fmaxf(limit, cl[c])) && cs[c] >= 0.0f && slot >= 0 && col != slot) {
+            const bool forRow = !(least > limit), forCol = offers && !(least > cl[c]);
+            const float w = (2.0f * (rs * cs[c])) / (rs + cs[c]) * acc[r][c];
+            acc[r][c] = w;
+            if (w != INFINITY) {
+              if (forRow && packKey(w, (unsigned)col) < last)
+                pending |= 1u << c;
+              if (forCol && bitsOf(w) <= colBits[T::colInTile(c)])
+                atomicMin(&pushed[col], packKey(w, (unsigned)slot));
+            }
+          }
+        }
+        if (first) {
+          // Empty lists: the row's kList lowest, one after the other, from the
+          // lowest of every lane.
+#pragma unroll 1
+          for (int q = 0; q < kList && __ballot(pending != 0) != 0; ++q) {
+            unsigned long long mineLow = kEmptyKey;
+#pragma unroll
+            for (int c = 0; c < TR; ++c)
+              if (pending >> c & 1)
+                mineLow = minKey(mineLow, packKey(acc[r][c], (unsigned)(col0 + T::colInTile(c))));
+            const unsigned long long low = rowMin16(mineLow);
+            if (low == mineLow && low != kEmptyKey) {
+#pragma unroll
+              for (int c = 0; c < TR; ++c)
+                if (col0 + T::colInTile(c) == keyIndex(low))
+                  pending &= ~(1u << c);
+            }
+            if (T::tc() == 0)
+              list[q] = low;
+          }
+        } else {
+          // One insertion per row at a time, by its 16 lanes together.
+          while (true) {
+            const unsigned long long work = __ballot(pending != 0);
+            if (work == 0)
+              break;
+            const unsigned long long mine = work & groupMask;
+            const int source = mine ? __ffsll((long long)mine) - 1 : lane;
+            const int c = __ffs(pending) - 1;
+            float wv = 0.0f;
+#pragma unroll
+            for (int cc = 0; cc < TR; ++cc)
+              if (cc == c)
+                wv = acc[r][cc];
+            const int colOf = c < 0 ? 0 : col0 + (c >> 2) * 64 + tc4 + (c & 3);
+            if (lane == source)
+              pending &= pending - 1;
+            const unsigned long long key =
+                packKey(__shfl(wv, source, 64), (unsigned int)__shfl(colOf, source, 64));
+            const int q = lane & 15;
+            if (mine && q < kList) {
+              const unsigned long long cur = list[q], prev = q > 0 ? list[q - 1] : 0;
+              if (cur > key)
+                list[q] = prev > key ? prev : key;
+            }
+            __builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront");
+            __builtin_amdgcn_wave_barrier();
+            __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "wavefront");
+            if (pending) {
+              const unsigned long long now = list[kList - 1];
+#pragma unroll
+              for (int cc = 0; cc < TR; ++cc)
+                if (!(packKey(acc[r][cc], (unsigned)(col0 + T::colInTile(cc))) < now))
+                  pending &= ~(1u << cc);
+            }
+          }
+        }
+      }
+      first = false;
+      __syncthreads(); // the tile is consumed
+    }
+    for (int i = tid; i < DIM * kList; i += T::THREADS) {
+      const int r = i / kList, at = rowTile * DIM + r;
+      if (at < rows)
+        partial[((size_t)at * splits + split) * kList + i % kList] = top[r][i % kList];
+    }
+  }
+}
+
+// The round's lists, 16 lanes per slot: a search row's from its parts (a lane
+// merges every 16th part, then the lanes' lowest leave in order), another's
+// with the lowest offer to it.
+__global__ void __launch_bounds__(256)
+    wardFinishKernel(Lists lists, const int *__restrict__ searchOf,
+                     const unsigned long long *__restrict__ partial,
+                     const unsigned long long *__restrict__ pushed,
+                     const int *__restrict__ mNow, const RoundState *st, int dim) {
+  if (roundOver(st))
+    return;
+  const int m = *mNow, i = (int)((blockIdx.x * blockDim.x + threadIdx.x) / 16);
+  if (i >= m)
+    return;
+  const int sub = threadIdx.x & 15;
+  unsigned long long *list = lists.keys + (size_t)i * kList;
+  const int place = searchOf[i];
+  unsigned long long key[kList];
+  if (place >= 0) {
+    const int splits = searchSplits(st->searches, m, dim);
+    const unsigned long long *part = partial + (size_t)place * splits * kList;
+#pragma unroll
+    for (int q = 0; q < kList; ++q)
+      key[q] = sub < splits ? part[sub * kList + q] : kEmptyKey;
+    for (int s = sub + 16; s < splits; s += 16)
+      for (int q = 0; q < kList; ++q) {
+        unsigned long long k = part[s * kList + q];
+        if (!(k < key[kList - 1]))
+          break; // the part's keys ascend
+#pragma unroll
+        for (int p = 0; p < kList; ++p) {
+          const unsigned long long cur = key[p];
+          key[p] = minKey(cur, k);
+          k = k < cur ? cur : k;
+        }
+      }
+    unsigned long long low = kEmptyKey;
+#pragma unroll
+    for (int q = 0; q < kList; ++q) {
+      low = rowMin16(key[0]);
+      if (key[0] == low) {
+#pragma unroll
+        for (int p = 0; p + 1 < kList; ++p)
+          key[p] = key[p + 1];
+        key[kList - 1] = kEmptyKey;
+      }
+      if (sub == 0)
+        list[q] = low;
+    }
+    if (sub == 0)
+      lists.bound[i] = low; // every other key is above the last
+  } else if (sub == 0) {
+    const unsigned long long offer = pushed[i];
+    if (!(offer < lists.bound[i]))
+      return;
+    int kept = 0;
+#pragma unroll
+    for (int q = 0; q < kList; ++q) {
+      key[q] = list[q];
+      kept += key[q] < offer;
+    }
+#pragma unroll
+    for (int q = 0; q < kList; ++q)
+      if (q >= kept)
+        list[q] = q == kept ? offer : kEmptyKey;
+    lists.bound[i] = offer; // what else was offered, or is beyond the list, is above it
+  }
+}
+
+__global__ void roundStartKernel(RoundState *st, int n) {
+  *st = RoundState{n, 0, 0, 0, 0};
 }
 
 // Every point its own cluster; rep = its original index (orig, null: the
@@ -528,12 +935,14 @@ int rnnWard(const float *X, int n, int d, const RnnOptions &opt, double *tree) {
     return 0;
   DevArray<double> c64a, c64b;
   DevArray<float> c32a, c32b;
-  DevArray<int> sizeA, sizeB, repA, repB, comp, survives, newIndex, blockTotals, numMerges;
-  DevArray<unsigned long long> nearest;
+  DevArray<int> sizeA, sizeB, repA, repB, comp, partner, survives, newIndex, searchOf, roundEnds;
+  DevArray<unsigned int> searchRows;
+  DevArray<unsigned long long> keysA, keysB, boundA, boundB, partial, pushed;
+  DevArray<unsigned char> scanTemp;
+  DevArray<RoundState> state;
   DevArray<DevMerge> merges;
   Status s;
   const size_t nd = (size_t)n * d;
-  const int scanBlocks = (n + kScanBlock - 1) / kScanBlock;
   s(c64a.alloc(nd));
   s(c64b.alloc(nd));
   s(c32a.alloc(nd));
@@ -543,88 +952,175 @@ int rnnWard(const float *X, int n, int d, const RnnOptions &opt, double *tree) {
   s(repA.alloc(n));
   s(repB.alloc(n));
   s(comp.alloc(n));
-  s(survives.alloc(n));
-  s(newIndex.alloc(n));
-  s(blockTotals.alloc(scanBlocks));
-  s(numMerges.alloc(1));
-  s(nearest.alloc(n));
+  s(partner.alloc(n));
+  s(survives.alloc((size_t)n + 1));
+  s(newIndex.alloc((size_t)n + 1));
+  s(searchOf.alloc(n));
+  s(searchRows.alloc(n));
+  s(keysA.alloc((size_t)n * kList));
+  s(keysB.alloc((size_t)n * kList));
+  s(boundA.alloc(n));
+  s(boundB.alloc(n));
+  s(pushed.alloc(n));
+  // A search has at most kSearchItems items or one split: rows x splits <=
+  // 128 kSearchItems, or the rows.
+  s(partial.alloc(((size_t)128 * kSearchItems + n) * kList));
+  s(scanTemp.alloc(scanTempBytes(n + 1)));
+  s(state.alloc(1));
+  s(roundEnds.alloc(n));
   s(merges.alloc(n - 1));
   if (!s.ok())
     return s.code;
   Clusters cur{c64a, c32a, sizeA, repA}, next{c64b, c32b, sizeB, repB};
+  Lists lists{keysA, boundA}, listsNext{keysB, boundB};
   hipLaunchKernelGGL(initClustersKernel, dim3(1024), dim3(256), 0, stream(), X, n, d, cur,
                      comp.get(), opt.orig);
-  s(fill(numMerges, 0, sizeof(int)));
-
-  std::vector<int> roundEnd;
-  int m = n, merged = 0;
-  enum { kNone, kDense, kChain } tail = kNone;
-  // Pruned passes (points in k-d order): merged clusters take the lower
-  // slot's place in the compacted order, so slots stay spatially coherent and
-  // the cluster tiles keep tight boxes. Every cluster needs its exact
-  // nearest, so no component bound is used; pruning stops for good once a
-  // pass computes more than half of the tile pairs.
-  bool pruneThisPass = opt.prune;
-  while (s.ok() && m > 1) {
-    if (opt.allowDense && m <= opt.denseBelow && wardMatrixFits(m)) {
-      tail = kDense;
-      break;
+  hipLaunchKernelGGL(roundStartKernel, dim3(1), dim3(1), 0, stream(), state.get(), n);
+  // Searches and their lists; count: the clusters, on the device, at most most.
+  auto search = [&](const int *count, int most) {
+    const int dim = most <= kSmallSearch ? 64 : 128;
+    {
+      PhaseTimer timer(kPhaseDistanceTiles);
+      auto launch = [&](auto side, auto fill) {
+        hipLaunchKernelGGL((wardSearchKernel<decltype(side)::value, decltype(fill)::value>),
+                           dim3(kSearchGroups * numCUs()), dim3(256), 0, stream(), cur.c32, d,
+                           cur.size, searchRows.get(), searchOf.get(), lists.bound, state.get(),
+                           count, partial.get(), pushed.get());
+      };
+      using Four = std::integral_constant<int, 4>;
+      using Eight = std::integral_constant<int, 8>;
+      using Fill = std::integral_constant<int, 32>;
+      if (dim == 64)
+        d <= 8 ? launch(Four{}, Eight{}) : launch(Four{}, Fill{});
+      else
+        d <= 8 ? launch(Eight{}, Eight{}) : launch(Eight{}, Fill{});
     }
-    s(fill(nearest, 0xff, m * sizeof(unsigned long long)));
+    PhaseTimer timer(kPhaseRnn);
+    hipLaunchKernelGGL(wardFinishKernel, dim3((most + 15) / 16), dim3(256), 0, stream(), lists,
+                       searchOf.get(), partial.get(), pushed.get(), count, state.get(), dim);
+    return (int)hipGetLastError();
+  };
+  auto gridOf = [](long long count) { return dim3((unsigned)((count + 255) / 256)); };
+
+  // A pruned pass (points in k-d order: merged clusters take the lower slot's
+  // place in the compacted order, so slots stay spatially coherent and the
+  // cluster tiles keep tight boxes) finds every cluster's nearest again: lists
+  // of one key. It stops for good once a pass computes more than half of the
+  // tile pairs, and the searches go on from its lists.
+  bool pruneThisPass = opt.prune;
+  DevArray<unsigned long long> nearest;
+  auto prunedPass = [&](int m) {
+    Status st;
+    if (!nearest.get())
+      st(nearest.alloc(n));
+    if (st.ok())
+      st(fill(nearest, 0xff, m * sizeof(unsigned long long)));
     WeightSpec w;
     w.kind = kWeightWard;
     w.size = cur.size;
-    if (m == n && opt.mixedFirstPass) {
-      // Every cluster is one point (size 1, component = slot): the Ward
-      // weight 2 * 1 * 1 / (1 + 1) * sq is sq exactly, and the mixed pass
-      // returns every point's exact (FP32 squared distance, slot) nearest.
-      int created = 0;
-      MixedPass *mp = mixedPassCreate(cur.c32, m, d, &created);
-      s(created);
-      if (mp) {
-        s(mixedPassRun(mp, comp, m, true, true, nearest));
-        mixedPassDestroy(mp);
-      }
-    } else if (pruneThisPass) {
-      double share = 1.0;
-      s(nearestOtherWalk(cur.c32, m, d, MetricSpec{kSqEuclidean, 2.0f}, w, comp, nullptr,
-                         nullptr, nearest, &share, opt.stats));
-      pruneThisPass = share <= kPruneGiveUpShare;
-    } else {
-      s(nearestOtherSymmetric(cur.c32, m, d, MetricSpec{kSqEuclidean, 2.0f}, w, comp, nullptr,
-                              nearest));
+    double share = 1.0;
+    if (st.ok())
+      st(nearestOtherWalk(cur.c32, m, d, MetricSpec{kSqEuclidean, 2.0f}, w, comp, nullptr, nullptr,
+                          nearest, &share, opt.stats));
+    pruneThisPass = share <= kPruneGiveUpShare;
+    if (st.ok())
+      hipLaunchKernelGGL(listsFromKeysKernel, gridOf(m), dim3(256), 0, stream(), nearest.get(), 1,
+                         m, lists);
+    st((int)hipGetLastError());
+    return st.code;
+  };
+
+  // The first lists: from the mixed pass (every cluster is one point, size 1,
+  // component = slot: the Ward weight 2 * 1 * 1 / (1 + 1) * sq is sq exactly,
+  // and the pass keeps every point's lowest exact (FP32 squared distance, slot)
+  // keys), from a pruned pass, or from a search of all rows.
+  if (opt.mixedFirstPass) {
+    int created = 0;
+    s(nearest.alloc(n));
+    MixedPass *mp = s.ok() ? mixedPassCreate(cur.c32, n, d, &created) : nullptr;
+    s(created);
+    if (mp) {
+      s(fill(nearest, 0xff, n * sizeof(unsigned long long)));
+      s(mixedPassRun(mp, comp, n, true, true, nearest));
+      int per = 0;
+      const unsigned long long *keys = mixedPassLists(mp, &per);
+      if (s.ok())
+        hipLaunchKernelGGL(listsFromKeysKernel, gridOf(n), dim3(256), 0, stream(), keys, per, n,
+                           lists);
+      s(sync()); // the pass's buffers are read
+      mixedPassDestroy(mp);
     }
-    {
-      PhaseTimer timer(kPhaseRnn);
-      const int blocks = (m + kScanBlock - 1) / kScanBlock;
-      hipLaunchKernelGGL(survivorsKernel, dim3((m + 255) / 256), dim3(256), 0, stream(),
-                         nearest.get(), m, survives.get());
-      hipLaunchKernelGGL(scanBlocksKernel, dim3(blocks), dim3(kScanBlock), 0, stream(),
-                         survives.get(), m, newIndex.get(), blockTotals.get());
-      hipLaunchKernelGGL(scanTotalsKernel, dim3(1), dim3(kScanBlock), 0, stream(),
-                         blockTotals.get(), blocks);
-      hipLaunchKernelGGL(addOffsetsKernel, dim3(blocks), dim3(kScanBlock), 0, stream(),
-                         newIndex.get(), m, blockTotals.get());
-      hipLaunchKernelGGL(rnnMergeKernel, dim3(2048), dim3(256), 0, stream(), cur, next,
-                         nearest.get(), newIndex.get(), m, d, merges.get(), numMerges.get());
+  } else if (opt.prune) {
+    s(prunedPass(n));
+  } else {
+    hipLaunchKernelGGL(searchAllKernel, gridOf(n), dim3(256), 0, stream(), n, searchRows.get(),
+                       searchOf.get(), pushed.get(), state.get());
+    s(search(&state.get()->m, n));
+  }
+  s((int)hipGetLastError());
+
+  RoundState host{n, 0, 0, 0, 0};
+  int queued = 0; // rounds queued so far
+  enum { kNone, kDense, kChain } tail = kNone;
+  while (s.ok() && host.m > 1) {
+    if (opt.allowDense && host.m <= opt.denseBelow && wardMatrixFits(host.m)) {
+      tail = kDense;
+      break;
+    }
+    // Up to kRoundsAhead rounds, launched for the clusters that the last read
+    // found; one at a time where a hand-over size is to be met, and while a
+    // round's work outweighs its read by far and shrinks the next launches.
+    const int ahead = opt.denseBelow > 0 || pruneThisPass ? 1
+                      : host.m > 32768                    ? 2
+                                                          : kRoundsAhead;
+    const int most = host.m;
+    for (int r = 0; r < ahead && s.ok(); ++r, ++queued) {
+      const int *count = newIndex.get() + most; // survivors: the next count
+      const bool small = most <= kSmallClusters;
+      {
+        PhaseTimer timer(kPhaseRnn);
+        if (small) {
+          hipLaunchKernelGGL(smallRoundKernel, dim3(1), dim3(kSmallThreads), 0, stream(), lists,
+                             state.get(), most, r == 0, opt.minProgress, roundEnds.get(),
+                             partner.get(), newIndex.get());
+        } else {
+          hipLaunchKernelGGL(survivorsKernel, gridOf(most + 1), dim3(256), 0, stream(), lists,
+                             state.get(), most, partner.get(), survives.get());
+          s(exclusiveScan(survives.get(), newIndex.get(), most + 1, scanTemp.get()));
+        }
+        const int slotBlocks = (most + 255) / 256;
+        const int blocks = (int)std::min<long long>(2048, ((long long)most * d + 255) / 256);
+        hipLaunchKernelGGL(rnnMergeKernel, dim3(slotBlocks + blocks), dim3(256), 0, stream(), cur,
+                           next, lists, listsNext, partner.get(), newIndex.get(), d, state.get(),
+                           merges.get(), searchRows.get(), searchOf.get(), pushed.get(),
+                           slotBlocks);
+      }
+      std::swap(cur, next);
+      std::swap(lists, listsNext);
+      int now = 0;
+      if (pruneThisPass)
+        s(download(&now, count, sizeof(now)));
+      s(pruneThisPass && now > 1 ? prunedPass(now) : search(count, most));
+      if (!small || r + 1 == ahead) {
+        PhaseTimer timer(kPhaseRnn);
+        hipLaunchKernelGGL(roundEndKernel, dim3(1), dim3(1), 0, stream(), state.get(), count,
+                           opt.minProgress, roundEnds.get());
+      }
       s((int)hipGetLastError());
     }
-    int total = 0;
-    s(download(&total, numMerges, sizeof(int)));
-    if (!s.ok())
-      break;
-    const int roundMerges = total - merged;
-    merged = total;
-    roundEnd.push_back(total);
-    std::swap(cur, next);
-    const int before = m;
-    m -= roundMerges;
-    if (m > 1 && (roundMerges == 0 || roundMerges < opt.minProgress * before)) {
-      tail = opt.allowDense && wardMatrixFits(m) ? kDense : kChain;
+    s(download(&host, state, sizeof(host)));
+    if (s.ok() && host.stop && host.m > 1) {
+      tail = opt.allowDense && wardMatrixFits(host.m) ? kDense : kChain;
       break;
     }
   }
+  // Queued rounds after the last swapped the buffers for nothing.
+  if ((queued - host.rounds) & 1)
+    std::swap(cur, next);
+  const int m = host.m, merged = host.merges;
+  std::vector<int> roundEnd(host.rounds);
   std::vector<DevMerge> dm(merged);
+  s(download(roundEnd.data(), roundEnds, roundEnd.size() * sizeof(int)));
   s(download(dm.data(), merges, merged * sizeof(DevMerge)));
   if (!s.ok())
     return s.code;

@@ -104,6 +104,28 @@ def test_rnn_matches_scipy(n, d):
     assert_same_dendrogram(Z, scipy_ward(X), rtol=1e-5, atol=1e-6)
 
 
+@pytest.mark.parametrize("n, d", [(5, 2), (9, 40), (65, 8), (129, 9), (1025, 33), (4100, 70),
+                                  (8193, 5)])
+@pytest.mark.parametrize("data", ["normal", "lattice"])
+def test_rnn_lists_against_the_chain(n, d, data):
+    # Rounds whose clusters keep lists of their nearest: fewer clusters than a
+    # list holds, the edges of the search tiles (64 rows), more features than
+    # one fill stages (32), and the most clusters one workgroup numbers (8,192);
+    # with ties, where lists end in equal keys. The chain finds each nearest by a
+    # scan of all clusters in FP64.
+    rng = np.random.default_rng(n + d)
+    X = rng.normal(size=(n, d)) if data == "normal" else rng.integers(0, 50, (n, d))
+    X = X.astype(np.float32)
+    rnn = cuhc.linkage(X, method="ward", algorithm="rnn")
+    chain = cuhc.linkage(X, method="ward", algorithm="nn_chain")
+    assert_valid_tree(rnn, n)
+    if data == "normal":
+        assert_same_dendrogram(rnn, chain, rtol=1e-5, atol=1e-6)
+    else:  # equal weights may pair either way: the lowest merges are the same
+        np.testing.assert_allclose(rnn[0, 2], chain[0, 2], rtol=1e-6)
+    np.testing.assert_array_equal(cuhc.linkage(X, method="ward", algorithm="rnn"), rnn)
+
+
 def test_rnn_many_points_and_error_bound():
     X = blobs(n_samples=6000, n_features=10, centers=25, seed=51)
     Z = cuhc.linkage(X, method="ward")
