@@ -98,10 +98,11 @@ int boruvkaMst(const float *X, int n, int d, MetricSpec m, WeightSpec w, const M
   // Rows settled from the learned candidate lists (mutual reachability,
   // alpha = 1) are closed to the walk.
   const bool useLists = opt.lists && opt.prune && w.kind == kWeightMReach && w.alpha == 1.0f;
-  // Without lists, a pruned mutual-reachability run has the first round's walk
-  // keep each row's 4 smallest keys over all other points, and settles the
-  // later rounds' rows from them.
-  const bool keepKeys = !useLists && opt.prune && w.kind == kWeightMReach;
+  // Without lists, the first round's walk keeps each row's 4 smallest keys over
+  // all other points, and the later rounds' rows settle from them: whatever
+  // share of the tiles that walk computes, it replaces most of the later
+  // rounds' passes.
+  const bool keepKeys = !useLists && opt.prune;
   DevArray<unsigned char> dClosed;
   DevArray<unsigned long long> dListCounters, dKept;
   if (useLists || keepKeys)
@@ -163,6 +164,7 @@ int boruvkaMst(const float *X, int n, int d, MetricSpec m, WeightSpec w, const M
           s(nearestOtherWalk(X, n, d, m, w, dComp, opt.devOrig, nullptr, dNearest, &share,
                              opt.stats, 1, dSkip, nullptr, dKept));
           keptValid = true;
+          share = 0.0; // the next rounds walk the rows that the keys leave open
         } else {
           if (keepKeys)
             s(settleFromKept(dKept, n, dComp, posOf, dSkip, dNearest, dCompBest, dClosed));

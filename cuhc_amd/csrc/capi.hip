@@ -10,6 +10,8 @@
 #include <algorithm>
 #include <atomic>
 #include <mutex>
+#include <new>
+#include <unordered_map>
 
 using namespace cuhc;
 
@@ -19,6 +21,9 @@ std::atomic<int> gPruneMode{kPruneAuto};
 std::atomic<int> gPrecision{0};
 std::mutex gStatsMutex;
 PassStats gPruneStats;
+// Sizes of the buffers handed out by cuhc_device_alloc.
+std::mutex gBuffersMutex;
+std::unordered_map<void *, size_t> gBuffers;
 
 bool validLinkageAlgorithm(int linkageId, int algorithmId, int metricId) {
   return algorithmId == kAlgDense || (algorithmId == kAlgMst && linkageId == kSingle) ||
@@ -82,8 +87,9 @@ int linkageImpl(const float *X, bool onDevice, int n, int d, int metricId, float
     bool prune = !mixed && shouldPrune(gPruneMode.load(), metricId, n, d);
     DevicePoints pts;
     s(onDevice ? pts.adopt(X, n, d, prune) : pts.upload(X, n, d, prune));
-    if (s.ok())
-      s(decidePruning(pts, n, d, m, prune));
+    // No sampled decision here: the walk that keeps keys pays whatever it
+    // prunes (50,021 points of 10 normal features, manhattan, whole calls:
+    // five symmetric passes 13.4 ms, the walks 10.8; 60,000 of 40 35 and 19).
     PassStats stats;
     if (s.ok())
       s(singleLinkageMst(pts, n, d, m, prune, mixed, &stats, tree));
@@ -362,21 +368,50 @@ int cuhc_set_precision(int mode) {
   return 0;
 }
 
+// Callers' buffers come from the library's cache of freed blocks (a fresh 335
+// MB buffer costs 0.4 ms of page mapping, more than the distance matrix that
+// fills it), which is bounded and given back as for the library's own. The
+// library stream may still work on a cached block, and the caller's streams on
+// a freed one: both are waited for, as hipFree waits.
 int cuhc_device_alloc(unsigned long long bytes, void **ptr) {
   *ptr = nullptr;
-  hipError_t e = hipMalloc(ptr, bytes);
-  if (e == hipErrorOutOfMemory) {
-    // The library's cache of freed blocks may hold the memory: release it and retry.
-    (void)hipGetLastError();
-    releaseCachedBlocks();
-    e = hipMalloc(ptr, bytes);
+  int s = deviceAlloc(ptr, (size_t)bytes);
+  if (s)
+    return s;
+  s = sync();
+  if (s == 0) {
+    try {
+      std::lock_guard<std::mutex> lock(gBuffersMutex);
+      gBuffers[*ptr] = (size_t)bytes;
+    } catch (const std::bad_alloc &) {
+      s = (int)hipErrorOutOfMemory;
+    }
   }
-  return (int)e;
+  if (s) {
+    deviceFree(*ptr, (size_t)bytes);
+    *ptr = nullptr;
+  }
+  return s;
 }
 
 void cuhc_release(void) { releaseLibraryState(); }
 
-int cuhc_device_free(void *ptr) { return ptr ? (int)hipFree(ptr) : 0; }
+int cuhc_device_free(void *ptr) {
+  if (!ptr)
+    return 0;
+  size_t bytes = 0;
+  {
+    std::lock_guard<std::mutex> lock(gBuffersMutex);
+    const auto it = gBuffers.find(ptr);
+    if (it == gBuffers.end())
+      return (int)hipFree(ptr); // not one of ours
+    bytes = it->second;
+    gBuffers.erase(it);
+  }
+  const int s = (int)hipDeviceSynchronize();
+  deviceFree(ptr, bytes);
+  return s;
+}
 
 int cuhc_copy_to_device(void *dst, const void *src, unsigned long long bytes) {
   return upload(dst, src, bytes);

@@ -386,9 +386,12 @@ DEV float boxLowerBound(const Metric &metric, const float *lowA, const float *hi
   return metric.finish(acc);
 }
 
-// Column tile visited at `step` from row tile I: I, I+1, I-1, I+2, ... (-1 if outside).
-DEV int walkTile(int rowTile, int step, int numTiles) {
-  const int off = (step + 1) >> 1;
+// Column tile visited at `step` from row tile I: I, I+1, I-1, I+2, ... (-1 if
+// outside). Of a walk in splits, split s takes I itself and every splits-th
+// pair after it.
+DEV int walkTile(int rowTile, int step, int numTiles, int splits = 1, int split = 0) {
+  const int pair = (step + 1) >> 1;
+  const int off = pair == 0 ? 0 : (pair - 1) * splits + split + 1;
   const int tile = (step & 1) ? rowTile + off : rowTile - off;
   return (tile >= 0 && tile < numTiles) ? tile : -1;
 }
@@ -455,6 +458,9 @@ template <class Weight> struct ColumnStage {
 // computed nearly twice the pairs (47% of all pairs of 100,000 points of 8
 // features against 26% by 32 rows). HDBSCAN's passes over 10^6 points of 8
 // features took 290 ms; by wave 235, and with the sparse tiles first 202.
+// With few row tiles a walk is split over gridDim.y workgroups, which share a
+// row's best through nearest[] (kept lists are merged afterwards, one per
+// split): the four passes over 100,000 points took 18.1 ms, and take 5.9.
 
 // The rows of a compact walk: n rows gathered into X (d features each) from
 // positions pos[0 .. n) of the full order (ascending); center[t] is the
@@ -477,7 +483,7 @@ constexpr int kKeptKeys = 4;
 // waits better than two (C3's four Borůvka walks: 298 ms with two waves, 265 ms
 // with three).
 template <class T, class Metric, class Weight, bool COMPACT = false, bool KEEP = false>
-__global__ void __launch_bounds__(256, (KEEP ? 3 : 1))
+__global__ void __launch_bounds__(256, (!KEEP ? 1 : T::FILL == 8 ? 3 : 2))
     nearestOtherWalkKernel(const float *__restrict__ X, int n, int d, Metric metric,
                            Weight weight, const int *__restrict__ comp,
                            const int *__restrict__ orig, Boxes boxes,
@@ -517,6 +523,7 @@ __global__ void __launch_bounds__(256, (KEEP ? 3 : 1))
   const int numTiles = boxes.numTiles;
   const int row0 = rowTile * T::DIM;
   const int center = COMPACT ? rows.center[rowTile] : rowTile;
+  const int splits = gridDim.y, split = blockIdx.y;
   const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
   // A row is open unless it lies past the end, in the skipped component, or
   // is closed (its exact answer is already in nearest[]).
@@ -612,16 +619,27 @@ __global__ void __launch_bounds__(256, (KEEP ? 3 : 1))
     return __shfl(need, 0, 64);
   };
 
-  const int steps = 2 * numTiles;
+  const int steps = 2 * ((numTiles + splits - 1) / splits) + 1;
   for (int base = 0; base < steps; base += kBatch) {
-    // Other workgroups may have found better edges for these components.
+    // Other workgroups may have found better edges for these components, and
+    // other splits for these rows.
     if (compBest && open)
       cap = fminf(cap, capOf(compBest[ownComp]));
+    if (!KEEP && splits > 1 && open) {
+      unsigned long long *shared = &nearest[posOf(ownRow)];
+      const unsigned long long mine = rowBest[own];
+      const unsigned long long theirs =
+          __hip_atomic_load(shared, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+      if (mine < theirs)
+        atomicMin(shared, mine);
+      else
+        rowBest[own] = theirs;
+    }
     const float reach = newBound();
     {
       // -1: never computed (outside the grid, or both sides wholly one component).
       const int step = base + lane;
-      const int colTile = step < steps ? walkTile(center, step, numTiles) : -1;
+      const int colTile = step < steps ? walkTile(center, step, numTiles, splits, split) : -1;
       float lb = -1.0f;
       if (colTile >= 0 && !(compLow == compHigh && boxes.minComp[colTile] == compLow &&
                             boxes.maxComp[colTile] == compLow)) {
@@ -654,7 +672,7 @@ __global__ void __launch_bounds__(256, (KEEP ? 3 : 1))
       }
       if (activeWaves == 0)
         continue;
-      const int colTile = walkTile(center, base + j, numTiles);
+      const int colTile = walkTile(center, base + j, numTiles, splits, split);
       computed += activeWaves;
       if (base + j >= computeSteps)
         continue; // estimate: counted against the bound reached so far, not computed
@@ -800,7 +818,7 @@ __global__ void __launch_bounds__(256, (KEEP ? 3 : 1))
     for (int e = threadIdx.x; e < T::DIM * kKeptKeys; e += T::THREADS) {
       const int i = e / kKeptKeys;
       if (row0 + i < nRows)
-        kept[(size_t)posOf(row0 + i) * kKeptKeys + e % kKeptKeys] = rowTop[e];
+        kept[((size_t)split * n + posOf(row0 + i)) * kKeptKeys + e % kKeptKeys] = rowTop[e];
     }
     for (int i = threadIdx.x; i < T::DIM; i += T::THREADS)
       rowBest[i] = rowTop[i * kKeptKeys];
@@ -976,6 +994,49 @@ struct DeviceBoxes {
 // overestimate of the pruned share: the bound would keep shrinking).
 constexpr int kEstimateSteps = 64;
 
+// Splits of a walk over rowTiles row tiles: enough workgroups to even out the
+// row tiles' very different lengths (a resident chip's worth several times
+// over), each with eight column tiles at least.
+int walkSplits(int rowTiles, int tiles, int most) {
+  const int wanted = 16 * numCUs() / std::max(1, rowTiles);
+  return std::max(1, std::min({wanted, tiles / 8, most}));
+}
+constexpr int kMostSplits = 64;
+constexpr int kKeptSplits = 4; // each split keeps a list of its own to merge
+
+// The lowest keys of a row's lists (ascending, distinct columns but for the
+// row's own tile, which every split walks) into the first list.
+__global__ void mergeKeptKernel(const unsigned long long *__restrict__ lists, int splits, int n,
+                                unsigned long long *__restrict__ kept) {
+  const int p = blockIdx.x * blockDim.x + threadIdx.x;
+  if (p >= n)
+    return;
+  unsigned long long key[kKeptKeys];
+#pragma unroll
+  for (int q = 0; q < kKeptKeys; ++q)
+    key[q] = lists[(size_t)p * kKeptKeys + q];
+  for (int s = 1; s < splits; ++s)
+#pragma unroll
+    for (int e = 0; e < kKeptKeys; ++e) {
+      unsigned long long k = lists[((size_t)s * n + p) * kKeptKeys + e];
+      bool known = false;
+#pragma unroll
+      for (int q = 0; q < kKeptKeys; ++q)
+        known |= key[q] == k;
+      if (known)
+        continue;
+#pragma unroll
+      for (int q = 0; q < kKeptKeys; ++q) {
+        const unsigned long long cur = key[q];
+        key[q] = minKey(cur, k);
+        k = k < cur ? cur : k;
+      }
+    }
+#pragma unroll
+  for (int q = 0; q < kKeptKeys; ++q)
+    kept[(size_t)p * kKeptKeys + q] = key[q];
+}
+
 // Dynamic LDS of the walk: a row box per wave.
 template <class T> size_t walkBoxBytes(int d) {
   return (size_t)(T::THREADS / 64) * 2 * d * sizeof(float);
@@ -1003,19 +1064,29 @@ int runWalk(const float *X, int n, int d, const Metric &metric, const Weight &we
   {
     PhaseTimer timer(kPhaseDistanceTiles);
     bool launched = false;
-    if constexpr (Weight::kHasValue) {
+    if constexpr (Weight::kDistBound) { // not Ward's, which keeps its own lists
       if (kept) {
+        const int splits = walkSplits(sampled, tiles, kKeptSplits);
+        DevArray<unsigned long long> lists;
+        if (splits > 1)
+          s(lists.alloc((size_t)splits * n * kKeptKeys));
+        if (!s.ok())
+          return s.code;
         hipLaunchKernelGGL((nearestOtherWalkKernel<T, Metric, Weight, false, true>),
-                           dim3(sampled), dim3(256), walkBoxBytes<T>(d), stream(), X, n, d,
+                           dim3(sampled, splits), dim3(256), walkBoxBytes<T>(d), stream(), X, n, d,
                            metric, weight, comp, orig, boxes.view, nullptr, nearest,
                            counter.get(), stride, stride > 1 ? kEstimateSteps : 0x7fffffff,
-                           skipComp, closedRows, RowSet{}, kept);
+                           skipComp, closedRows, RowSet{}, splits > 1 ? lists.get() : kept);
+        if (splits > 1)
+          hipLaunchKernelGGL(mergeKeptKernel, dim3((n + 255) / 256), dim3(256), 0, stream(),
+                             lists.get(), splits, n, kept);
         launched = true;
       }
     }
     if (!launched)
-      hipLaunchKernelGGL((nearestOtherWalkKernel<T, Metric, Weight>), dim3(sampled), dim3(256),
-                         walkBoxBytes<T>(d), stream(), X, n, d, metric, weight, comp, orig,
+      hipLaunchKernelGGL((nearestOtherWalkKernel<T, Metric, Weight>),
+                         dim3(sampled, stride > 1 ? 1 : walkSplits(sampled, tiles, kMostSplits)),
+                         dim3(256), walkBoxBytes<T>(d), stream(), X, n, d, metric, weight, comp, orig,
                          boxes.view, compBest, nearest, counter.get(), stride,
                          stride > 1 ? kEstimateSteps : 0x7fffffff, skipComp, closedRows,
                          RowSet{}, nullptr);
@@ -1122,8 +1193,8 @@ int runWalkOpen(const float *X, int n, int d, const Metric &metric, const Weight
   rows.center = center;
   {
     PhaseTimer timer(kPhaseDistanceTiles);
-    hipLaunchKernelGGL((nearestOtherWalkKernel<T, Metric, Weight, true>), dim3(rowTiles),
-                       dim3(256), walkBoxBytes<T>(d), stream(), X, n, d, metric, weight, comp,
+    hipLaunchKernelGGL((nearestOtherWalkKernel<T, Metric, Weight, true>),
+                       dim3(rowTiles, walkSplits(rowTiles, tiles, kMostSplits)), dim3(256), walkBoxBytes<T>(d), stream(), X, n, d, metric, weight, comp,
                        orig, colBoxes.view, compBest, nearest, counter.get(), 1, 0x7fffffff,
                        skipComp, closedRows, rows, nullptr);
     s((int)hipGetLastError());
@@ -1149,7 +1220,7 @@ int nearestOtherWalk(const float *X, int n, int d, MetricSpec m, WeightSpec w, c
                      const unsigned char *closedRows, unsigned long long *kept) {
   if (!metricHasBoxBound(m.id))
     return kErrInvalidMetric;
-  if (kept && (w.kind != kWeightMReach || closedRows || stride != 1))
+  if (kept && (w.kind == kWeightWard || closedRows || stride != 1))
     return kErrInvalidAlgorithm;
   if (w.kind == kWeightWard) {
     if (m.id != kSqEuclidean)
@@ -1168,13 +1239,11 @@ int nearestOtherWalk(const float *X, int n, int d, MetricSpec m, WeightSpec w, c
       return withWeightFor(metric, w, [&](auto weight) {
         return withFill(d, [&](auto fill) {
           using T = Tile<8, decltype(fill)::value>;
-          // Closed rows come with mutual-reachability weights (their answers
-          // settled from candidate lists): walk the open rows only.
-          if constexpr (decltype(weight)::kHasValue) {
-            if (closedRows && stride == 1)
-              return runWalkOpen<T>(X, n, d, metric, weight, comp, orig, compBest, nearest,
-                                    share, stats, skipComp, closedRows);
-          }
+          // Closed rows (their answers settled from lists): walk the open rows
+          // only.
+          if (closedRows && stride == 1)
+            return runWalkOpen<T>(X, n, d, metric, weight, comp, orig, compBest, nearest, share,
+                                  stats, skipComp, closedRows);
           return runWalk<T>(X, n, d, metric, weight, comp, orig, compBest, nearest, share,
                             stats, stride, skipComp, closedRows, kept);
         });
@@ -1216,12 +1285,34 @@ __global__ void settleFromKeptKernel(const unsigned long long *__restrict__ kept
 
 } // namespace
 
+namespace {
+
+// Rows left open whose list ends above the best edge known for their component:
+// every point the list misses weighs at least its last key, so the row cannot
+// hold the component's smallest edge, and closes without an answer.
+__global__ void closeHopelessKernel(const unsigned long long *__restrict__ kept, int n,
+                                    const int *__restrict__ comp,
+                                    const unsigned int *__restrict__ compBest,
+                                    unsigned char *__restrict__ closed) {
+  for (int p = blockIdx.x * blockDim.x + threadIdx.x; p < n; p += gridDim.x * blockDim.x)
+    if (!closed[p]) {
+      const unsigned long long last = kept[(size_t)p * kKeptKeys + kKeptKeys - 1];
+      if (last == kEmptyKey || (unsigned int)(last >> 32) > compBest[comp[p]])
+        closed[p] = 1;
+    }
+}
+
+} // namespace
+
 int settleFromKept(const unsigned long long *kept, int n, const int *comp, const int *posOf,
                    const int *skipComp, unsigned long long *nearest, unsigned int *compBest,
                    unsigned char *closed) {
   const int blocks = std::max(1, std::min(4 * numCUs(), (n + 255) / 256));
   hipLaunchKernelGGL(settleFromKeptKernel, dim3(blocks), dim3(256), 0, stream(), kept, n, comp,
                      posOf, skipComp, nearest, compBest, closed);
+  if (compBest)
+    hipLaunchKernelGGL(closeHopelessKernel, dim3(blocks), dim3(256), 0, stream(), kept, n, comp,
+                       compBest, closed);
   return (int)hipGetLastError();
 }
 

@@ -53,6 +53,27 @@ def test_core_methods_agree(k, metric):
             hdbscan_tree(X, k, metric=metric, core_method="fused")
 
 
+@pytest.mark.parametrize("k", [1, 15, 16, 17, 33, 64])
+@pytest.mark.parametrize("data", ["lattice", "blobs"])
+@pytest.mark.parametrize("pruning", ["always", "never"])
+def test_core_lists_and_select_edges(k, data, pruning):
+    # The fused lists at the edges of their 16-lane insertions and the radix
+    # select (auto's choice for few points), on many equal distances and on
+    # rows that end in the last tile's first wave; pruned by waves of 32 rows.
+    if data == "lattice":
+        X = np.random.default_rng(k).integers(0, 7, (901, 3)).astype(np.float32)
+    else:
+        X = blobs(n_samples=670, n_features=9, centers=5, noise_fraction=0.1, seed=k)
+    expected = oracle.core_distances(X, k)
+    _lib.set_pruning(pruning)
+    try:
+        for method in ["fused", "auto"]:
+            _, core = hdbscan_tree(X, k, core_method=method)
+            np.testing.assert_array_equal(core, expected)
+    finally:
+        _lib.set_pruning("auto")
+
+
 @pytest.mark.parametrize("n_features", [2, 8])
 @pytest.mark.parametrize("k", [1, 5, 40])
 @pytest.mark.parametrize("alpha", [1.0, 0.7, 1.7])

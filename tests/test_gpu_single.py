@@ -38,6 +38,23 @@ def test_contraction_forms(data, n):
     np.testing.assert_array_equal(run(X, "manhattan"), oracle.single_linkage(X, "manhattan"))
 
 
+@pytest.mark.parametrize("n, d", [(1100, 2), (4111, 20), (16500, 6)])
+@pytest.mark.parametrize("metric", ["euclidean", "manhattan", "chebyshev"])
+@pytest.mark.parametrize("data", ["lattice", "far groups"])
+def test_split_walks_and_kept_keys(n, d, metric, data):
+    # Walks split over workgroups (few row tiles, eight column tiles or more),
+    # whose kept lists are merged, and rows closed by their list's last key: ties
+    # at the last key, and groups with no near neighbour outside.
+    rng = np.random.default_rng(n)
+    if data == "lattice":
+        X = rng.integers(0, 5, (n, d))
+    else:
+        X = rng.normal(size=(n, d)) + 100.0 * rng.integers(0, 4, (n, 1))
+    X = X.astype(np.float32)
+    np.testing.assert_array_equal(run(X, metric, pruning="always"),
+                                  oracle.single_linkage(X, metric))
+
+
 @pytest.mark.parametrize("n, d", [(129, 1), (257, 3), (1025, 65), (4000, 2), (20001, 5)])
 @pytest.mark.parametrize("spread", ["even", "outlier", "constant"])
 def test_spatial_order_shapes(n, d, spread):
