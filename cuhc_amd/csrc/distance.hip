@@ -996,12 +996,17 @@ constexpr int kEstimateSteps = 64;
 
 // Splits of a walk over rowTiles row tiles: enough workgroups to even out the
 // row tiles' very different lengths (a resident chip's worth several times
-// over), each with eight column tiles at least.
-int walkSplits(int rowTiles, int tiles, int most) {
-  const int wanted = 16 * numCUs() / std::max(1, rowTiles);
+// over), each with eight column tiles at least. However many row tiles
+// there are, a split walks about longest column tiles at most: a later round
+// leaves a few sparse rows that walk all the way alone (rounds 3 and 4 over 10^6
+// points of 8 features, 7,813 tiles: 30 ms each, 6 of them VALU work; by 1,024
+// tiles 13 ms).
+int walkSplits(int rowTiles, int tiles, int most, int longest) {
+  const int wanted = std::max(16 * numCUs() / std::max(1, rowTiles), tiles / longest);
   return std::max(1, std::min({wanted, tiles / 8, most}));
 }
 constexpr int kMostSplits = 64;
+constexpr int kLongestWalk = 1024;
 constexpr int kKeptSplits = 4; // each split keeps a list of its own to merge
 
 // The lowest keys of a row's lists (ascending, distinct columns but for the
@@ -1066,7 +1071,7 @@ int runWalk(const float *X, int n, int d, const Metric &metric, const Weight &we
     bool launched = false;
     if constexpr (Weight::kDistBound) { // not Ward's, which keeps its own lists
       if (kept) {
-        const int splits = walkSplits(sampled, tiles, kKeptSplits);
+        const int splits = walkSplits(sampled, tiles, kKeptSplits, 0x7fffffff);
         DevArray<unsigned long long> lists;
         if (splits > 1)
           s(lists.alloc((size_t)splits * n * kKeptKeys));
@@ -1085,7 +1090,8 @@ int runWalk(const float *X, int n, int d, const Metric &metric, const Weight &we
     }
     if (!launched)
       hipLaunchKernelGGL((nearestOtherWalkKernel<T, Metric, Weight>),
-                         dim3(sampled, stride > 1 ? 1 : walkSplits(sampled, tiles, kMostSplits)),
+                         dim3(sampled, stride > 1 ? 1 : walkSplits(sampled, tiles, kMostSplits,
+                                                                   kLongestWalk)),
                          dim3(256), walkBoxBytes<T>(d), stream(), X, n, d, metric, weight, comp, orig,
                          boxes.view, compBest, nearest, counter.get(), stride,
                          stride > 1 ? kEstimateSteps : 0x7fffffff, skipComp, closedRows,
@@ -1194,7 +1200,8 @@ int runWalkOpen(const float *X, int n, int d, const Metric &metric, const Weight
   {
     PhaseTimer timer(kPhaseDistanceTiles);
     hipLaunchKernelGGL((nearestOtherWalkKernel<T, Metric, Weight, true>),
-                       dim3(rowTiles, walkSplits(rowTiles, tiles, kMostSplits)), dim3(256), walkBoxBytes<T>(d), stream(), X, n, d, metric, weight, comp,
+                       dim3(rowTiles, walkSplits(rowTiles, tiles, kMostSplits, kLongestWalk)),
+                       dim3(256), walkBoxBytes<T>(d), stream(), X, n, d, metric, weight, comp,
                        orig, colBoxes.view, compBest, nearest, counter.get(), 1, 0x7fffffff,
                        skipComp, closedRows, rows, nullptr);
     s((int)hipGetLastError());
