@@ -14,7 +14,19 @@
 //   4-pass MSB-first byte radix select over the FP32 bit patterns with
 //   per-wave LDS histograms.
 // Both are exact and bit-identical (the k-th smallest value is unique).
+//
+// Bound by FP32 VALU work and, where the walks' lengths differ, by the longest:
+// the pruned pass over all points takes its row tiles largest box first, as
+// sparse rows walk farthest (10^6 points, k = 25: 122 to 104 ms; before, 72 ms
+// of it issued VALU instructions). With few row tiles a walk is split over
+// gridDim.y workgroups. Each keeps a list of its own columns; rows share a bound
+// (kthBits), the smallest k-th distance that any split has found, and first the
+// one within the home tile, from a pass of its own: values from the bound on
+// are left out. A second kernel takes the k-th of a row's lists and bound
+// (100,000 points, k = 25: 7.6 to 5.9 ms; 6.5 without the order of the tiles,
+// 7.5 without the first bound, as every split filled its lists with far values).
 #include "mst.hpp"
+#include "primitives.hpp"
 #include "tile.hpp"
 
 #include <algorithm>
@@ -30,8 +42,13 @@ struct CoreBoxes {
   int numTiles = 0;
 };
 
-DEV int walkTileCore(int rowTile, int step, int numTiles) {
-  const int off = (step + 1) >> 1;
+// Of a walk in splits, split 0 takes the home tile and split s every splits-th
+// pair of tiles beside it (-1: none): each column tile is one split's.
+DEV int walkTileCore(int rowTile, int step, int numTiles, int splits = 1, int split = 0) {
+  const int pair = (step + 1) >> 1;
+  if (pair == 0 && split > 0)
+    return -1;
+  const int off = pair == 0 ? 0 : (pair - 1) * splits + split + 1;
   const int tile = (step & 1) ? rowTile + off : rowTile - off;
   return (tile >= 0 && tile < numTiles) ? tile : -1;
 }
@@ -87,7 +104,8 @@ __global__ void __launch_bounds__(256, (coreMinWaves<T, Metric>()))
     kthNearestFusedKernel(const float *__restrict__ X, int n, int d, Metric metric, int k,
                           float *__restrict__ core, CoreBoxes boxes, int stepLimit,
                           const float *__restrict__ rowsX, int numRows,
-                          const int *__restrict__ rowPos, const int *__restrict__ tileList) {
+                          const int *__restrict__ rowPos, const int *__restrict__ tileList,
+                          unsigned int *__restrict__ kthBits, float *__restrict__ partial) {
   constexpr int TR = T::TR, kWaves = T::THREADS / 64, kWaveRows = T::WAVE_ROWS;
   constexpr int kBatch = 64; // walk steps whose box bounds are computed at once
   __shared__ __align__(16) TileSmem<T> sm;
@@ -96,6 +114,8 @@ __global__ void __launch_bounds__(256, (coreMinWaves<T, Metric>()))
   __shared__ float lowerBound[kWaves][kBatch];
   __shared__ unsigned long long within[kWaves];
   __shared__ float largestKth[kWaves];
+  // Per row, the smallest k-th distance published by any split.
+  __shared__ float sharedKth[T::DIM];
   extern __shared__ float lists[]; // [DIM][k], then the waves' row boxes [kWaves][2 d] if pruning
 
   const int rowTile = tileList ? tileList[blockIdx.x] : (int)blockIdx.x;
@@ -103,8 +123,11 @@ __global__ void __launch_bounds__(256, (coreMinWaves<T, Metric>()))
   const float *A = rowsX ? rowsX : X;
   const int nA = rowsX ? numRows : n;
   const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
+  const int splits = gridDim.y, split = blockIdx.y;
   for (int i = threadIdx.x; i < T::DIM * k; i += T::THREADS)
     lists[i] = INFINITY;
+  for (int i = threadIdx.x; i < T::DIM; i += T::THREADS)
+    sharedKth[i] = splits > 1 && row0 + i < nA ? __uint_as_float(kthBits[row0 + i]) : INFINITY;
   const bool prune = boxes.numTiles > 0;
   float *rowBox = lists + T::DIM * k + wave * 2 * d;
   if (prune) {
@@ -146,12 +169,13 @@ __global__ void __launch_bounds__(256, (coreMinWaves<T, Metric>()))
   // workgroup skips it when every wave does. Every wave computes its bounds of
   // 64 steps at once; only the steps some wave still had within reach when
   // the batch began are looked at again.
-  const int steps = min(2 * numTiles, stepLimit);
+  const int steps = min(2 * ((numTiles + splits - 1) / splits) + 1, stepLimit);
+  int computed = 0; // tiles, of the workgroup
   for (int base = 0; base < steps; base += kBatch) {
     unsigned long long todo;
     {
       const int step = base + lane;
-      const int colTile = step < steps ? walkTileCore(homeTile, step, numTiles) : -1;
+      const int colTile = step < steps ? walkTileCore(homeTile, step, numTiles, splits, split) : -1;
       float lb = 0.0f;
       if (prune && colTile >= 0)
         lb = coreBoxBound(metric, rowBox, rowBox + d, boxes.low + (size_t)colTile * d,
@@ -184,7 +208,7 @@ __global__ void __launch_bounds__(256, (coreMinWaves<T, Metric>()))
         if (!any)
           continue;
       }
-      const int col0 = walkTileCore(homeTile, base + j, numTiles) * T::DIM;
+      const int col0 = walkTileCore(homeTile, base + j, numTiles, splits, split) * T::DIM;
       // With an accumulator bound the tile holds raw accumulators, and only the
       // pairs within the bound of the row's current k-th distance are finished
       // (most pairs of a tile are not, which skips their sqrt).
@@ -202,7 +226,7 @@ __global__ void __launch_bounds__(256, (coreMinWaves<T, Metric>()))
           float *list = lists + rit * k;
           unsigned int pending = 0;
           if (row < nA) {
-            const float kth = list[k - 1];
+            const float kth = fminf(list[k - 1], sharedKth[rit]);
             const int self = rowsX ? rowPos[row] : row;
             if constexpr (kFilter) {
               const float limit = metric.accBound(kth);
@@ -263,9 +287,22 @@ __global__ void __launch_bounds__(256, (coreMinWaves<T, Metric>()))
           }
         }
         // The wave's rows are its own: it refreshes their largest k-th itself.
-        if (prune && changed) {
+        const bool share = splits > 1 && (computed & 3) == 0;
+        if (prune && (changed || share)) {
           const int i = wave * kWaveRows + (lane & (kWaveRows - 1));
-          float largest = row0 + i < nA ? lists[i * k + k - 1] : -1.0f;
+          float largest = -1.0f;
+          if (row0 + i < nA) {
+            largest = fminf(lists[i * k + k - 1], sharedKth[i]);
+            if (share && lane < kWaveRows) {
+              const unsigned int bits = __hip_atomic_load(&kthBits[row0 + i], __ATOMIC_RELAXED,
+                                                          __HIP_MEMORY_SCOPE_AGENT);
+              if (__float_as_uint(largest) < bits)
+                atomicMin(&kthBits[row0 + i], __float_as_uint(largest));
+              else
+                largest = __uint_as_float(bits);
+              sharedKth[i] = largest;
+            }
+          }
 #pragma unroll
           for (int m = kWaveRows / 2; m > 0; m >>= 1)
             largest = fmaxf(largest, __shfl_xor(largest, m, 64));
@@ -273,15 +310,61 @@ __global__ void __launch_bounds__(256, (coreMinWaves<T, Metric>()))
             largestKth[wave] = largest;
         }
       }
+      ++computed;
       __syncthreads(); // the tile is consumed, the largest k-th distances are current
     }
     if (prune)
       __syncthreads(); // lowerBound is rewritten by the next batch
   }
   __syncthreads();
+  if (splits > 1) {
+    const size_t first = ((size_t)split * n + row0) * k;
+    for (int e = threadIdx.x; e < T::DIM * k; e += T::THREADS)
+      if (row0 + e / k < nA)
+        partial[first + e] = lists[e];
+    return;
+  }
   for (int i = threadIdx.x; i < T::DIM; i += T::THREADS)
     if (row0 + i < nA)
       core[rowsX ? rowPos[row0 + i] : row0 + i] = lists[i * k + k - 1];
+}
+
+constexpr int kMostCoreSplits = 8;
+
+// The k-th smallest value of a row's ascending lists (one per split, +inf
+// padded), by a thread per row, or the row's last bound: the lists hold every
+// value below it that can be among the k smallest, but not those equal to it.
+__global__ void __launch_bounds__(256)
+    kthOfListsKernel(const float *__restrict__ partial, int splits, int n, int k,
+                     const unsigned int *__restrict__ kthBits, float *__restrict__ core) {
+  const int p = blockIdx.x * blockDim.x + threadIdx.x;
+  if (p >= n)
+    return;
+  const size_t stride = (size_t)n * k;
+  const float *list = partial + (size_t)p * k;
+  float head[kMostCoreSplits];
+  int at[kMostCoreSplits];
+#pragma unroll
+  for (int s = 0; s < kMostCoreSplits; ++s) {
+    at[s] = 0;
+    head[s] = s < splits ? list[s * stride] : INFINITY;
+  }
+  float kth = INFINITY;
+  for (int q = 0; q < k; ++q) {
+    kth = head[0];
+#pragma unroll
+    for (int s = 1; s < kMostCoreSplits; ++s)
+      kth = fminf(kth, head[s]);
+    bool taken = false;
+#pragma unroll
+    for (int s = 0; s < kMostCoreSplits; ++s)
+      if (!taken && s < splits && head[s] == kth) {
+        taken = true;
+        ++at[s];
+        head[s] = at[s] < k ? list[s * stride + at[s]] : INFINITY;
+      }
+  }
+  core[p] = fminf(kth, __uint_as_float(kthBits[p]));
 }
 
 __global__ void coreBoxesKernel(const float *__restrict__ X, int n, int d, int tileDim,
@@ -382,6 +465,41 @@ template <class F> int withMetricCore(MetricSpec m, F &&f) {
   }
 }
 
+// The tiles by the size of their boxes (squared diagonal, to 7 bits of
+// mantissa), largest first.
+__global__ void boxSizeKeysKernel(CoreBoxes boxes, int d, unsigned int *__restrict__ keys,
+                                  int *__restrict__ tiles) {
+  const int t = blockIdx.x * blockDim.x + threadIdx.x;
+  if (t >= boxes.numTiles)
+    return;
+  float sq = 0.0f;
+  for (int f = 0; f < d; ++f) {
+    const float side = boxes.high[(size_t)t * d + f] - boxes.low[(size_t)t * d + f];
+    sq = fmaf(side, side, sq);
+  }
+  keys[t] = 0x7fffu - (__float_as_uint(sq) >> 16);
+  tiles[t] = t;
+}
+
+int sparseFirst(const CoreBoxes &boxes, int tiles, int d, DevArray<int> &order) {
+  DevArray<unsigned int> keys, sorted;
+  DevArray<int> from;
+  DevArray<unsigned char> temp;
+  Status s;
+  s(keys.alloc(tiles));
+  s(sorted.alloc(tiles));
+  s(from.alloc(tiles));
+  s(order.alloc(tiles));
+  s(temp.alloc(sortTempBytes32(tiles)));
+  if (!s.ok())
+    return s.code;
+  hipLaunchKernelGGL(boxSizeKeysKernel, dim3((tiles + 255) / 256), dim3(256), 0, stream(), boxes, d,
+                     keys.get(), from.get());
+  s((int)hipGetLastError());
+  s(radixSortPairs(keys, sorted, from, order, tiles, 15, temp));
+  return s.code;
+}
+
 // tileList (device, numListed entries): only those row tiles.
 int coreFused(const float *X, int n, int d, MetricSpec m, int k, float *core, bool prune,
               int stepLimit = 0x7fffffff, const int *tileList = nullptr, int numListed = 0) {
@@ -404,10 +522,38 @@ int coreFused(const float *X, int n, int d, MetricSpec m, int k, float *core, bo
         boxes = CoreBoxes{low, high, tiles};
         smem += (T::THREADS / 64) * 2 * d * sizeof(float);
       }
+      // Splits: enough workgroups to even out walks of very different lengths
+      // (a resident chip's worth several times over), each with eight column
+      // tiles at least. Without the memory for their lists (at most 130 MiB),
+      // one.
+      int splits = 1;
+      DevArray<unsigned int> kthBits;
+      DevArray<float> partial;
+      DevArray<int> order;
+      const bool whole = boxes.numTiles > 0 && !tileList && stepLimit >= 2 * tiles;
+      if (whole) {
+        splits = std::max(1, std::min({16 * numCUs() / tiles, tiles / 8, kMostCoreSplits}));
+        if (splits > 1 && (kthBits.alloc(n) || partial.alloc((size_t)splits * n * k))) {
+          (void)hipGetLastError();
+          splits = 1;
+        }
+        s(sparseFirst(boxes, tiles, d, order));
+        tileList = order;
+      }
+      if (!s.ok())
+        return s.code;
       PhaseTimer timer(kPhaseCore);
-      hipLaunchKernelGGL((kthNearestFusedKernel<T, Metric>), dim3(tileList ? numListed : tiles),
-                         dim3(256), smem, stream(), X, n, d, metric, k, core, boxes, stepLimit,
-                         nullptr, 0, nullptr, tileList);
+      if (splits > 1)
+        hipLaunchKernelGGL((kthNearestFusedKernel<T, Metric>), dim3(tiles), dim3(256), smem,
+                           stream(), X, n, d, metric, k, reinterpret_cast<float *>(kthBits.get()),
+                           CoreBoxes{}, 1, nullptr, 0, nullptr, nullptr, nullptr, nullptr);
+      hipLaunchKernelGGL((kthNearestFusedKernel<T, Metric>),
+                         dim3(numListed ? numListed : tiles, splits), dim3(256), smem, stream(), X,
+                         n, d, metric, k, core, boxes, stepLimit, nullptr, 0, nullptr, tileList,
+                         kthBits.get(), partial.get());
+      if (splits > 1)
+        hipLaunchKernelGGL(kthOfListsKernel, dim3((n + 255) / 256), dim3(256), 0, stream(),
+                           partial.get(), splits, n, k, kthBits.get(), core);
       s((int)hipGetLastError());
       s(sync());
       return s.code;
@@ -501,7 +647,7 @@ int coreForRowsFused(const float *X, int n, int d, MetricSpec m, int k, const in
       PhaseTimer timer(kPhaseCore);
       hipLaunchKernelGGL((kthNearestFusedKernel<T, Metric>), dim3(rowTiles), dim3(256), smem,
                          stream(), X, n, d, metric, k, core, boxes, 0x7fffffff,
-                         rowData.get(), numRows, rows, nullptr);
+                         rowData.get(), numRows, rows, nullptr, nullptr, nullptr);
       st((int)hipGetLastError());
       st(sync());
       return st.code;

@@ -74,6 +74,25 @@ def test_core_lists_and_select_edges(k, data, pruning):
         _lib.set_pruning("auto")
 
 
+@pytest.mark.parametrize("n, d", [(1920, 3), (1921, 3), (2177, 9), (5003, 3), (8999, 9)])
+@pytest.mark.parametrize("k, metric", [(1, "euclidean"), (25, "euclidean"), (64, "chebyshev")])
+@pytest.mark.parametrize("data", ["lattice", "blobs"])
+def test_pruned_core_walks_in_splits(n, d, k, metric, data):
+    # One walk of a row tile over one (n = 1,920), two, five and eight
+    # workgroups, with many equal distances and with rows whose k nearest lie
+    # in other splits' columns.
+    if data == "lattice":
+        X = np.random.default_rng(n).integers(0, 12, (n, d)).astype(np.float32)
+    else:
+        X = blobs(n_samples=n, n_features=d, centers=5, noise_fraction=0.1, seed=k)
+    _lib.set_pruning("always")
+    try:
+        _, core = hdbscan_tree(X, k, metric=metric, core_method="fused")
+    finally:
+        _lib.set_pruning("auto")
+    np.testing.assert_array_equal(core, oracle.core_distances(X, k, metric=metric))
+
+
 @pytest.mark.parametrize("n_features", [2, 8])
 @pytest.mark.parametrize("k", [1, 5, 40])
 @pytest.mark.parametrize("alpha", [1.0, 0.7, 1.7])
