@@ -409,8 +409,12 @@ int cuhc_device_free(void *ptr) {
     gBuffers.erase(it);
   }
   const int s = (int)hipDeviceSynchronize();
+  if (s) { // perhaps still in use: not for the next call
+    (void)hipFree(ptr);
+    return s;
+  }
   deviceFree(ptr, bytes);
-  return s;
+  return 0;
 }
 
 int cuhc_copy_to_device(void *dst, const void *src, unsigned long long bytes) {
