@@ -107,6 +107,7 @@ __global__ void __launch_bounds__(256, (coreMinWaves<T, Metric>()))
                           const int *__restrict__ rowPos, const int *__restrict__ tileList,
                           unsigned int *__restrict__ kthBits, float *__restrict__ partial) {
   constexpr int TR = T::TR, kWaves = T::THREADS / 64, kWaveRows = T::WAVE_ROWS;
+  static_assert(T::ROWS_BY_WAVE, "a wave's rows are consecutive");
   constexpr int kBatch = 64; // walk steps whose box bounds are computed at once
   __shared__ __align__(16) TileSmem<T> sm;
   // Per wave: the bounds of the batch's steps, the steps within its largest
@@ -506,7 +507,7 @@ int coreFused(const float *X, int n, int d, MetricSpec m, int k, float *core, bo
   return withMetricCore(m, [&](auto metric) {
     using Metric = decltype(metric);
     auto run = [&](auto fill) {
-      using T = typename TileFor<Metric, decltype(fill)::value>::type;
+      using T = typename TileFor<Metric, decltype(fill)::value, true>::type;
       const int tiles = (n + T::DIM - 1) / T::DIM;
       size_t smem = (size_t)T::DIM * k * sizeof(float);
       CoreBoxes boxes;
@@ -627,7 +628,7 @@ int coreForRowsFused(const float *X, int n, int d, MetricSpec m, int k, const in
   return withMetricCore(m, [&](auto metric) {
     using Metric = decltype(metric);
     auto run = [&](auto fill) {
-      using T = typename TileFor<Metric, decltype(fill)::value>::type;
+      using T = typename TileFor<Metric, decltype(fill)::value, true>::type;
       const int rowTiles = (numRows + T::DIM - 1) / T::DIM;
       size_t smem = (size_t)T::DIM * k * sizeof(float);
       CoreBoxes boxes;

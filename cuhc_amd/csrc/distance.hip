@@ -495,7 +495,7 @@ __global__ void __launch_bounds__(256, (!KEEP ? 1 : T::FILL == 8 ? 3 : 2))
                            unsigned long long *__restrict__ kept) {
   constexpr int TR = T::TR, kWaves = T::THREADS / 64, kWaveRows = T::WAVE_ROWS;
   constexpr int kBatch = 64;
-  static_assert(TR == 8 && kWaveRows == 32, "a wave's rows are its lower 32 lanes");
+  static_assert(TR == 8 && kWaveRows == 32 && T::ROWS_BY_WAVE, "a wave's rows are its lower 32 lanes");
   __shared__ unsigned long long rowTop[KEEP ? T::DIM * kKeptKeys : 1];
   // Rows: the full order's tiles, or (COMPACT) the gathered rows, whose
   // position in the full order indexes comp, the weight values, closedRows
@@ -1233,7 +1233,7 @@ int nearestOtherWalk(const float *X, int n, int d, MetricSpec m, WeightSpec w, c
     if (m.id != kSqEuclidean)
       return kErrInvalidMetric;
     return withFill(d, [&](auto fill) {
-      using T = Tile<8, decltype(fill)::value>;
+      using T = Tile<8, decltype(fill)::value, true>;
       return runWalk<T>(X, n, d, SqEuclidean{}, WardWeight{w.size}, comp, orig, compBest,
                         nearest, share, stats, stride, skipComp, closedRows);
     });
@@ -1245,7 +1245,7 @@ int nearestOtherWalk(const float *X, int n, int d, MetricSpec m, WeightSpec w, c
     } else {
       return withWeightFor(metric, w, [&](auto weight) {
         return withFill(d, [&](auto fill) {
-          using T = Tile<8, decltype(fill)::value>;
+          using T = Tile<8, decltype(fill)::value, true>;
           // Closed rows (their answers settled from lists): walk the open rows
           // only.
           if (closedRows && stride == 1)

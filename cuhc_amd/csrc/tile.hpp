@@ -2,12 +2,14 @@
 //
 // A workgroup of 256 threads (4 waves) owns a DIM x DIM tile of the distance
 // matrix, DIM = 16 * TR. Thread t = (tr, tc) = (t / 16, t % 16) owns TR x TR
-// outputs: columns (c / 4) * 64 + 4 tc + c % 4, and of the 4 TR consecutive
-// rows of its wave the rows (r / 4) * 16 + 4 (tr % 4) + r % 4, so that a wave
-// can leave out a tile that none of its rows needs. The 16 threads of one tile
-// row are 16 consecutive lanes of one wave, so row reductions are xor-shuffles
-// inside a 16-lane group, and the 4 threads of a wave that share a column tc
-// are lanes tc, tc+16, tc+32, tc+48.
+// outputs: columns (c / 4) * 64 + 4 tc + c % 4 and the same pattern for rows, or
+// (BY_WAVE) of the 4 TR consecutive rows of its wave the rows (r / 4) * 16 +
+// 4 (tr % 4) + r % 4, so that a wave can leave out a tile that none of its rows
+// needs; passes that compute every tile keep the first form (by wave the
+// symmetric pass spills two registers more: 99,001 points of 90 features 158
+// ms, 165 by wave). The 16 threads of one tile row are 16 consecutive lanes of
+// one wave, so row reductions are xor-shuffles inside a 16-lane group, and the 4
+// threads of a wave that share a column tc are lanes tc, tc+16, tc+32, tc+48.
 //
 // Features are staged in LDS transposed (feature-major, rows padded to DIM + 4
 // floats so the transposed stores spread over the banks) FILL features at a
@@ -21,7 +23,7 @@
 
 namespace cuhc {
 
-template <int TR_, int FILL_> struct Tile {
+template <int TR_, int FILL_, bool BY_WAVE = false> struct Tile {
   static constexpr int TR = TR_;          // outputs per thread side (4 or 8)
   static constexpr int DIM = 16 * TR;     // tile side in points
   static constexpr int FILL = FILL_;      // features staged per LDS fill (multiple of 8)
@@ -32,9 +34,12 @@ template <int TR_, int FILL_> struct Tile {
 
   DEV static int tr() { return threadIdx.x >> 4; }
   DEV static int tc() { return threadIdx.x & 15; }
-  static constexpr int WAVE_ROWS = 4 * TR; // consecutive rows of a wave
+  static constexpr int WAVE_ROWS = 4 * TR; // rows of a wave (consecutive BY_WAVE)
+  static constexpr bool ROWS_BY_WAVE = BY_WAVE;
+  static constexpr int GROUP_STEP = BY_WAVE ? 16 : 64; // rows between groups of 4
   DEV static int rowInTile(int r) {
-    return WAVE_ROWS * (tr() >> 2) + (r >> 2) * 16 + 4 * (tr() & 3) + (r & 3);
+    return (BY_WAVE ? WAVE_ROWS * (tr() >> 2) + 4 * (tr() & 3) : 4 * tr()) +
+           (r >> 2) * GROUP_STEP + (r & 3);
   }
   DEV static int colInTile(int c) { return (c >> 2) * 64 + 4 * tc() + (c & 3); }
 };
@@ -135,7 +140,7 @@ DEV void computeTile(TileSmem<T> &sm, const float *__restrict__ A, int nA,
         float av[TR], bv[TR];
 #pragma unroll
         for (int h = 0; h < TR / 4; ++h) {
-          const float4 a4 = *reinterpret_cast<const float4 *>(&sm.a[k][row4 + h * 16]);
+          const float4 a4 = *reinterpret_cast<const float4 *>(&sm.a[k][row4 + h * T::GROUP_STEP]);
           const float4 b4 = *reinterpret_cast<const float4 *>(&sm.b[k][h * 64 + tc4]);
           av[4 * h + 0] = a4.x; av[4 * h + 1] = a4.y; av[4 * h + 2] = a4.z; av[4 * h + 3] = a4.w;
           bv[4 * h + 0] = b4.x; bv[4 * h + 1] = b4.y; bv[4 * h + 2] = b4.z; bv[4 * h + 3] = b4.w;
@@ -173,8 +178,8 @@ DEV void stageRows(TileSmem<T> &sm, const float *__restrict__ A, int nA, int d, 
 
 // Tile geometry per metric: wide (cosine) accumulators get 4x4 outputs per
 // thread so they stay in registers.
-template <class Metric, int FILL> struct TileFor {
-  using type = Tile<Metric::kWide ? 4 : 8, FILL>;
+template <class Metric, int FILL, bool BY_WAVE = false> struct TileFor {
+  using type = Tile<Metric::kWide ? 4 : 8, FILL, BY_WAVE>;
 };
 
 // Linear index over the upper triangle of tile pairs, t = J (J + 1) / 2 + I

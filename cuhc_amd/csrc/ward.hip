@@ -332,7 +332,7 @@ __global__ void __launch_bounds__(256, 3)
                      const unsigned long long *__restrict__ bound, const RoundState *st,
                      const int *__restrict__ mNow, unsigned long long *__restrict__ partial,
                      unsigned long long *__restrict__ pushed) {
-  using T = Tile<TR_, FILL>;
+  using T = Tile<TR_, FILL, true>;
   constexpr int TR = T::TR, DIM = T::DIM;
   __shared__ __align__(16) TileSmem<T> sm;
   __shared__ unsigned long long top[DIM][kList];
