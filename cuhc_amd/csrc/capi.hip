@@ -10,8 +10,6 @@
 #include <algorithm>
 #include <atomic>
 #include <mutex>
-#include <new>
-#include <unordered_map>
 
 using namespace cuhc;
 
@@ -21,9 +19,6 @@ std::atomic<int> gPruneMode{kPruneAuto};
 std::atomic<int> gPrecision{0};
 std::mutex gStatsMutex;
 PassStats gPruneStats;
-// Sizes of the buffers handed out by cuhc_device_alloc.
-std::mutex gBuffersMutex;
-std::unordered_map<void *, size_t> gBuffers;
 
 bool validLinkageAlgorithm(int linkageId, int algorithmId, int metricId) {
   return algorithmId == kAlgDense || (algorithmId == kAlgMst && linkageId == kSingle) ||
@@ -368,54 +363,13 @@ int cuhc_set_precision(int mode) {
   return 0;
 }
 
-// Callers' buffers come from the library's cache of freed blocks (a fresh 335
-// MB buffer costs 0.4 ms of page mapping, more than the distance matrix that
-// fills it), which is bounded and given back as for the library's own. The
-// library stream may still work on a cached block, and the caller's streams on
-// a freed one: both are waited for, as hipFree waits.
 int cuhc_device_alloc(unsigned long long bytes, void **ptr) {
-  *ptr = nullptr;
-  int s = deviceAlloc(ptr, (size_t)bytes);
-  if (s)
-    return s;
-  s = sync();
-  if (s == 0) {
-    try {
-      std::lock_guard<std::mutex> lock(gBuffersMutex);
-      gBuffers[*ptr] = (size_t)bytes;
-    } catch (const std::bad_alloc &) {
-      s = (int)hipErrorOutOfMemory;
-    }
-  }
-  if (s) {
-    deviceFree(*ptr, (size_t)bytes);
-    *ptr = nullptr;
-  }
-  return s;
+  return callerAlloc(ptr, (size_t)bytes);
 }
 
 void cuhc_release(void) { releaseLibraryState(); }
 
-int cuhc_device_free(void *ptr) {
-  if (!ptr)
-    return 0;
-  size_t bytes = 0;
-  {
-    std::lock_guard<std::mutex> lock(gBuffersMutex);
-    const auto it = gBuffers.find(ptr);
-    if (it == gBuffers.end())
-      return (int)hipFree(ptr); // not one of ours
-    bytes = it->second;
-    gBuffers.erase(it);
-  }
-  const int s = (int)hipDeviceSynchronize();
-  if (s) { // perhaps still in use: not for the next call
-    (void)hipFree(ptr);
-    return s;
-  }
-  deviceFree(ptr, bytes);
-  return 0;
-}
+int cuhc_device_free(void *ptr) { return callerFree(ptr); }
 
 int cuhc_copy_to_device(void *dst, const void *src, unsigned long long bytes) {
   return upload(dst, src, bytes);

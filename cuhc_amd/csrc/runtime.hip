@@ -1,5 +1,6 @@
 #include "runtime.hpp"
 
+#include "caller_buffers.hpp"
 #include "common.hpp"
 
 #include <algorithm>
@@ -98,6 +99,75 @@ void releaseCache(DeviceCache &cache) {
 }
 } // namespace
 
+// Callers' buffers over the HIP runtime. The pool outlives every static object
+// (a buffer may be freed while the process ends); its kept buffers go with
+// releaseLibraryState().
+namespace {
+static_assert(kStatusInvalidValue == (int)hipErrorInvalidValue &&
+                  kStatusOutOfMemory == (int)hipErrorOutOfMemory,
+              "the statuses are HIP's");
+
+struct HipBuffers {
+  int current(int *device) { return (int)hipGetDevice(device); }
+  // An error is returned, and left to no later call.
+  int allocate(void **p, size_t bytes) {
+    const hipError_t e = hipMalloc(p, bytes);
+    if (e != hipSuccess) {
+      *p = nullptr;
+      (void)hipGetLastError();
+    }
+    return (int)e;
+  }
+  int release(void *p) {
+    const hipError_t e = hipFree(p);
+    if (e != hipSuccess)
+      (void)hipGetLastError();
+    return (int)e;
+  }
+  int wait(int device) {
+    int now = 0;
+    Status s;
+    s((int)hipGetDevice(&now));
+    if (s.ok() && now != device)
+      s((int)hipSetDevice(device));
+    if (s.ok())
+      s((int)hipDeviceSynchronize());
+    if (now != device)
+      s((int)hipSetDevice(now));
+    return s.code;
+  }
+  // Whether p is an allocation of at least so many bytes.
+  bool covers(void *p, size_t bytes) {
+    hipDeviceptr_t base = nullptr;
+    size_t size = 0;
+    if (hipMemGetAddressRange(&base, &size, (hipDeviceptr_t)p) != hipSuccess) {
+      (void)hipGetLastError();
+      return false;
+    }
+    return base == (hipDeviceptr_t)p && size >= bytes;
+  }
+  void releaseOther() { releaseCachedBlocks(); }
+  // A 64th of device memory (4.5 GB of 288), so that what a caller has freed is
+  // there for the process's other allocators too.
+  size_t keepLimit() {
+    static const size_t limit = [] {
+      size_t freeBytes = 0, totalBytes = 0;
+      return hipMemGetInfo(&freeBytes, &totalBytes) == hipSuccess ? totalBytes / 64 : (size_t)0;
+    }();
+    return limit;
+  }
+};
+
+CallerBuffers<HipBuffers> &callerBuffers() {
+  static CallerBuffers<HipBuffers> *buffers = new CallerBuffers<HipBuffers>;
+  return *buffers;
+}
+} // namespace
+
+int callerAlloc(void **p, size_t bytes) { return callerBuffers().alloc(p, bytes); }
+
+int callerFree(void *p) { return callerBuffers().free(p); }
+
 namespace {
 struct Workspace {
   char *base = nullptr;
@@ -144,9 +214,10 @@ int deviceAlloc(void **p, size_t bytes) {
     return 0;
   }
   hipError_t e = hipMalloc(p, cls);
-  if (e == hipErrorOutOfMemory && cache.bytes > 0) {
+  if (e == hipErrorOutOfMemory && (cache.bytes > 0 || callerBuffers().keptBytes() > 0)) {
     (void)hipGetLastError();
     releaseCache(cache);
+    callerBuffers().releaseKept();
     e = hipMalloc(p, cls);
   }
   return (int)e;
@@ -182,7 +253,7 @@ void deviceFree(void *p, size_t bytes) {
 size_t cachedDeviceBytes() {
   DeviceCache &cache = deviceCache();
   std::lock_guard<std::mutex> lock(cache.mutex);
-  return cache.bytes;
+  return cache.bytes + callerBuffers().keptBytes();
 }
 
 int upload(void *dst, const void *src, size_t bytes) {
@@ -393,6 +464,7 @@ void releaseCachedBlocks() {
 
 void releaseLibraryState() {
   releaseCachedBlocks();
+  callerBuffers().releaseKept();
   {
     PinnedStage &st = pinnedStage();
     std::lock_guard<std::mutex> lock(st.mutex);

@@ -44,10 +44,14 @@ bool inWorkspace();
 
 // Device memory through the library's cache of freed blocks (runtime.hip).
 // deviceFree takes the size given to deviceAlloc. cachedDeviceBytes: memory
-// held by the cache (free for the library's own use).
+// held by the cache and by callers' freed buffers (free for the library's use).
 int deviceAlloc(void **p, size_t bytes);
 void deviceFree(void *p, size_t bytes);
 size_t cachedDeviceBytes();
+
+// Buffers that callers hold and free (caller_buffers.hpp).
+int callerAlloc(void **p, size_t bytes);
+int callerFree(void *p);
 
 // Owning device allocation.
 template <class T> struct DevArray {
@@ -99,9 +103,9 @@ int featureRanges(const float *X, int n, int d, float *low, float *high);
 int checkFinite(const float *X, size_t count);
 
 // Releases what the library holds between calls: the cached device blocks,
-// the pinned staging buffer and the library stream (recreated on next use).
-// Runs from an exit handler registered when the stream is first created, so
-// that it precedes the HIP runtime's own teardown.
+// callers' freed buffers, the pinned staging buffer and the library stream
+// (recreated on next use). Runs from an exit handler registered when the
+// stream is first created, so that it precedes the HIP runtime's own teardown.
 void releaseLibraryState();
 // Frees the cached device blocks only.
 void releaseCachedBlocks();

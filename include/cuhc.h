@@ -151,8 +151,12 @@ int cuhc_hdbscan_tree_device(const float *deviceX, int n, int d, int metricId, f
 
 /* Device buffers on the library's HIP runtime, for callers that keep inputs
  * resident in HBM across calls (the *_device entry points). Return a status.
- * cuhc_device_alloc releases the library's cache of freed blocks and retries
- * when device memory is short. */
+ * cuhc_device_alloc allocates on the calling thread's current device, and
+ * releases the library's cache of freed blocks and retries when device memory
+ * is short. cuhc_device_free waits for the buffer's device; freeing a buffer a
+ * second time is an error (hipErrorInvalidValue). Freed buffers of up to a 64th
+ * of device memory in all stay with the library for later requests of the same
+ * size; cuhc_release gives them back. */
 int cuhc_device_alloc(unsigned long long bytes, void **ptr);
 int cuhc_device_free(void *ptr);
 int cuhc_copy_to_device(void *dst, const void *src, unsigned long long bytes);
@@ -175,8 +179,9 @@ int cuhc_mfma_probe(int shape, int workgroups, int iters, float *msPerLaunch,
                     double *flopsPerLaunch);
 
 /* Frees what the library keeps between calls: its cache of freed device
- * blocks, the pinned staging buffer and its HIP stream (recreated on the next
- * call). Also runs from an exit handler, before the HIP runtime's teardown. */
+ * blocks, callers' freed buffers, the pinned staging buffer and its HIP stream
+ * (recreated on the next call). Also runs from an exit handler, before the HIP
+ * runtime's teardown. */
 void cuhc_release(void);
 
 /* Per-phase GPU timing with HIP events on the library stream (0 = off).
