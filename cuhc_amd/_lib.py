@@ -76,6 +76,7 @@ _declare("cuhc_set_timing", _int, _int)
 _declare("cuhc_read_timings", None, _f64p, _i64p, _i64p, _int)
 _declare("cuhc_reset_timings", None)
 _declare("cuhc_release", None)
+_declare("cuhc_set_allocation_limit", None, ctypes.c_ulonglong)
 _declare("cuhc_mixed_stats", None, _u64p, _u64p, _u64p, _u64p)
 _declare("cuhc_learned_stats", None, _u64p, _u64p, _u64p, _u64p, _u64p, _u64p, _u64p)
 _declare("cuhc_set_learned_training", _int, _int)

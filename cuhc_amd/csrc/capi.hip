@@ -60,7 +60,9 @@ constexpr int kLearnedAutoMaxK = 128;
 // lists where the pass is not pruned: the select reads every row's distances
 // four times (0.05 ms for 2,003 points, 0.9 for 12,000, 3.3 for 24,000,
 // whatever k), the lists insert row by row on few workgroups (k = 25: 0.96,
-// 2.2 and 3.6 ms; k = 5: 0.38, 1.2 and 2.1; k = 60: 2.0, 3.9 and 6.2).
+// 2.2 and 3.6 ms; k = 5: 0.38, 1.2 and 2.1; k = 60: 2.0, 3.9 and 6.2). Its rows
+// take 4 n bytes each (all n of them, if a quarter of the free memory holds
+// them); the lists remain the way without that memory.
 constexpr int radixAutoPoints(int k) { return 14000 + 350 * k; }
 
 int linkageImpl(const float *X, bool onDevice, int n, int d, int metricId, float metricParam,
@@ -156,7 +158,7 @@ int hdbscanImpl(const float *X, bool onDevice, int n, int d, int metricId, float
   if (s.ok())
     s(decidePruning(pts, n, d, m, prune));
   if (coreMethod == kCoreAuto && method == kCoreFused && !prune && n <= radixAutoPoints(minSamples))
-    method = kCoreRadix;
+    method = kCoreRadixElseFused;
   PassStats stats;
   if (s.ok()) {
     if (n == 1) {
@@ -366,6 +368,8 @@ int cuhc_set_precision(int mode) {
 int cuhc_device_alloc(unsigned long long bytes, void **ptr) {
   return callerAlloc(ptr, (size_t)bytes);
 }
+
+void cuhc_set_allocation_limit(unsigned long long bytes) { setAllocationLimit((size_t)bytes); }
 
 void cuhc_release(void) { releaseLibraryState(); }
 

@@ -720,7 +720,12 @@ int coreDistances(const float *X, int n, int d, MetricSpec m, int k, float *core
     return coreLearned(X, n, d, m, k, core, prune);
   if (method == kCoreFused || (method == kCoreAuto && k <= kMaxFusedK))
     return coreFused(X, n, d, m, k, core, prune);
-  return coreRadix(X, n, d, m, k, core);
+  const int status = coreRadix(X, n, d, m, k, core);
+  if (method == kCoreRadixElseFused && status == (int)hipErrorOutOfMemory) {
+    (void)hipGetLastError();
+    return coreFused(X, n, d, m, k, core, prune);
+  }
+  return status;
 }
 
 } // namespace cuhc

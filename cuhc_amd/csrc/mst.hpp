@@ -107,7 +107,15 @@ int boruvkaMst(const float *X, int n, int d, MetricSpec m, WeightSpec w, const M
 // kCoreLearned (an extension): radius proposals from the trained network seed
 // the pruned gather and a radix select; rows whose proposal fails fall back to
 // the exact full search. All methods give identical values.
-enum CoreMethod : int { kCoreAuto = 0, kCoreFused = 1, kCoreRadix = 2, kCoreLearned = 3 };
+// kCoreRadixElseFused (chosen by auto only, k <= kMaxFusedK): the radix select,
+// or without the memory for its rows of distances the fused lists, which need none.
+enum CoreMethod : int {
+  kCoreAuto = 0,
+  kCoreFused = 1,
+  kCoreRadix = 2,
+  kCoreLearned = 3,
+  kCoreRadixElseFused = 4,
+};
 constexpr int kMaxFusedK = 64;
 int coreDistances(const float *X, int n, int d, MetricSpec m, int k, float *core, int method,
                   bool prune);

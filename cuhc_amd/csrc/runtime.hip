@@ -192,7 +192,17 @@ WorkspaceScope::~WorkspaceScope() {
 
 bool inWorkspace() { return tWorkspace != nullptr; }
 
+namespace {
+thread_local size_t tAllocationLimit = 0;
+}
+
+void setAllocationLimit(size_t bytes) { tAllocationLimit = bytes; }
+
 int deviceAlloc(void **p, size_t bytes) {
+  if (tAllocationLimit && bytes > tAllocationLimit) {
+    *p = nullptr;
+    return (int)hipErrorOutOfMemory;
+  }
   if (Workspace *w = tWorkspace) {
     const size_t want = sliceBytes(bytes);
     if (want > w->bytes - w->used) {

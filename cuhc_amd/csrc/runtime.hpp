@@ -48,6 +48,9 @@ bool inWorkspace();
 int deviceAlloc(void **p, size_t bytes);
 void deviceFree(void *p, size_t bytes);
 size_t cachedDeviceBytes();
+// deviceAlloc refuses larger requests of the calling thread as out of memory
+// (0: none). For tests of what runs without memory.
+void setAllocationLimit(size_t bytes);
 
 // Buffers that callers hold and free (caller_buffers.hpp).
 int callerAlloc(void **p, size_t bytes);

@@ -178,6 +178,10 @@ int cuhc_copy_device(void *dst, const void *src, unsigned long long bytes);
 int cuhc_mfma_probe(int shape, int workgroups, int iters, float *msPerLaunch,
                     double *flopsPerLaunch);
 
+/* Test hook: the library's own allocations above so many bytes fail as out of
+ * memory on the calling thread (0, the default: none does). */
+void cuhc_set_allocation_limit(unsigned long long bytes);
+
 /* Frees what the library keeps between calls: its cache of freed device
  * blocks, callers' freed buffers, the pinned staging buffer and its HIP stream
  * (recreated on the next call). Also runs from an exit handler, before the HIP

@@ -202,3 +202,20 @@ def test_pruned_large_blobs_and_noise_identical(metric, k, alpha):
             _lib.set_pruning("auto")
     np.testing.assert_array_equal(out["always"][1], out["never"][1])
     np.testing.assert_array_equal(out["always"][0], out["never"][0])
+
+
+@pytest.mark.parametrize("metric", ["euclidean", "cosine"])
+def test_default_core_pass_without_memory_for_distance_rows(metric):
+    # auto takes the radix select for few unpruned points; where its rows of
+    # distances (36 MB) find no memory, the fused lists give the same values.
+    X = blobs(n_samples=3000, n_features=5, seed=6)
+    Z, core = hdbscan_tree(X, 12, metric=metric)
+    _lib.lib.cuhc_set_allocation_limit(8 << 20)
+    try:
+        Zl, cl = hdbscan_tree(X, 12, metric=metric)
+        with pytest.raises(RuntimeError, match="memory"):  # asked for by name: refused as before
+            hdbscan_tree(X, 12, metric=metric, core_method="radix")
+    finally:
+        _lib.lib.cuhc_set_allocation_limit(0)
+    np.testing.assert_array_equal(cl, core)
+    np.testing.assert_array_equal(Zl, Z)
