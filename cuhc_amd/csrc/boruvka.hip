@@ -101,14 +101,18 @@ int boruvkaMst(const float *X, int n, int d, MetricSpec m, WeightSpec w, const M
   // Without lists, the first round's walk keeps each row's 4 smallest keys over
   // all other points, and the later rounds' rows settle from them: whatever
   // share of the tiles that walk computes, it replaces most of the later
-  // rounds' passes.
-  const bool keepKeys = !useLists && opt.prune;
+  // rounds' passes. Without the memory for them (33 bytes a point) the rounds
+  // walk every row or, past the give-up share, compute every pair once.
+  bool keepKeys = !useLists && opt.prune;
   DevArray<unsigned char> dClosed;
   DevArray<unsigned long long> dListCounters, dKept;
-  if (useLists || keepKeys)
+  if (useLists)
     s(dClosed.alloc(n));
-  if (keepKeys)
-    s(dKept.alloc((size_t)n * 4));
+  if (keepKeys && (dKept.alloc((size_t)n * 4) || dClosed.alloc(n))) {
+    (void)hipGetLastError();
+    dKept.release();
+    keepKeys = false;
+  }
   if (useLists) {
     s(dListCounters.alloc(64 * 16));
     if (s.ok())

@@ -1071,12 +1071,13 @@ int runWalk(const float *X, int n, int d, const Metric &metric, const Weight &we
     bool launched = false;
     if constexpr (Weight::kDistBound) { // not Ward's, which keeps its own lists
       if (kept) {
-        const int splits = walkSplits(sampled, tiles, kKeptSplits, 0x7fffffff);
+        // Without the memory for the splits' lists, one split.
+        int splits = walkSplits(sampled, tiles, kKeptSplits, 0x7fffffff);
         DevArray<unsigned long long> lists;
-        if (splits > 1)
-          s(lists.alloc((size_t)splits * n * kKeptKeys));
-        if (!s.ok())
-          return s.code;
+        if (splits > 1 && lists.alloc((size_t)splits * n * kKeptKeys)) {
+          (void)hipGetLastError();
+          splits = 1;
+        }
         hipLaunchKernelGGL((nearestOtherWalkKernel<T, Metric, Weight, false, true>),
                            dim3(sampled, splits), dim3(256), walkBoxBytes<T>(d), stream(), X, n, d,
                            metric, weight, comp, orig, boxes.view, nullptr, nearest,

@@ -295,3 +295,19 @@ def test_pruned_large_clustered_identical(metric):
                         for c, s in zip(centres, rng.uniform(0.2, 3.0, 25))]).astype(np.float32)
     np.testing.assert_array_equal(run(X, metric, pruning="always"),
                                   run(X, metric, pruning="never"))
+
+
+@pytest.mark.parametrize("limit", [200_000, 90_000])
+@pytest.mark.parametrize("metric", ["euclidean", "manhattan"])
+def test_pruned_rounds_without_memory_for_kept_keys(metric, limit):
+    # 3,000 points keep 96,000 bytes of keys, and three times that while the
+    # keeping walk runs in three splits: without the larger one walk keeps them,
+    # without either the rounds run on nothing kept. Every other request is
+    # below 40,000 bytes.
+    X = blobs(n_samples=3000, n_features=3, centers=9, noise_fraction=0.1, seed=3)
+    _lib.lib.cuhc_set_allocation_limit(limit)
+    try:
+        Z = run(X, metric, pruning="always")
+    finally:
+        _lib.lib.cuhc_set_allocation_limit(0)
+    np.testing.assert_array_equal(Z, oracle.single_linkage(X, metric))
