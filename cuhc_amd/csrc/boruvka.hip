@@ -119,6 +119,10 @@ int boruvkaMst(const float *X, int n, int d, MetricSpec m, WeightSpec w, const M
       s(fill(dListCounters, 0, dListCounters.bytes()));
   }
   bool keptValid = false; // dKept holds the first round's lists
+  // Of the tile pairs, computed by the walk that kept them. Plain weights only:
+  // under mutual reachability the later walks leave out more than that one did
+  // (HDBSCAN of 100,000 x 14 normal points 46.8 ms, by this share 49.1).
+  double keptShare = 0.0;
   if (s.ok())
     s(resetComponents(dComp, n));
   MixedPass *mixed = nullptr;
@@ -168,13 +172,19 @@ int boruvkaMst(const float *X, int n, int d, MetricSpec m, WeightSpec w, const M
           s(nearestOtherWalk(X, n, d, m, w, dComp, opt.devOrig, nullptr, dNearest, &share,
                              opt.stats, 1, dSkip, nullptr, dKept));
           keptValid = true;
+          keptShare = w.kind == kWeightPlain ? share : 0.0;
           share = 0.0; // the next rounds walk the rows that the keys leave open
         } else {
           if (keepKeys)
             s(settleFromKept(dKept, n, dComp, posOf, dSkip, dNearest, dCompBest, dClosed));
           s(nearestOtherWalk(X, n, d, m, w, dComp, opt.devOrig, dCompBest, dNearest, &share,
                              opt.stats, 1, dSkip,
-                             useLists || keepKeys ? dClosed.get() : nullptr));
+                             useLists || keepKeys ? dClosed.get() : nullptr, nullptr,
+                             keptShare));
+          if (s.ok() && share < 0.0) { // too many open rows: every pair, once
+            s(nearestOtherSymmetric(X, n, d, m, w, dComp, opt.devOrig, dNearest));
+            share = 0.0; // the next round's open rows decide again
+          }
         }
         pruneThisPass = share <= kPruneGiveUpShare;
       } else {

@@ -1148,7 +1148,7 @@ template <class T, class Metric, class Weight>
 int runWalkOpen(const float *X, int n, int d, const Metric &metric, const Weight &weight,
                 const int *comp, const int *orig, unsigned int *compBest,
                 unsigned long long *nearest, double *share, PassStats *stats,
-                const int *skipComp, const unsigned char *closedRows) {
+                const int *skipComp, const unsigned char *closedRows, double keptShare) {
   const int tiles = (n + T::DIM - 1) / T::DIM;
   Status s;
   DevArray<int> flags, index, rowPos;
@@ -1167,6 +1167,13 @@ int runWalkOpen(const float *X, int n, int d, const Metric &metric, const Weight
   s(download(&nOpen, index.get() + n, sizeof(int)));
   if (!s.ok())
     return s.code;
+  // A walk of every row that leaves out few pairs takes 2.3 symmetric passes
+  // (92,000 points of 60 features in blobs, manhattan: 33 and 13.3 ms; whole
+  // calls 92.8 ms with the walks alone, 73.5 with this rule).
+  if (keptShare * nOpen > 0.5 * n) {
+    *share = -1.0;
+    return 0;
+  }
   if (4LL * nOpen > 3LL * n) // most rows open: the full order's tiles
     return runWalk<T>(X, n, d, metric, weight, comp, orig, compBest, nearest, share, stats, 1,
                       skipComp, closedRows);
@@ -1225,7 +1232,8 @@ int runWalkOpen(const float *X, int n, int d, const Metric &metric, const Weight
 int nearestOtherWalk(const float *X, int n, int d, MetricSpec m, WeightSpec w, const int *comp,
                      const int *orig, unsigned int *compBest, unsigned long long *nearest,
                      double *share, PassStats *stats, int stride, const int *skipComp,
-                     const unsigned char *closedRows, unsigned long long *kept) {
+                     const unsigned char *closedRows, unsigned long long *kept,
+                     double keptShare) {
   if (!metricHasBoxBound(m.id))
     return kErrInvalidMetric;
   if (kept && (w.kind == kWeightWard || closedRows || stride != 1))
@@ -1251,7 +1259,7 @@ int nearestOtherWalk(const float *X, int n, int d, MetricSpec m, WeightSpec w, c
           // only.
           if (closedRows && stride == 1)
             return runWalkOpen<T>(X, n, d, metric, weight, comp, orig, compBest, nearest, share,
-                                  stats, skipComp, closedRows);
+                                  stats, skipComp, closedRows, keptShare);
           return runWalk<T>(X, n, d, metric, weight, comp, orig, compBest, nearest, share,
                             stats, stride, skipComp, closedRows, kept);
         });

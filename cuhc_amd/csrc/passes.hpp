@@ -95,11 +95,14 @@ struct PassStats {
 // rows or sampling): every row also keeps its 4 smallest keys over
 // the other components (ascending, empty keys ~0 padded), searched without
 // the component bounds, for settling rows in later rounds.
+// keptShare (with closed rows): the share of the tile pairs that the keeping
+// walk computed. Where the open rows' walk would compute more pairs than
+// nearestOtherSymmetric at that share, it computes none: *share = -1.
 int nearestOtherWalk(const float *X, int n, int d, MetricSpec m, WeightSpec w, const int *comp,
                      const int *orig, unsigned int *compBest, unsigned long long *nearest,
                      double *share, PassStats *stats, int rowTileStride = 1,
                      const int *skipComp = nullptr, const unsigned char *closedRows = nullptr,
-                     unsigned long long *kept = nullptr);
+                     unsigned long long *kept = nullptr, double keptShare = 0.0);
 
 // Rows settled from the 4 keys each row kept in an earlier round (kept, by
 // position; keys carry original indices, posOf maps them to positions, null:

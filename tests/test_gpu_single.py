@@ -311,3 +311,19 @@ def test_pruned_rounds_without_memory_for_kept_keys(metric, limit):
     finally:
         _lib.lib.cuhc_set_allocation_limit(0)
     np.testing.assert_array_equal(Z, oracle.single_linkage(X, metric))
+
+
+@pytest.mark.parametrize("n, d", [(2000, 12), (6000, 40)])
+@pytest.mark.parametrize("metric", ["manhattan", "chebyshev"])
+def test_rounds_that_walk_too_many_rows(n, d, metric):
+    # Blobs among noise whose boxes leave out few pairs: after the noise, most
+    # rows are open again, and their round computes every pair once instead of
+    # walking them. The walks compute the keeping one's tiles (all of them at
+    # most) and half as many again in a later one; with that round's walk it
+    # were twice as many and more.
+    X = blobs(n_samples=n, n_features=d, centers=20, noise_fraction=0.1, seed=d)
+    _lib.prune_stats()
+    Z = run(X, metric, pruning="always")
+    computed, _ = _lib.prune_stats()
+    np.testing.assert_array_equal(Z, oracle.single_linkage(X, metric))
+    assert computed < 1.75 * ((n + 127) // 128) ** 2
