@@ -327,3 +327,52 @@ def test_rounds_that_walk_too_many_rows(n, d, metric):
     computed, _ = _lib.prune_stats()
     np.testing.assert_array_equal(Z, oracle.single_linkage(X, metric))
     assert computed < 1.75 * ((n + 127) // 128) ** 2
+
+
+def pruned_share(X, metric="euclidean"):
+    _lib.prune_stats()
+    run(X, metric, pruning="always")
+    computed, total = _lib.prune_stats()
+    return computed / total
+
+
+@pytest.mark.parametrize("value", [1e6, 1e15])
+@pytest.mark.parametrize("columns", [1, 4])
+def test_sentinel_values_leave_the_order_its_levels(columns, value):
+    # 3% of the rows hold a far value in each of the columns (at most 12% of the
+    # rows): the others' ranges still split where they would without, so the
+    # walks compute about the tiles that they compute without those values, and
+    # those of the rows that hold them.
+    rng = np.random.default_rng(7)
+    X = rng.uniform(size=(30_000, 4)).astype(np.float32)
+    far = X.copy()
+    for f in range(columns):
+        far[rng.choice(len(X), 900, replace=False), f] = value
+    near, with_far = pruned_share(X), pruned_share(far)
+    print(columns, value, near, with_far)
+    assert with_far < 2 * near + 0.03 * columns
+
+
+def test_spread_beyond_float32_leaves_the_order_its_levels():
+    # Two points whose difference overflows: the ABI takes them where a spanning
+    # tree of finite distances exists (the Python surface refuses them). All
+    # others prune as they do without those two.
+    n, chebyshev = 20_000, 3
+    X = np.random.default_rng(9).uniform(size=(n, 2)).astype(np.float32)
+
+    def tree(pruning):
+        Z = np.empty((n - 1, 4))
+        _lib.set_pruning(pruning)
+        _lib.prune_stats()
+        try:
+            _lib.check(_lib.lib.cuhc_linkage(_lib.float_ptr(X), n, 2, chebyshev, 2.0, 0, 1,
+                                             _lib.double_ptr(Z)))
+        finally:
+            _lib.set_pruning("auto")
+        return Z, _lib.prune_stats()
+
+    _, (near, total) = tree("always")
+    X[:2] = [[-3e38, 0], [3e38, 0]]
+    Z, (computed, _) = tree("always")
+    np.testing.assert_array_equal(Z, tree("never")[0])
+    assert computed < 1.5 * near
