@@ -117,7 +117,7 @@ void releaseCachedBlocks();
 // cuhc_set_timing(1) turns it on. A phase is bracketed by begin()/end(); the
 // elapsed time is collected at the next collect() (after a stream sync).
 enum Phase : int {
-  kPhaseDistanceTiles = 0,  // FP32 direct-form all-pairs passes (Boruvka, Ward)
+  kPhaseDistanceTiles = 0,  // FP32 direct-form passes (Boruvka's rounds, Ward's searches)
   kPhaseMfmaCandidates = 1, // FP16 MFMA candidate pass
   kPhaseRecheck = 2,        // FP32 recheck of certified candidates
   kPhaseCore = 3,           // core distances

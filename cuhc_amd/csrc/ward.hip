@@ -75,6 +75,7 @@ struct RoundState {
   int searches; // rows of the current search
   int stop;     // a round fell below the wanted progress: queued rounds do nothing
   int rounds;   // rounds done
+  unsigned long long pairs; // weights computed by the searches
 };
 
 struct Lists {
@@ -522,13 +523,15 @@ __global__ void __launch_bounds__(256)
     wardFinishKernel(Lists lists, const int *__restrict__ searchOf,
                      const unsigned long long *__restrict__ partial,
                      const unsigned long long *__restrict__ pushed,
-                     const int *__restrict__ mNow, const RoundState *st, int dim) {
+                     const int *__restrict__ mNow, RoundState *st, int dim) {
   if (roundOver(st))
     return;
   const int m = *mNow, i = (int)((blockIdx.x * blockDim.x + threadIdx.x) / 16);
   if (i >= m)
     return;
   const int sub = threadIdx.x & 15;
+  if (i == 0 && sub == 0)
+    st->pairs += (unsigned long long)st->searches * (unsigned long long)m;
   unsigned long long *list = lists.keys + (size_t)i * kList;
   const int place = searchOf[i];
   unsigned long long key[kList];
@@ -584,7 +587,7 @@ __global__ void __launch_bounds__(256)
 }
 
 __global__ void roundStartKernel(RoundState *st, int n) {
-  *st = RoundState{n, 0, 0, 0, 0};
+  *st = RoundState{n, 0, 0, 0, 0, 0};
 }
 
 // Every point its own cluster; rep = its original index (orig, null: the
@@ -1059,7 +1062,7 @@ int rnnWard(const float *X, int n, int d, const RnnOptions &opt, double *tree) {
   }
   s((int)hipGetLastError());
 
-  RoundState host{n, 0, 0, 0, 0};
+  RoundState host{n, 0, 0, 0, 0, 0};
   int queued = 0; // rounds queued so far
   enum { kNone, kDense, kChain } tail = kNone;
   while (s.ok() && host.m > 1) {
@@ -1113,6 +1116,11 @@ int rnnWard(const float *X, int n, int d, const RnnOptions &opt, double *tree) {
       tail = opt.allowDense && wardMatrixFits(host.m) ? kDense : kChain;
       break;
     }
+  }
+  if (s.ok() && timingEnabled()) {
+    RoundState end{};
+    s(download(&end, state, sizeof(end)));
+    addUnits(kPhaseDistanceTiles, (long long)end.pairs);
   }
   // Queued rounds after the last swapped the buffers for nothing.
   if ((queued - host.rounds) & 1)

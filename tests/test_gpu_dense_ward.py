@@ -220,3 +220,19 @@ def test_rnn_pruned_equals_unpruned(n_features):
     print(n_features, stats)
     assert 0 < computed < total  # some tile pairs were skipped
     assert stats["never"] == (0, 0)
+
+
+def test_ward_searches_count_their_pairs():
+    # The first search takes all rows against all columns; the later ones some.
+    from cuhc_amd import _lib
+    n = 3000
+    X = np.random.default_rng(2).normal(size=(n, 5)).astype(np.float32)
+    _lib.set_timing(True)
+    try:
+        _lib.reset_timings()
+        cuhc.linkage(X, method="ward", algorithm="rnn")
+        ms, launches, pairs = _lib.read_timings()["distance_tiles"]
+    finally:
+        _lib.set_timing(False)
+    assert ms > 0 and launches > 1
+    assert n * n < pairs < n * n * launches
