@@ -376,3 +376,13 @@ def test_spread_beyond_float32_leaves_the_order_its_levels():
     Z, (computed, _) = tree("always")
     np.testing.assert_array_equal(Z, tree("never")[0])
     assert computed < 1.5 * near
+
+
+@pytest.mark.parametrize("metric", ["manhattan", "chebyshev"])
+def test_chain_of_600_000_hooks(metric):
+    # Points one apart on a line: in the first round every point hooks onto the
+    # one before it. The climb's limit has a slack that covers 262,144 hooks.
+    n = 600_000
+    Z = run(np.arange(n, dtype=np.float32)[:, None], metric)
+    np.testing.assert_array_equal(Z[:, 2], 1.0)
+    np.testing.assert_array_equal(Z[:, 3], np.arange(2, n + 1))
