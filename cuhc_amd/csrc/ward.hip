@@ -6,9 +6,9 @@
 // them in FP64 (c_a + (c_b - c_a) * n_b / (n_a + n_b), exact for duplicate
 // centroids); merge heights are accumulated in FP64,
 // sqrt(2 n_a n_b / (n_a + n_b) * sum (c_a - c_b)^2). The RNN rounds choose
-// nearest neighbours with the FP32 all-pairs pass on an FP32 copy of the
-// centroids and Ward's FP32 weight (symmetric bit for bit, so the closest
-// pair always sees each other and every round makes progress).
+// nearest neighbours by FP32 searches of an FP32 copy of the centroids and
+// Ward's FP32 weight (symmetric bit for bit, so the closest pair always sees
+// each other and every round makes progress).
 #include "linkage.hpp"
 #include "mst.hpp"
 #include "primitives.hpp"
@@ -55,8 +55,9 @@ struct DevMerge {
 // nearest, ties included, is the one a pass over all pairs would find.
 //
 // Bound by FP32 VALU work at large m, by launches and dependent waits at small:
-// the component count stays on the device, so that rounds are queued several
-// at a time, each of 5 launches (7 above 4,096 clusters), without a host read.
+// the cluster count stays on the device, so that rounds are queued several at a
+// time without a host read, each of 4 launches (up to 8,192 clusters; 8 above,
+// three of them the scan that numbers the survivors).
 // A pass over all pairs per round and its read took 4.3 ms for 3,001 points of
 // 13 features (55 rounds) and 99 ms for 100,000 of 32 (95 rounds); now 2.6 and
 // 61 ms.
@@ -288,7 +289,8 @@ __global__ void searchAllKernel(int n, unsigned int *searchRows, int *searchOf,
     st->searches = n;
 }
 
-// Lists from an exact pass that kept `per` lowest keys of every point.
+// Lists from an exact pass that kept `per` lowest keys of every point: each
+// list's bound is the last of them that it takes.
 __global__ void listsFromKeysKernel(const unsigned long long *__restrict__ keys, int per, int n,
                                     Lists lists) {
   const int i = blockIdx.x * blockDim.x + threadIdx.x;
@@ -296,7 +298,7 @@ __global__ void listsFromKeysKernel(const unsigned long long *__restrict__ keys,
     return;
   for (int q = 0; q < kList; ++q)
     lists.keys[(size_t)i * kList + q] = q < per ? keys[(size_t)i * per + q] : kEmptyKey;
-  lists.bound[i] = keys[(size_t)i * per + per - 1];
+  lists.bound[i] = keys[(size_t)i * per + min(per, kList) - 1];
 }
 
 // Minimum over the 16 lanes of a tile row, in all of them (DPP row rotations).
