@@ -12,8 +12,9 @@
 // values (missing entries coded as 1e9, say) must not take the steps from those
 // around the middle, which alone count: with steps over the whole sample's spread
 // the walks over 30,000 points of 4 features, 3% of the rows at 1e6 in each,
-// computed 24% of the tiles, now 9%, and 5% without those values. A range is named by its path (a bit per level), which orders
-// ranges as they lie and needs no more bits than there are levels.
+// computed 24% of the tiles, now 9%, and 5% without those values. A range is
+// named by its path (a bit per level), which orders ranges as they lie and needs
+// no more bits than there are levels.
 // Bound by launches up to some 10^5 points, then by the sorts' passes. With the
 // order made on the host (16 threads; points on the device were copied there
 // first) whole calls took: single linkage, manhattan, 50,021 x 10, 18.9 ms, now
