@@ -16,8 +16,9 @@
 // fn: rows with fn in {a, b} are rescanned unless the merged distance is still
 // the row's minimum; row a's new fn is the minimum of its new distances.
 //
-// The merge loop is one cooperative persistent kernel (one workgroup per CU)
-// that makes up to kMaxBatch merges per two grid barriers.
+// The merge loop is a cooperative persistent kernel (one workgroup per CU)
+// that makes up to kMaxBatch merges per two grid barriers, or, where few merges
+// of a batch stand, another that makes one per barrier (denseChainKernel).
 // Workgroup g owns a contiguous range of slots (rows): their fn, size, bound
 // and pending flag live in its LDS, it alone writes D(k, a) / D(a, k) for its
 // rows k, and every workgroup keeps the active flags of all slots as a bitmask
@@ -64,6 +65,7 @@ constexpr int kChunk = 8192;                     // columns per initial-scan wor
 constexpr int kWaves = kThreads / 64;
 constexpr int kRescanCols = 1024;                // columns per rescan work item (one wave)
 constexpr int kRescanPer = kRescanCols / 64;
+constexpr int kScanPer = 16;                     // columns per thread and step of a lone row's scan
 constexpr int kMaxOwned = 2048;                  // rows per workgroup (LDS row state)
 constexpr int kUpdatePer = 4;                    // owned rows per lane per load batch
 constexpr int kMaxBatch = 16;                    // merges per batch
@@ -71,6 +73,14 @@ constexpr int kMinGroups = 8;                    // workgroups of the merge kern
 constexpr int kTop = 4;                          // lowest rows carried in a record
 constexpr int kInlineRows = 6;                   // pending rows carried in a record
 constexpr int kRecordWords = 12;                 // u64 words per workgroup record (96 bytes)
+constexpr int kStepWords = 6;                    // the same of a single merge (48 bytes)
+// A running average of the merges that stand per batch (the last 16 or so): the
+// batch loop is left for single merges below kFewStand. Batches take 25 to 30 us
+// and single merges 7 to 14 (n = 2,000 to 30,000). Runs of single merges start at
+// kFirstRun and double while the batches between them make fewer merges than
+// that; the average starts low after a run, so that the try is short.
+constexpr float kFewStand = 2.0f, kFirstAverage = 4.0f, kNextAverage = 2.5f;
+constexpr int kFirstRun = 256, kLongestRun = 4096;
 constexpr int kGroup = 16;                       // workgroups per first-level barrier counter
 constexpr int kLineWords = 32;                   // one 128-byte line in 32-bit words
 constexpr unsigned int kSpinLimit = 1u << 22;    // barrier polls (seconds) before aborting
@@ -169,16 +179,28 @@ DEV bool gridBarrier(const Barrier &bar, unsigned int &generation, int *ok) {
   return *ok != 0;
 }
 
+// At a kernel's start, before its first barrier: the generation that the last
+// kernel left, and whether one of its waits gave up.
+DEV unsigned int barrierGeneration(const Barrier &bar) {
+  return __hip_atomic_load(bar.words, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+}
+DEV bool barrierAborted(const Barrier &bar) {
+  return __hip_atomic_load(bar.words + kLineWords, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT) != 0;
+}
+
 struct DenseState {
   float *D;
   int n;
   int firstNewId;
   int per;   // rows per workgroup
   int batch; // merges per batch (at most kMaxBatch)
+  float average; // merges per batch that the batch loop starts from
   int *size; // cluster size and scipy id by slot
   int *id;
   // Per slot, [2][n]: the forward nearest key and the second lowest key of
   // the row, from denseInitKernel and, while a row is pending, from its rescan.
+  // Between the kernels of the merge loop every row's, a pending one's nearest
+  // empty and its bound in the other's place.
   unsigned long long *scanned;
   // One record per workgroup (kRecordWords words): [0..3] its kTop lowest
   // selection keys, [4..5] their fn columns, [6] the lowest lower-bound key of
@@ -188,6 +210,13 @@ struct DenseState {
   // the first half of the next, so a barrier lies between any write and read.
   unsigned long long *records;
   int *pendingRows;
+  // Single merges: one record of kStepWords words per workgroup, in two buffers
+  // that alternate by merge (a barrier lies between): its lowest selection key,
+  // that key's column, the two lowest keys of its part of row a, and the lowest
+  // lower-bound key of its pending rows.
+  unsigned long long *steps; // [2][G][kStepWords]
+  unsigned int *active;      // between the kernels: bit j = slot j active
+  int *done;                 // between the kernels: merges made
   // Per merge of the batch and workgroup, [kMaxBatch][G]: the two lowest keys
   // of its part of row a, and the ordered bits of its smallest new distance.
   // Written in the first half, read in the second.
@@ -308,6 +337,8 @@ DEV void waveSync() {
 // (64-byte lines around scattered 4-byte entries) at large n. One merge per
 // barrier took 14.0 us per merge at n = 5,003 and 15.8 us at n = 100,000;
 // batches take 2.2 us (437 batches of 25 us) and 5.8 us.
+// Where few merges of a batch stand it hands over to denseChainKernel; a form
+// that limited its batches to one merge instead kept both barriers and halves.
 // Keeping a bound below a row's other keys beside its fn (instead of its old
 // fn as a pending row's bound) took n = 5,003 from 610 batches to 437: fewer
 // selections meet a pending row. One instantiation per linkage, short loops
@@ -344,7 +375,7 @@ __global__ void __launch_bounds__(kThreads) denseMergeKernel(DenseState s) {
   __shared__ unsigned long long rowFn[kMaxBatch], rowNext[kMaxBatch];
   __shared__ unsigned int newMin[kMaxBatch];
   __shared__ int batchCount; // merges in the batch, or -1: no pair is left
-  __shared__ unsigned long long waveKey[3 * kWaves];
+  __shared__ unsigned long long waveKey[2 * kWaves];
   __shared__ int waveInt[2 * kWaves];
   __shared__ __align__(16) unsigned long long topKey[kWaves * kTop];
   __shared__ int barrierOk;
@@ -358,7 +389,10 @@ __global__ void __launch_bounds__(kThreads) denseMergeKernel(DenseState s) {
   float *newDist = reinterpret_cast<float *>(dynamicLds + words);
   const int maxChunks = (n - 1 + kRescanCols - 1) / kRescanCols;
   const int rankers = kThreads / G, rankSpan = (G + rankers - 1) / rankers;
-  unsigned int generation = 0;
+  int done = *s.done;
+  if (done >= n - 1 || barrierAborted(s.bar))
+    return;
+  unsigned int generation = barrierGeneration(s.bar);
   const bool clocked = s.clocks && g == 0 && tid == 0;
   unsigned long long ticks[4] = {0, 0, 0, 0}, t0 = 0;
   auto lap = [&](int part) {
@@ -375,16 +409,13 @@ __global__ void __launch_bounds__(kThreads) denseMergeKernel(DenseState s) {
   // This workgroup's kTop lowest settled rows, wave by wave (thread t looks
   // at rows t, t + kThreads, ...; keys are distinct, so the next lowest is the
   // lowest above the last).
-  // Only the first `count` are looked for.
-  auto waveTop = [&](int count) {
+  auto waveTop = [&]() {
     auto keyOf = [&](int r) {
       return r < rows && !ownPending[r] ? selectionKey(ownFn[r], mine0 + r) : kEmptyKey;
     };
     const unsigned long long first = keyOf(tid); // most workgroups own at most kThreads rows
-    if (lane >= count && lane < kTop)
-      topKey[wave * kTop + lane] = kEmptyKey;
     unsigned long long last = 0;
-    for (int q = 0; q < count; ++q) {
+    for (int q = 0; q < kTop; ++q) {
       unsigned long long best = q == 0 || first > last ? first : kEmptyKey;
       for (int r = tid + kThreads; r < rows; r += kThreads) {
         const unsigned long long key = keyOf(r);
@@ -455,34 +486,37 @@ __global__ void __launch_bounds__(kThreads) denseMergeKernel(DenseState s) {
     return (int)(unsigned)(i & 1 ? w >> 32 : w);
   };
 
-  // Every slot starts active and settled.
-  for (int w = tid; w < words; w += kThreads) {
-    const int rest = n - 32 * w;
-    activeBits[w] = rest >= 32 ? 0xffffffffu : (1u << rest) - 1u;
-  }
+  for (int w = tid; w < words; w += kThreads)
+    activeBits[w] = s.active[w];
+  if (tid == 0)
+    pendCount = 0;
+  __syncthreads();
   for (int r = tid; r < rows; r += kThreads) {
     ownFn[r] = s.scanned[mine0 + r];
     ownNext[r] = s.scanned[n + mine0 + r];
     ownSize[r] = s.size[mine0 + r];
     ownSlot[r] = -1;
-    ownPending[r] = 0;
+    const bool pending = ownFn[r] == kEmptyKey && ownNext[r] != kEmptyKey;
+    ownPending[r] = pending;
+    if (pending) {
+      pendRow[atomicAdd(&pendCount, 1)] = mine0 + r;
+      s.scanned[n + mine0 + r] = kEmptyKey;
+    }
   }
-  if (tid == 0)
-    pendCount = 0;
-  waveTop(kTop);
+  waveTop();
   __syncthreads();
   writeRecord();
+  if (pendCount > kInlineRows)
+    for (int i = tid; i < pendCount; i += kThreads)
+      s.pendingRows[(size_t)g * per + i] = pendRow[i];
   if (!gridBarrier(s.bar, generation, &barrierOk))
     return;
   if (clocked)
     t0 = wall_clock64();
 
-  // The batch's limit. Where each merge takes in the cluster just made (a
-  // chain), a batch is cut to its first merge and its row is scanned again: a
-  // batch of one costs less. So such a cut limits the next batches to one,
-  // twice as many of them as the cut before.
-  int limit = s.batch, hold = 0, holdNext = 1;
-  for (int done = 0; done < n - 1;) {
+  float average = s.average; // merges that stand per batch
+  bool leave = false;        // no more batches: pending rows settle, then the loop is left
+  while (done < n - 1) {
     // ---- First half: select the batch.
     unsigned long long sel[kTop], bound = kEmptyKey;
     unsigned int col[kTop] = {};
@@ -535,11 +569,9 @@ __global__ void __launch_bounds__(kThreads) denseMergeKernel(DenseState s) {
         incl += v;
     }
     const bool spill = __ballot(cnt > kInlineRows) != 0;
-    unsigned long long lowestHead = limit == 1 ? waveMinKey(sel[0]) : kEmptyKey;
     if (lane == 0) {
       waveKey[wave] = bound;
       waveKey[kWaves + wave] = guard;
-      waveKey[2 * kWaves + wave] = lowestHead;
       waveInt[kWaves + wave] = spill;
     }
     if (lane == 63)
@@ -551,7 +583,6 @@ __global__ void __launch_bounds__(kThreads) denseMergeKernel(DenseState s) {
     for (int w = 0; w < kWaves; ++w) {
       bound = minKey(bound, waveKey[w]);
       guard = minKey(guard, waveKey[kWaves + w]);
-      lowestHead = minKey(lowestHead, waveKey[2 * kWaves + w]);
       start += w < wave ? waveInt[w] : 0;
       listCount += waveInt[w];
       spilled |= waveInt[kWaves + w] != 0;
@@ -566,7 +597,7 @@ __global__ void __launch_bounds__(kThreads) denseMergeKernel(DenseState s) {
       listStart[G] = listCount;
     // The kMaxBatch lowest heads' workgroups hold the kMaxBatch lowest keys:
     // each head's rank, by kThreads / G threads per head.
-    if (limit > 1 && tid < rankers * G) {
+    if (tid < rankers * G) {
       const int i = tid % G, lo = tid / G * rankSpan, hi = min(G, lo + rankSpan);
       const unsigned long long key = heads[i];
       int below = 0;
@@ -586,12 +617,7 @@ __global__ void __launch_bounds__(kThreads) denseMergeKernel(DenseState s) {
         ownSlot[j - mine0] = (signed char)(kMaxBatch + at);
     };
     __syncthreads();
-    if (limit == 1) {
-      if (sel[0] == lowestHead && lowestHead < bound)
-        take(0, keyIndex(sel[0]), (int)col[0], sel[0]);
-      if (tid == 0)
-        batchCount = lowestHead < bound ? 1 : bound == kEmptyKey ? -1 : 0;
-    } else if (tid < G && sel[0] != kEmptyKey) {
+    if (tid < G && sel[0] != kEmptyKey) {
       const int r = headRank[tid];
       if (r < kMaxBatch) {
 #pragma unroll
@@ -601,9 +627,8 @@ __global__ void __launch_bounds__(kThreads) denseMergeKernel(DenseState s) {
         }
       }
     }
-    if (limit > 1)
-      __syncthreads();
-    if (wave == 0 && limit > 1) {
+    __syncthreads();
+    if (wave == 0) {
       const unsigned long long key = cand[lane];
       // Nor any key above the last of the chosen heads: a workgroup that is
       // not among them may have a lower one.
@@ -639,11 +664,12 @@ __global__ void __launch_bounds__(kThreads) denseMergeKernel(DenseState s) {
       const unsigned long long inMask = ((stop & -stop) - 1) & ~retired;
       const bool in = inMask >> lane & 1;
       const int at = __popcll(inMask & ((1ull << lane) - 1));
+      const int limit = leave ? 0 : s.batch;
       if (in && at < limit)
         take(at, i, j, k);
       if (lane == 0)
         batchCount = valid == 0 && bound == kEmptyKey ? -1 : min(limit, __popcll(inMask));
-    } else if (wave > 0) {
+    } else {
       // The pending rows are scanned again (no distance is written in this
       // half), one column chunk per wave and step.
       const unsigned int numItems = (unsigned)listCount * (unsigned)maxChunks;
@@ -682,6 +708,7 @@ __global__ void __launch_bounds__(kThreads) denseMergeKernel(DenseState s) {
         for (int r = done + tid; r < n - 1; r += kThreads)
           for (int c = 0; c < 4; ++c)
             s.tree[(size_t)r * 4 + c] = -1.0;
+      done = n - 1;
       break;
     }
     const int numInstall = pendCount;
@@ -851,17 +878,12 @@ __global__ void __launch_bounds__(kThreads) denseMergeKernel(DenseState s) {
       const unsigned long long cut = __ballot(lane >= m || (lane > 0 && !(own < before)));
       valid = __ffsll((long long)cut) - 1; // m <= 16: lane 63 is cut
     }
+    if (leave) // every row is settled
+      break;
     const bool whole = valid == m;
-    if (!whole && valid == 1) {
-      limit = 1;
-      hold = holdNext;
-      holdNext = min(2 * holdNext, 256);
-    } else if (hold > 0) {
-      --hold;
-    } else {
-      limit = s.batch;
-      if (valid > 1)
-        holdNext = 1;
+    if (m > 0) {
+      average += ((float)valid - average) * (1.0f / 16);
+      leave = average < kFewStand;
     }
     int slotsA[kMaxBatch], slotsB[kMaxBatch]; // uniform
     {
@@ -954,7 +976,7 @@ __global__ void __launch_bounds__(kThreads) denseMergeKernel(DenseState s) {
       ownFn[r] = f;
       ownNext[r] = other;
     }
-    waveTop(limit == 1 ? 1 : kTop);
+    waveTop();
     __syncthreads();
     writeRecord();
     if (tid >= 64 && tid < 64 + m) {
@@ -983,9 +1005,313 @@ __global__ void __launch_bounds__(kThreads) denseMergeKernel(DenseState s) {
       return;
     lap(2);
   }
+  // The state of the loop, for a run of single merges.
+  for (int r = tid; r < rows; r += kThreads) {
+    s.scanned[mine0 + r] = ownFn[r];
+    s.scanned[n + mine0 + r] = ownFn[r] == kEmptyKey ? kEmptyKey : ownNext[r];
+  }
+  if (g == 0)
+    for (int w = tid; w < words; w += kThreads)
+      s.active[w] = activeBits[w];
+  if (g == 0 && tid == 0)
+    *s.done = done;
   if (clocked)
     for (int i = 0; i < 4; ++i)
-      s.clocks[i] = ticks[i];
+      s.clocks[i] += ticks[i];
+}
+
+// A run of merges made one at a time, one grid barrier each: for chains, where
+// every merge takes in the cluster just made or ties with the next (duplicates),
+// so that a batch keeps its first merge only. A merge is committed in the phase
+// that computes its distances; row a's new nearest is known in the next phase,
+// from every workgroup's part of the row. A row that loses its nearest is
+// pending, its other keys' bound below all of its keys, and is scanned again,
+// by its own workgroup, only when no settled row's key is below that bound: in
+// a chain of single linkage such a row is nearer to the grown cluster and joins
+// it before. (Scanned at once, chains of 30,000 points took up to 33 us per
+// merge, of 100,000 41.)
+// Bound by latency, as the batches: one barrier and three dependent round trips
+// per merge. Chains of single linkage took 25 us per merge as batches of one (n =
+// 30,000; 16 at 2,000), two barriers each, and 14 in a loop of this kind that
+// scanned rows over all workgroups in the next phase; now 7 (n = 2,000) to 11.5.
+template <int LINKAGE>
+__global__ void __launch_bounds__(kThreads) denseChainKernel(DenseState s, int run) {
+  extern __shared__ unsigned int activeBits[]; // [(n + 31) / 32]
+  // Per row, as in the batch loop; a pending row's fn is empty, its next a bound
+  // below all of its keys. Both are empty for a row that has none.
+  __shared__ unsigned long long ownFn[kMaxOwned], ownNext[kMaxOwned];
+  __shared__ int ownSize[kMaxOwned];
+  __shared__ int scanRow[kMaxOwned]; // rows to scan again
+  __shared__ int scanCount;
+  // Per wave: lowest key, its column, the two lowest of row a's part, bound.
+  __shared__ unsigned long long inKey[kWaves], inFn[kWaves], inNext[kWaves], inBound[kWaves];
+  __shared__ unsigned int inCol[kWaves];
+  __shared__ unsigned long long outKey[kWaves], outFn[kWaves], outNext[kWaves], outBound[kWaves];
+  __shared__ unsigned int outCol[kWaves];
+  __shared__ int barrierOk;
+
+  const int n = s.n, per = s.per;
+  const int G = gridDim.x, g = blockIdx.x;
+  const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
+  const int mine0 = min(n, g * per), mine1 = min(n, mine0 + per), rows = mine1 - mine0;
+  const int words = (n + 31) >> 5;
+  int done = *s.done;
+  if (done >= n - 1 || barrierAborted(s.bar))
+    return;
+  const int until = min(n - 1, done + run);
+  unsigned int generation = barrierGeneration(s.bar);
+  const bool clocked = s.clocks && g == 0 && tid == 0;
+  unsigned long long ticks[4] = {0, 0, 0, 0}, t0 = clocked ? wall_clock64() : 0;
+  auto lap = [&](int part) {
+    if (clocked) {
+      const unsigned long long t = wall_clock64();
+      ticks[part] += t - t0;
+      t0 = t;
+    }
+  };
+  auto entry = [&](int i, int j) -> size_t {
+    return i < j ? condensedIndex(i, j, n) : condensedIndex(j, i, n);
+  };
+  for (int w = tid; w < words; w += kThreads)
+    activeBits[w] = s.active[w];
+  // A thread holds rows tid, tid + kThreads, ...: only it touches their state.
+  // key, col and bound: over its rows, the lowest settled key, its column, and
+  // the lowest bound of a pending row.
+  unsigned long long key = kEmptyKey, bound = kEmptyKey;
+  unsigned int col = 0;
+  auto note = [&](int r) {
+    const unsigned long long f = ownFn[r];
+    const unsigned long long k = selectionKey(f == kEmptyKey ? ownNext[r] : f, mine0 + r);
+    if (f == kEmptyKey) {
+      bound = minKey(bound, k);
+    } else if (k < key) {
+      key = k;
+      col = keyIndex(f);
+    }
+  };
+  for (int r = tid; r < rows; r += kThreads) {
+    ownFn[r] = s.scanned[mine0 + r];
+    ownNext[r] = s.scanned[n + mine0 + r];
+    ownSize[r] = s.size[mine0 + r];
+    note(r);
+  }
+  if (tid == 0)
+    scanCount = 0;
+  // The workgroup's record: the waves' results through LDS, by wave 0.
+  auto publish = [&](unsigned long long part, unsigned long long partNext, int buffer) {
+    unsigned long long low = waveMinKey(key), least = waveMinKey(bound);
+    waveLowest2(part, partNext);
+    if (low != kEmptyKey ? key == low : lane == 0) { // keys are distinct
+      outKey[wave] = low;
+      outCol[wave] = col;
+      outFn[wave] = part;
+      outNext[wave] = partNext;
+      outBound[wave] = least;
+    }
+    lap(1);
+    __syncthreads();
+    if (wave != 0)
+      return;
+    const unsigned long long k = lane < kWaves ? outKey[lane] : kEmptyKey;
+    part = lane < kWaves ? outFn[lane] : kEmptyKey;
+    partNext = lane < kWaves ? outNext[lane] : kEmptyKey;
+    least = waveMinKey(lane < kWaves ? outBound[lane] : kEmptyKey);
+    low = waveMinKey(k);
+    waveLowest2(part, partNext);
+    if (low != kEmptyKey ? k == low : lane == 0) {
+      ulonglong2 *r = reinterpret_cast<ulonglong2 *>(s.steps + ((size_t)buffer * G + g) * kStepWords);
+      r[0] = make_ulonglong2(low, (unsigned long long)outCol[lane]);
+      r[1] = make_ulonglong2(part, partNext);
+      r[2] = make_ulonglong2(least, 0);
+    }
+  };
+  publish(kEmptyKey, kEmptyKey, 0);
+  if (!gridBarrier(s.bar, generation, &barrierOk))
+    return;
+  lap(2);
+
+  int prevA = -1, prevSize = 0;
+  for (int buffer = 0;; buffer ^= 1) {
+    // The lowest pair, and the previous merge's row from its parts.
+    unsigned long long fn = kEmptyKey, next = kEmptyKey;
+    key = bound = kEmptyKey;
+    if (tid < G) {
+      const ulonglong2 *r =
+          reinterpret_cast<const ulonglong2 *>(s.steps + ((size_t)buffer * G + tid) * kStepWords);
+      const ulonglong2 v = r[0], part = r[1];
+      bound = r[2].x;
+      key = v.x;
+      col = (unsigned)v.y;
+      fn = part.x;
+      next = part.y;
+    }
+    unsigned long long low = waveMinKey(key), least = waveMinKey(bound);
+    waveLowest2(fn, next);
+    if (low != kEmptyKey ? key == low : lane == 0) {
+      inKey[wave] = low;
+      inCol[wave] = col;
+      inFn[wave] = fn;
+      inNext[wave] = next;
+      inBound[wave] = least;
+    }
+    __syncthreads();
+    low = least = fn = next = kEmptyKey;
+#pragma unroll
+    for (int w = 0; w < kWaves; ++w) {
+      if (inKey[w] < low) {
+        low = inKey[w];
+        col = inCol[w];
+      }
+      least = minKey(least, inBound[w]);
+      offer(fn, next, inFn[w]);
+      next = minKey(next, inNext[w]);
+    }
+    if (prevA >= mine0 && prevA < mine1 && (prevA - mine0) % kThreads == tid) {
+      ownFn[prevA - mine0] = fn;
+      ownNext[prevA - mine0] = next;
+      ownSize[prevA - mine0] = prevSize;
+      s.size[prevA] = prevSize;
+    }
+    if (done == until)
+      break;
+    if (prevA >= 0 && selectionKey(fn, prevA) < low) {
+      low = selectionKey(fn, prevA);
+      col = keyIndex(fn);
+    }
+    if (least != kEmptyKey && !(low < least)) {
+      // A pending row may hold the lowest key: those whose bound is not above it
+      // are scanned, and the records published again.
+      for (int r = tid; r < rows; r += kThreads)
+        if (ownFn[r] == kEmptyKey && ownNext[r] != kEmptyKey &&
+            selectionKey(ownNext[r], mine0 + r) <= low)
+          scanRow[atomicAdd(&scanCount, 1)] = r;
+      __syncthreads();
+      const int scans = scanCount;
+      for (int i = 0; i < scans; ++i) {
+        const int r = scanRow[i], k = mine0 + r;
+        const size_t base = condensedIndex(k, k + 1, n) - (size_t)(k + 1);
+        unsigned long long lowest = kEmptyKey, second = kEmptyKey;
+        for (int j0 = k + 1; j0 < n; j0 += kThreads * kScanPer) {
+          float v[kScanPer];
+#pragma unroll
+          for (int u = 0; u < kScanPer; ++u) {
+            const int j = j0 + tid + u * kThreads;
+            v[u] = j < n ? s.D[base + j] : 0.0f;
+          }
+#pragma unroll
+          for (int u = 0; u < kScanPer; ++u) {
+            const int j = j0 + tid + u * kThreads;
+            if (j < n && isActive(activeBits, j))
+              offer(lowest, second, denseKey(v[u], (unsigned)j));
+          }
+        }
+        waveLowest2(lowest, second);
+        if (lane == 0) {
+          outFn[wave] = lowest;
+          outNext[wave] = second;
+        }
+        __syncthreads();
+        if (r % kThreads == tid) {
+          lowest = second = kEmptyKey;
+          for (int w = 0; w < kWaves; ++w) {
+            offer(lowest, second, outFn[w]);
+            second = minKey(second, outNext[w]);
+          }
+          ownFn[r] = lowest;
+          ownNext[r] = second;
+        }
+        __syncthreads(); // outFn is written again
+      }
+      if (tid == 0)
+        scanCount = 0;
+      key = bound = kEmptyKey;
+      for (int r = tid; r < rows; r += kThreads)
+        note(r);
+      prevA = -1;
+      publish(kEmptyKey, kEmptyKey, buffer ^ 1);
+      lap(3);
+      if (!gridBarrier(s.bar, generation, &barrierOk))
+        return;
+      lap(2);
+      continue;
+    }
+    if (low == kEmptyKey) {
+      // No pair (non-finite distances): the remaining rows report -1, as in the
+      // batch loop.
+      if (g == 0)
+        for (int r = done + tid; r < n - 1; r += kThreads)
+          for (int c = 0; c < 4; ++c)
+            s.tree[(size_t)r * 4 + c] = -1.0;
+      done = n - 1;
+      break;
+    }
+    const int a = keyIndex(low), b = (int)col;
+    const float dab = fromOrderedBits((unsigned)(low >> 32));
+    // The previous merge's size is on its way to memory.
+    const int na = a == prevA ? prevSize : s.size[a];
+    const int nb = b == prevA ? prevSize : s.size[b];
+    lap(0);
+
+    unsigned long long part = kEmptyKey, partNext = kEmptyKey;
+    key = bound = kEmptyKey;
+    for (int r = tid; r < rows; r += kThreads) {
+      const int k = mine0 + r;
+      if (!isActive(activeBits, k))
+        continue;
+      if (k == a || k == b) { // b retires; a's nearest is known in the next phase
+        ownFn[r] = kEmptyKey;
+        ownNext[r] = kEmptyKey;
+        continue;
+      }
+      const float dak = s.D[entry(a, k)], dbk = s.D[entry(b, k)];
+      const float nd = lanceWilliams<LINKAGE>(dak, dbk, dab, na, nb, ownSize[r]);
+      s.D[entry(a, k)] = nd;
+      const unsigned long long c = k < a ? denseKey(nd, (unsigned)a) : kEmptyKey;
+      if (k > a)
+        offer(part, partNext, denseKey(nd, (unsigned)k));
+      unsigned long long f = ownFn[r], other = ownNext[r];
+      const int at = f == kEmptyKey ? -1 : keyIndex(f);
+      if (f == kEmptyKey || at == a || at == b) // pending, or its nearest is gone
+        f = c < other ? c : kEmptyKey;
+      else
+        offer(f, other, c);
+      ownFn[r] = f;
+      ownNext[r] = other;
+      note(r);
+    }
+    publish(part, partNext, buffer ^ 1);
+    if (tid == 0) {
+      activeBits[b >> 5] &= ~(1u << (b & 31));
+      if (g == 0) {
+        double *row = s.tree + (size_t)done * 4;
+        const int ia = s.id[a], ib = s.id[b];
+        row[0] = (double)min(ia, ib);
+        row[1] = (double)max(ia, ib);
+        row[2] = (double)dab;
+        row[3] = (double)(na + nb);
+        s.id[a] = s.firstNewId + done;
+      }
+    }
+    prevA = a;
+    prevSize = na + nb;
+    ++done;
+    lap(3);
+    if (!gridBarrier(s.bar, generation, &barrierOk))
+      return;
+    lap(2);
+  }
+  for (int r = tid; r < rows; r += kThreads) {
+    s.scanned[mine0 + r] = ownFn[r];
+    s.scanned[n + mine0 + r] = ownNext[r];
+  }
+  if (g == 0)
+    for (int w = tid; w < words; w += kThreads)
+      s.active[w] = activeBits[w];
+  if (g == 0 && tid == 0)
+    *s.done = done;
+  if (clocked)
+    for (int i = 0; i < 4; ++i)
+      s.clocks[i] += ticks[i];
 }
 
 __global__ void denseSetupKernel(DenseState s, const int *initialSize, const int *initialId) {
@@ -995,6 +1321,13 @@ __global__ void denseSetupKernel(DenseState s, const int *initialSize, const int
     s.scanned[i] = kEmptyKey;
     s.scanned[s.n + i] = kEmptyKey;
   }
+  const int words = (s.n + 31) >> 5; // every slot is active
+  for (int w = blockIdx.x * blockDim.x + threadIdx.x; w < words; w += gridDim.x * blockDim.x) {
+    const int rest = s.n - 32 * w;
+    s.active[w] = rest >= 32 ? 0xffffffffu : (1u << rest) - 1u;
+  }
+  if (blockIdx.x == 0 && threadIdx.x == 0)
+    *s.done = 0;
 }
 
 __global__ void denseInitItemsKernel(int2 *items, int n) {
@@ -1024,8 +1357,8 @@ int denseLinkageOnCondensed(float *D, int n, int linkage, const int *initialSize
     return kErrInvalidShape; // beyond any condensed matrix that fits in HBM
   DenseState st{};
   DevArray<int> size, id;
-  DevArray<unsigned long long> scanned, records, partFn, partNext;
-  DevArray<unsigned int> partMin;
+  DevArray<unsigned long long> scanned, records, steps, partFn, partNext;
+  DevArray<unsigned int> partMin, active;
   DevArray<int> pendingRows;
   DevArray<int2> initItems;
   DevArray<double> tree;
@@ -1035,7 +1368,8 @@ int denseLinkageOnCondensed(float *D, int n, int linkage, const int *initialSize
   const int maxChunks = (n - 1 + kChunk - 1) / kChunk;
   const long long initCount = (long long)(n - 1) * maxChunks;
   const int groups = (G + kGroup - 1) / kGroup;
-  const size_t numBarrierWords = (size_t)kLineWords * (3 + groups);
+  // The barrier's words, then the merges made.
+  const size_t numBarrierWords = (size_t)kLineWords * (3 + groups), doneWord = numBarrierWords;
   // The merge kernel keeps one bit per slot and the batch's new distances of
   // its rows in LDS beside its static arrays.
   const size_t activeBytes = (size_t)(n + 31) / 32 * sizeof(unsigned int);
@@ -1045,6 +1379,10 @@ int denseLinkageOnCondensed(float *D, int n, int linkage, const int *initialSize
   s((int)hipDeviceGetAttribute(&maxLds, hipDeviceAttributeMaxSharedMemoryPerBlock, device));
   if (!s.ok())
     return s.code;
+  const void *chain = linkage == kSingle     ? (const void *)denseChainKernel<kSingle>
+                      : linkage == kComplete ? (const void *)denseChainKernel<kComplete>
+                      : linkage == kAverage  ? (const void *)denseChainKernel<kAverage>
+                                             : (const void *)denseChainKernel<kWard>;
   const void *kernel = linkage == kSingle     ? (const void *)denseMergeKernel<kSingle>
                        : linkage == kComplete ? (const void *)denseMergeKernel<kComplete>
                        : linkage == kAverage  ? (const void *)denseMergeKernel<kAverage>
@@ -1062,13 +1400,15 @@ int denseLinkageOnCondensed(float *D, int n, int linkage, const int *initialSize
   s(id.alloc(n));
   s(scanned.alloc((size_t)2 * n));
   s(records.alloc((size_t)G * kRecordWords));
+  s(steps.alloc((size_t)2 * G * kStepWords));
+  s(active.alloc((n + 31) / 32));
   s(partFn.alloc((size_t)kMaxBatch * G));
   s(partNext.alloc((size_t)kMaxBatch * G));
   s(partMin.alloc((size_t)kMaxBatch * G));
   s(pendingRows.alloc((size_t)G * per));
   s(initItems.alloc(initCount));
   s(tree.alloc((size_t)(n - 1) * 4));
-  s(barrierWords.alloc(numBarrierWords));
+  s(barrierWords.alloc(numBarrierWords + 1));
   if (!s.ok())
     return s.code;
   st.D = D;
@@ -1083,6 +1423,9 @@ int denseLinkageOnCondensed(float *D, int n, int linkage, const int *initialSize
   st.id = id;
   st.scanned = scanned;
   st.records = records;
+  st.steps = steps;
+  st.active = active;
+  st.done = reinterpret_cast<int *>(barrierWords.get() + doneWord);
   st.pendingRows = pendingRows;
   st.items = initItems;
   st.tree = tree;
@@ -1104,17 +1447,32 @@ int denseLinkageOnCondensed(float *D, int n, int linkage, const int *initialSize
                      dim3((unsigned)std::max<long long>(1, std::min<long long>(initCount, 8LL * G))),
                      dim3(kThreads), 0, stream(), st, (int)initCount);
   s((int)hipGetLastError());
-  if (s.ok()) {
+  // Batches until the tree is whole or few merges of a batch stand; then a run of
+  // single merges, and batches again.
+  std::vector<unsigned int> words(numBarrierWords + 1);
+  int from = 0, run = kFirstRun; // merges made when the batches begin
+  st.average = kFirstAverage;
+  while (s.ok()) {
     void *args[] = {&st};
     s((int)hipLaunchCooperativeKernel(kernel, dim3(G), dim3(kThreads),
                                       args, (unsigned int)dynamicBytes, stream()));
+    s(sync());
+    if (s.ok())
+      s(download(words.data(), barrierWords, words.size() * sizeof(unsigned int)));
+    if (s.ok() && words[kLineWords])
+      return (int)hipErrorLaunchTimeOut; // a barrier wait exceeded its limit
+    const int done = (int)words[doneWord];
+    if (!s.ok() || done >= n - 1)
+      break;
+    if (done - from >= kFirstRun)
+      run = kFirstRun;
+    void *runArgs[] = {&st, &run};
+    s((int)hipLaunchCooperativeKernel(chain, dim3(G), dim3(kThreads), runArgs,
+                                      (unsigned int)activeBytes, stream()));
+    from = std::min(n - 1, done + run);
+    run = std::min(2 * run, kLongestRun);
+    st.average = kNextAverage;
   }
-  s(sync());
-  unsigned int aborted = 0;
-  if (s.ok())
-    s(download(&aborted, barrierWords.get() + kLineWords, sizeof(aborted)));
-  if (s.ok() && aborted)
-    return (int)hipErrorLaunchTimeOut; // a barrier wait exceeded its limit
   if (s.ok() && st.clocks) {
     unsigned long long ticks[4];
     s(download(ticks, clocks, sizeof(ticks)));

@@ -236,3 +236,24 @@ def test_ward_searches_count_their_pairs():
         _lib.set_timing(False)
     assert ms > 0 and launches > 1
     assert n * n < pairs < n * n * launches
+
+
+@pytest.mark.parametrize("method", ["single", "complete", "average", "ward"])
+@pytest.mark.parametrize("n", [513, 2600])
+@pytest.mark.parametrize("data", ["chain", "duplicates", "shells"])
+def test_dense_runs_of_single_merges(method, n, data):
+    # Where few merges of a batch stand the loop makes runs of single merges: one
+    # growing cluster that takes in the rest (64 features), tied merges
+    # (50 copies of each point), and shells around a point, whose rows lose their
+    # nearest and wait with a bound (settled within a run, or handed back to the
+    # batches with it).
+    rng = np.random.default_rng(n)
+    X = rng.normal(size=(n, 64))
+    if data == "duplicates":
+        X = np.repeat(rng.normal(size=(n // 50 + 1, 8)), 50, axis=0)[:n]
+    elif data == "shells":
+        X /= np.linalg.norm(X, axis=1, keepdims=True)
+        X *= rng.uniform(0.5, 1.5, (n, 1))
+    X = X.astype(np.float32)
+    Z = cuhc.linkage(X, method=method, algorithm="dense")
+    np.testing.assert_array_equal(Z, oracle.dense_linkage(X, method))
