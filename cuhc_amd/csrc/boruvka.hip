@@ -30,7 +30,7 @@ int DevicePoints::arrange(const float *X, int n, int d) {
 // Both entry paths check the coordinates first (kErrNonFinite for NaN or
 // infinity): the FP16 candidate kernels are compiled without NaN semantics and
 // the k-d order needs ordered comparisons.
-int DevicePoints::upload(const float *hostPoints, int n, int d, bool spatial) {
+int DevicePoints::upload(const float *hostPoints, int n, int d, bool spatial, bool keep) {
   const size_t count = (size_t)n * d;
   Status s;
   s(points.alloc(count));
@@ -41,13 +41,25 @@ int DevicePoints::upload(const float *hostPoints, int n, int d, bool spatial) {
     s(checkFinite(points, count));
     return s.code;
   }
-  DevArray<float> raw;
   s(raw.alloc(count));
   s(cuhc::upload(raw, hostPoints, count * sizeof(float)));
   s(checkFinite(raw, count));
   if (s.ok())
     s(arrange(raw, n, d));
+  if (keep)
+    given = raw;
+  else
+    raw.release();
   return s.code;
+}
+
+void DevicePoints::leaveOrder() {
+  if (!inOrder || !given)
+    return;
+  external = given;
+  points.release();
+  orig.release();
+  inOrder = false;
 }
 
 // The caller may have written devicePoints on another stream of this HIP
@@ -66,6 +78,7 @@ int DevicePoints::adopt(const float *devicePoints, int n, int d, bool spatial) {
   s(points.alloc(count));
   if (s.ok())
     s(arrange(devicePoints, n, d));
+  given = devicePoints;
   return s.code;
 }
 

@@ -39,13 +39,15 @@ bool useMixed(int metricId, int d) {
 
 // Decides pruning for points in spatial order (auto mode samples a pruned
 // pass, reference src/capi.cu:101-119; here the sampled row tiles compute
-// their first 64 walk steps and count the rest against the bound reached).
-int decidePruning(const DevicePoints &pts, int n, int d, MetricSpec m, bool &prune) {
+// their first 64 walk steps and count the rest against the bound reached); most:
+// the largest share of pairs that pays.
+int decidePruning(const DevicePoints &pts, int n, int d, MetricSpec m, bool &prune,
+                  double most = kPruneGiveUpShare) {
   if (!prune || gPruneMode.load() == kPruneAlways)
     return 0;
   double share = 1.0;
   const int status = estimatePrunedShare(pts.data(), n, d, m, &share);
-  prune = status == 0 && share <= kPruneGiveUpShare;
+  prune = status == 0 && share <= most;
   return status;
 }
 
@@ -101,9 +103,14 @@ int linkageImpl(const float *X, bool onDevice, int n, int d, int metricId, float
     const MetricSpec sq{kSqEuclidean, 2.0f};
     bool prune = shouldPrune(gPruneMode.load(), kSqEuclidean, n, d);
     DevicePoints pts;
-    s(onDevice ? pts.adopt(X, n, d, prune) : pts.upload(X, n, d, prune));
+    s(onDevice ? pts.adopt(X, n, d, prune) : pts.upload(X, n, d, prune, prune));
     if (s.ok())
-      s(decidePruning(pts, n, d, sq, prune));
+      s(decidePruning(pts, n, d, sq, prune, kWardPruneShare));
+    // Searches over all pairs take the given order: in k-d order a row's nearest
+    // lie together, and its list fills with far ones before they come up (60,000
+    // points of 8 features 22.8 ms, now 18.1; 16.8 without order and sample).
+    if (!prune)
+      pts.leaveOrder();
     PassStats stats;
     RnnOptions opt;
     opt.prune = prune && pts.ordered();

@@ -15,14 +15,19 @@ struct DevicePoints {
   DevArray<int> orig; // only when ordered
   bool inOrder = false;
   bool ordered() const { return inOrder; }
-  // Uploads hostPoints (n x d), in spatial order if spatial is set.
-  int upload(const float *hostPoints, int n, int d, bool spatial);
+  // Uploads hostPoints (n x d), in spatial order if spatial is set; keep: with
+  // the points in their given order too, for leaveOrder.
+  int upload(const float *hostPoints, int n, int d, bool spatial, bool keep = false);
   // Adopts device-resident points (no copy unless spatial order is wanted).
   int adopt(const float *devicePoints, int n, int d, bool spatial);
+  // Back to the given order (adopted points, or uploaded with keep).
+  void leaveOrder();
   // The spatial order of X into orig and points.
   int arrange(const float *X, int n, int d);
   const float *data() const { return external ? external : points.get(); }
   const float *external = nullptr;
+  const float *given = nullptr; // while ordered
+  DevArray<float> raw;
 };
 
 // Edges of a spanning forest in device memory (original indices, u < v): u, v

@@ -368,8 +368,13 @@ __global__ void __launch_bounds__(256, 3)
       (&top[0][0])[i] = kEmptyKey;
     __syncthreads();
     bool first = true;
-    for (int colTile = split; colTile < colTiles; colTile += splits) {
-      const int col0 = colTile * DIM;
+    // From the column tile nearest the first row's own, and around: where slots
+    // are in spatial order the lists are tight from there on.
+    const int count = (colTiles - split + splits - 1) / splits;
+    const int start = min(count - 1, max(0, rowSlot[0] / DIM - split) / splits);
+    for (int i = 0; i < count; ++i) {
+      const int at = start + i < count ? start + i : start + i - count;
+      const int col0 = (split + at * splits) * DIM;
       float acc[TR][TR];
 #pragma unroll
       for (int r = 0; r < TR; ++r)
@@ -1010,8 +1015,8 @@ int rnnWard(const float *X, int n, int d, const RnnOptions &opt, double *tree) {
   // A pruned pass (points in k-d order: merged clusters take the lower slot's
   // place in the compacted order, so slots stay spatially coherent and the
   // cluster tiles keep tight boxes) finds every cluster's nearest again: lists
-  // of one key. It stops for good once a pass computes more than half of the
-  // tile pairs, and the searches go on from its lists.
+  // of one key. It stops for good once a pass computes more than
+  // kWardGiveUpShare of the tile pairs, and the searches go on from its lists.
   bool pruneThisPass = opt.prune;
   DevArray<unsigned long long> nearest;
   auto prunedPass = [&](int m) {
@@ -1027,7 +1032,7 @@ int rnnWard(const float *X, int n, int d, const RnnOptions &opt, double *tree) {
     if (st.ok())
       st(nearestOtherWalk(cur.c32, m, d, MetricSpec{kSqEuclidean, 2.0f}, w, comp, nullptr, nullptr,
                           nearest, &share, opt.stats));
-    pruneThisPass = share <= kPruneGiveUpShare;
+    pruneThisPass = share <= kWardGiveUpShare;
     if (st.ok())
       hipLaunchKernelGGL(listsFromKeysKernel, gridOf(m), dim3(256), 0, stream(), nearest.get(), 1,
                          m, lists);

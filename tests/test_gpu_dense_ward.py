@@ -257,3 +257,25 @@ def test_dense_runs_of_single_merges(method, n, data):
     X = X.astype(np.float32)
     Z = cuhc.linkage(X, method=method, algorithm="dense")
     np.testing.assert_array_equal(Z, oracle.dense_linkage(X, method))
+
+
+@pytest.mark.parametrize("d, held", [(5, "host"), (5, "device"), (20, "host"), (20, "device")])
+def test_ward_takes_the_given_order_where_pruning_does_not_pay(d, held):
+    # The points are put in k-d order for a sampled pass; where it computes most
+    # pairs the searches run over the points as given: the tree of an unpruned
+    # run bit for bit (another order of slots rounds some heights otherwise).
+    from cuhc_amd import _lib
+    X = np.random.default_rng(d).standard_cauchy((17_000, d)).astype(np.float32)
+    dev = _lib.DeviceArray(X)
+    trees = {}
+    try:
+        for mode in ["auto", "never"]:
+            _lib.set_pruning(mode)
+            _lib.prune_stats()
+            trees[mode] = cuhc.linkage(X if held == "host" else dev, method="ward",
+                                       algorithm="rnn")
+            assert _lib.prune_stats() == (0, 0)
+    finally:
+        _lib.set_pruning("auto")
+        dev.free()
+    np.testing.assert_array_equal(trees["auto"], trees["never"])
