@@ -65,7 +65,14 @@ constexpr int kLearnedAutoMaxK = 128;
 // 2.2 and 3.6 ms; k = 5: 0.38, 1.2 and 2.1; k = 60: 2.0, 3.9 and 6.2). Its rows
 // take 4 n bytes each (all n of them, if a quarter of the free memory holds
 // them); the lists remain the way without that memory.
-constexpr int radixAutoPoints(int k) { return 14000 + 350 * k; }
+// From 128 features on, also while the lists' tiles of 128 rows do not fill the
+// chip: what is left over between the CUs then outweighs the select (30,000
+// points, k = 8: 128 features 21.0 and 17.2 ms, 300 55 and 39, 784 120 and 71; 64
+// features 15.9 and 17.0; 60,000 of 200 109 and 111).
+int radixAutoPoints(int k, int d) {
+  const int points = 14000 + 350 * k;
+  return d >= 128 ? std::max(points, 128 * numCUs()) : points;
+}
 
 int linkageImpl(const float *X, bool onDevice, int n, int d, int metricId, float metricParam,
                 int linkageId, int algorithmId, double *tree) {
@@ -164,7 +171,8 @@ int hdbscanImpl(const float *X, bool onDevice, int n, int d, int metricId, float
   s(onDevice ? pts.adopt(X, n, d, spatial) : pts.upload(X, n, d, spatial));
   if (s.ok())
     s(decidePruning(pts, n, d, m, prune));
-  if (coreMethod == kCoreAuto && method == kCoreFused && !prune && n <= radixAutoPoints(minSamples))
+  if (coreMethod == kCoreAuto && method == kCoreFused && !prune &&
+      n <= radixAutoPoints(minSamples, d))
     method = kCoreRadixElseFused;
   PassStats stats;
   if (s.ok()) {

@@ -107,7 +107,8 @@ __global__ void __launch_bounds__(256, (coreMinWaves<T, Metric>()))
                           const int *__restrict__ rowPos, const int *__restrict__ tileList,
                           unsigned int *__restrict__ kthBits, float *__restrict__ partial) {
   constexpr int TR = T::TR, kWaves = T::THREADS / 64, kWaveRows = T::WAVE_ROWS;
-  static_assert(T::ROWS_BY_WAVE, "a wave's rows are consecutive");
+  // Pruned: bounds by wave, whose rows are consecutive then.
+  constexpr bool kPruned = T::ROWS_BY_WAVE;
   constexpr int kBatch = 64; // walk steps whose box bounds are computed at once
   __shared__ __align__(16) TileSmem<T> sm;
   // Per wave: the bounds of the batch's steps, the steps within its largest
@@ -129,7 +130,7 @@ __global__ void __launch_bounds__(256, (coreMinWaves<T, Metric>()))
     lists[i] = INFINITY;
   for (int i = threadIdx.x; i < T::DIM; i += T::THREADS)
     sharedKth[i] = splits > 1 && row0 + i < nA ? __uint_as_float(kthBits[row0 + i]) : INFINITY;
-  const bool prune = boxes.numTiles > 0;
+  const bool prune = kPruned && boxes.numTiles > 0;
   float *rowBox = lists + T::DIM * k + wave * 2 * d;
   if (prune) {
     const int row = row0 + wave * kWaveRows + (lane & (kWaveRows - 1));
@@ -215,8 +216,8 @@ __global__ void __launch_bounds__(256, (coreMinWaves<T, Metric>()))
       // (most pairs of a tile are not, which skips their sqrt).
       constexpr bool kFilter = Metric::kAccFilter;
       float v[TR][TR];
-      computeTile<T, Metric, !kFilter, kRowsResident, true>(sm, A, nA, X, n, d, metric, row0,
-                                                            col0, v, NoExtraStage{}, active);
+      computeTile<T, Metric, !kFilter, kRowsResident, kPruned>(sm, A, nA, X, n, d, metric, row0,
+                                                               col0, v, NoExtraStage{}, active);
       if (active) {
         unsigned long long changed = 0;
 #pragma unroll
@@ -466,6 +467,19 @@ template <class F> int withMetricCore(MetricSpec m, F &&f) {
   }
 }
 
+// run(fill, pruned) for the features staged per fill, and for tiles with rows by
+// wave where the pass prunes. Without, every tile is computed, and rows by wave
+// and barriers left to the caller take longer (30,000 points, k = 8, 300 features
+// 59.1 ms, now 55.0; 784 129 and 120).
+template <class Metric, class F> int withTile(int d, bool prune, F &&run) {
+  using Eight = std::integral_constant<int, 8>;
+  using Fill = std::integral_constant<int, 32>;
+  if constexpr (Metric::kBoxBound)
+    if (prune)
+      return d <= 8 ? run(Eight{}, std::true_type{}) : run(Fill{}, std::true_type{});
+  return d <= 8 ? run(Eight{}, std::false_type{}) : run(Fill{}, std::false_type{});
+}
+
 // The tiles by the size of their boxes (squared diagonal, to 7 bits of
 // mantissa), largest first.
 __global__ void boxSizeKeysKernel(CoreBoxes boxes, int d, unsigned int *__restrict__ keys,
@@ -506,14 +520,14 @@ int coreFused(const float *X, int n, int d, MetricSpec m, int k, float *core, bo
               int stepLimit = 0x7fffffff, const int *tileList = nullptr, int numListed = 0) {
   return withMetricCore(m, [&](auto metric) {
     using Metric = decltype(metric);
-    auto run = [&](auto fill) {
-      using T = typename TileFor<Metric, decltype(fill)::value, true>::type;
+    auto run = [&](auto fill, auto pruned) {
+      using T = typename TileFor<Metric, decltype(fill)::value, decltype(pruned)::value>::type;
       const int tiles = (n + T::DIM - 1) / T::DIM;
       size_t smem = (size_t)T::DIM * k * sizeof(float);
       CoreBoxes boxes;
       DevArray<float> low, high;
       Status s;
-      if (prune && Metric::kBoxBound) {
+      if (decltype(pruned)::value) {
         s(low.alloc((size_t)tiles * d));
         s(high.alloc((size_t)tiles * d));
         if (!s.ok())
@@ -559,9 +573,7 @@ int coreFused(const float *X, int n, int d, MetricSpec m, int k, float *core, bo
       s(sync());
       return s.code;
     };
-    if (d <= 8)
-      return run(std::integral_constant<int, 8>{});
-    return run(std::integral_constant<int, 32>{});
+    return withTile<Metric>(d, prune, run);
   });
 }
 
@@ -627,14 +639,14 @@ int coreForRowsFused(const float *X, int n, int d, MetricSpec m, int k, const in
     return s.code;
   return withMetricCore(m, [&](auto metric) {
     using Metric = decltype(metric);
-    auto run = [&](auto fill) {
-      using T = typename TileFor<Metric, decltype(fill)::value, true>::type;
+    auto run = [&](auto fill, auto pruned) {
+      using T = typename TileFor<Metric, decltype(fill)::value, decltype(pruned)::value>::type;
       const int rowTiles = (numRows + T::DIM - 1) / T::DIM;
       size_t smem = (size_t)T::DIM * k * sizeof(float);
       CoreBoxes boxes;
       DevArray<float> low, high;
       Status st;
-      if (prune && Metric::kBoxBound) {
+      if (decltype(pruned)::value) {
         const int tiles = (n + T::DIM - 1) / T::DIM;
         st(low.alloc((size_t)tiles * d));
         st(high.alloc((size_t)tiles * d));
@@ -653,9 +665,7 @@ int coreForRowsFused(const float *X, int n, int d, MetricSpec m, int k, const in
       st(sync());
       return st.code;
     };
-    if (d <= 8)
-      return run(std::integral_constant<int, 8>{});
-    return run(std::integral_constant<int, 32>{});
+    return withTile<Metric>(d, prune, run);
   });
 }
 

@@ -53,6 +53,21 @@ def test_core_methods_agree(k, metric):
             hdbscan_tree(X, k, metric=metric, core_method="fused")
 
 
+@pytest.mark.parametrize("n,d,k", [(127, 127, 2), (129, 128, 2), (1500, 300, 7),
+                                   (16_500, 128, 2)])
+@pytest.mark.parametrize("metric", ["euclidean", "manhattan"])
+def test_core_methods_agree_at_many_features(n, d, k, metric):
+    # Without pruning the lists take the plain tiles; auto takes the select from
+    # 128 features on, also past the points up to which it does below. One value
+    # per pair in all of them: equal bits.
+    X = np.random.default_rng(d).normal(size=(n, d)).astype(np.float32)
+    _, auto = hdbscan_tree(X, k, metric=metric)
+    _, fused = hdbscan_tree(X, k, metric=metric, core_method="fused")
+    _, radix = hdbscan_tree(X, k, metric=metric, core_method="radix")
+    np.testing.assert_array_equal(auto, radix)
+    np.testing.assert_array_equal(fused, radix)
+
+
 @pytest.mark.parametrize("k", [1, 15, 16, 17, 33, 64])
 @pytest.mark.parametrize("data", ["lattice", "blobs"])
 @pytest.mark.parametrize("pruning", ["always", "never"])
