@@ -9,19 +9,20 @@
 //     that was queued when it was freed, on every stream, as hipFree waits;
 //   - freeing a buffer a second time is an error, as for hipFree, and frees
 //     nothing; a pointer that is no buffer of this pool goes to the runtime;
-//   - at most Device::keepLimit() bytes are kept, and given back by
-//     releaseKept(), which also runs where an allocation finds no memory.
+//   - at most Device::keepLimit() bytes are kept, the oldest making way, and
+//     given back by releaseKept(), which also runs where an allocation finds no
+//     memory.
 // No HIP types here: the file compiles on the host alone.
 #pragma once
 
+#include "kept_blocks.hpp"
+
 #include <stddef.h>
 
-#include <map>
 #include <mutex>
 #include <new>
 #include <unordered_map>
 #include <utility>
-#include <vector>
 
 namespace cuhc {
 
@@ -95,18 +96,12 @@ public:
 
   void releaseKept() {
     std::lock_guard<std::mutex> lock(mutex_);
-    for (auto &entry : kept_)
-      for (void *p : entry.second) {
-        buffers_.erase(p);
-        (void)device_.release(p);
-      }
-    kept_.clear();
-    keptBytes_ = 0;
+    kept_.clear([this](void *p) { forget(p); });
   }
 
   size_t keptBytes() {
     std::lock_guard<std::mutex> lock(mutex_);
-    return keptBytes_;
+    return kept_.bytes();
   }
 
 private:
@@ -119,35 +114,27 @@ private:
 
   void *takeKept(int on, size_t bytes) {
     std::lock_guard<std::mutex> lock(mutex_);
-    const auto it = kept_.find(Key{on, bytes});
-    if (it == kept_.end() || it->second.empty())
-      return nullptr;
-    void *p = it->second.back();
-    it->second.pop_back();
-    keptBytes_ -= bytes;
-    buffers_[p].held = true;
+    void *p = kept_.take(Key{on, bytes});
+    if (p)
+      buffers_[p].held = true;
     return p;
   }
 
   bool keep(void *p, const Buffer &b) {
     const size_t limit = device_.keepLimit();
     std::lock_guard<std::mutex> lock(mutex_);
-    if (b.bytes > limit || keptBytes_ > limit - b.bytes)
-      return false;
-    try {
-      kept_[Key{b.device, b.bytes}].push_back(p);
-    } catch (const std::bad_alloc &) {
-      return false;
-    }
-    keptBytes_ += b.bytes;
-    return true;
+    return kept_.put(Key{b.device, b.bytes}, p, b.bytes, limit, [this](void *q) { forget(q); });
+  }
+
+  void forget(void *p) {
+    buffers_.erase(p);
+    (void)device_.release(p);
   }
 
   Device device_;
   std::mutex mutex_;
   std::unordered_map<void *, Buffer> buffers_; // handed out, or kept
-  std::map<Key, std::vector<void *>> kept_;
-  size_t keptBytes_ = 0;
+  KeptBlocks<Key> kept_;
 };
 
 } // namespace cuhc

@@ -2,12 +2,12 @@
 
 #include "caller_buffers.hpp"
 #include "common.hpp"
+#include "kept_blocks.hpp"
 
 #include <algorithm>
 #include <atomic>
 #include <cstdlib>
 #include <mutex>
-#include <unordered_map>
 
 namespace cuhc {
 
@@ -67,14 +67,14 @@ int numCUs() {
 // 256 B below) and handed to the next request of the same class. All work
 // runs on the one library stream, so a reused block is only touched by work
 // ordered after every earlier use of it. The cache holds at most a quarter of
-// device memory; when hipMalloc fails, the cache is released and the request
-// retried. releaseLibraryState() frees it (at exit, before the runtime's own
-// teardown).
+// device memory, the oldest blocks making way; when hipMalloc fails, the cache
+// is released and the request retried. releaseLibraryState() frees it (at exit,
+// before the runtime's own teardown).
 namespace {
 struct DeviceCache {
   std::mutex mutex;
-  std::unordered_map<size_t, std::vector<void *>> blocks;
-  size_t bytes = 0, limit = 0;
+  KeptBlocks<size_t> blocks; // by size class
+  size_t limit = 0;
 };
 
 DeviceCache &deviceCache() {
@@ -91,11 +91,7 @@ size_t sizeClass(size_t bytes) {
 void releaseCache(DeviceCache &cache) {
   if (hipStream_t st = gStream.load())
     (void)hipStreamSynchronize(st);
-  for (auto &entry : cache.blocks)
-    for (void *p : entry.second)
-      (void)hipFree(p);
-  cache.blocks.clear();
-  cache.bytes = 0;
+  cache.blocks.clear([](void *p) { (void)hipFree(p); });
 }
 } // namespace
 
@@ -216,15 +212,11 @@ int deviceAlloc(void **p, size_t bytes) {
   DeviceCache &cache = deviceCache();
   const size_t cls = sizeClass(bytes);
   std::lock_guard<std::mutex> lock(cache.mutex);
-  auto it = cache.blocks.find(cls);
-  if (it != cache.blocks.end() && !it->second.empty()) {
-    *p = it->second.back();
-    it->second.pop_back();
-    cache.bytes -= cls;
+  *p = cache.blocks.take(cls);
+  if (*p)
     return 0;
-  }
   hipError_t e = hipMalloc(p, cls);
-  if (e == hipErrorOutOfMemory && (cache.bytes > 0 || callerBuffers().keptBytes() > 0)) {
+  if (e == hipErrorOutOfMemory && (cache.blocks.bytes() > 0 || callerBuffers().keptBytes() > 0)) {
     (void)hipGetLastError();
     releaseCache(cache);
     callerBuffers().releaseKept();
@@ -252,18 +244,16 @@ void deviceFree(void *p, size_t bytes) {
     else
       cache.limit = (size_t)16 << 30;
   }
-  if (cache.bytes + cls > cache.limit) {
-    (void)hipFree(p);
-    return;
-  }
-  cache.blocks[cls].push_back(p);
-  cache.bytes += cls;
+  // hipFree waits for the device: blocks that make way are not in use then.
+  const auto release = [](void *q) { (void)hipFree(q); };
+  if (!cache.blocks.put(cls, p, cls, cache.limit, release))
+    release(p);
 }
 
 size_t cachedDeviceBytes() {
   DeviceCache &cache = deviceCache();
   std::lock_guard<std::mutex> lock(cache.mutex);
-  return cache.bytes + callerBuffers().keptBytes();
+  return cache.blocks.bytes() + callerBuffers().keptBytes();
 }
 
 int upload(void *dst, const void *src, size_t bytes) {

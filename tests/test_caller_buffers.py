@@ -86,16 +86,32 @@ int main(int argc, char **argv) {
     CHECK(pool.alloc(&c, 100) == 0 && c == a);
   } else if (!std::strcmp(test, "bounds")) {
     CHECK(pool.alloc(&a, 600) == 0 && pool.alloc(&b, 600) == 0 && pool.alloc(&c, 1001) == 0);
-    CHECK(pool.free(a) == 0 && pool.free(b) == 0 && pool.free(c) == 0);
-    CHECK(pool.keptBytes() == 600 && world.live.size() == 1 && world.live.count(a) == 1);
+    CHECK(pool.free(a) == 0 && pool.free(b) == 0 && pool.free(c) == 0); // the latest is kept
+    CHECK(pool.keptBytes() == 600 && world.live.size() == 1 && world.live.count(b) == 1);
     world.room = 700; // the kept buffer makes way
-    CHECK(pool.alloc(&b, 650) == 0 && world.others == 1 && world.live.count(a) == 0);
+    void *kept = b;
+    CHECK(pool.alloc(&b, 650) == 0 && world.others == 1 && world.live.count(kept) == 0);
     CHECK(pool.alloc(&c, 650) == cuhc::kStatusOutOfMemory && c == nullptr);
     CHECK(pool.alloc(&c, ~(size_t)0) == cuhc::kStatusOutOfMemory && c == nullptr);
     CHECK(pool.free(b) == 0);
     pool.releaseKept();
     CHECK(pool.keptBytes() == 0 && world.live.empty());
     CHECK(pool.free(b) == cuhc::kStatusInvalidValue);
+  } else if (!std::strcmp(test, "oldest")) { // many sizes: those of the latest calls are kept
+    cuhc::KeptBlocks<size_t> blocks;
+    std::vector<int> gone;
+    auto release = [&](void *p) { gone.push_back((int)(size_t)p); };
+    for (size_t i = 1; i <= 12; ++i) // keys 1 2 3 1 2 3 ..., 100 bytes each
+      CHECK(blocks.put((i - 1) % 3 + 1, (void *)i, 100, 1000, release));
+    CHECK((gone == std::vector<int>{1, 2}) && blocks.bytes() == 1000);
+    CHECK((size_t)blocks.take(1) == 10 && (size_t)blocks.take(1) == 7 && (size_t)blocks.take(1) == 4);
+    CHECK(!blocks.take(1) && !blocks.take(9) && blocks.bytes() == 700);
+    CHECK(blocks.put(7, (void *)20, 650, 1000, release) && blocks.bytes() == 950);
+    CHECK((gone == std::vector<int>{1, 2, 3, 5, 6, 8}));
+    CHECK(!blocks.put(7, (void *)21, 1001, 1000, release) && gone.size() == 6);
+    blocks.clear(release);
+    CHECK((gone == std::vector<int>{1, 2, 3, 5, 6, 8, 9, 11, 12, 20}) && blocks.bytes() == 0);
+    CHECK(!blocks.take(7));
   } else if (!std::strcmp(test, "failed_wait")) { // perhaps still in use: not kept
     CHECK(pool.alloc(&a, 100) == 0);
     world.waitStatus = 719;
@@ -145,8 +161,8 @@ def driver(tmp_path_factory):
     return exe
 
 
-@pytest.mark.parametrize("rule", ["second_free", "foreign", "devices", "bounds", "failed_wait",
-                                  "threads"])
+@pytest.mark.parametrize("rule", ["second_free", "foreign", "devices", "bounds", "oldest",
+                                  "failed_wait", "threads"])
 def test_rules(driver, rule):
     run = subprocess.run([str(driver), rule], capture_output=True, text=True)
     assert run.returncode == 0, run.stdout
